@@ -65,8 +65,13 @@ struct HubMeta {
 // ------------------------------------------------------------ wave tasks --
 // Roots per cursor atomic of the wave-task kernel (measured on RMAT-22:
 // chunks shrinking to one root at the end of the list 39.0 ms; fixed chunks
-// of 4 / 8 / 16 / 32: 37.6 / 37.0 / 36.9 / 36.8 ms).
+// of 4 / 8 / 16 / 32: 37.6 / 37.0 / 36.9 / 36.8 ms).  A list that gives each
+// wave no more roots than one chunk is dealt out round robin instead, without
+// the cursor: chunks of 32 would leave most of the chip idle behind a few
+// waves' chains of dependent loads (RMAT-12 4-cliques, 3 K roots: 584 us on
+// about 100 waves), chunks of 1 would queue on the cursor's line.
 constexpr uint32_t kWaveTaskChunk = 32;
+constexpr uint32_t kWaveBlocksPerCU = 6;  // resident 256-thread workgroups (6 waves per SIMD)
 
 // One task per wave, |N+(u)| <= 64.  LDS per wave: L[64], 128-slot hash,
 // 64 bitmap rows (one u64 each) and the row descriptors.  Tasks are small,
@@ -103,7 +108,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
     uint32_t qcur = 0xFFFFFFFFu;
     const uint32_t workers = gridDim.x * WPB;
     TaskChunk chunk(ntasks, workers, 2, kWaveTaskChunk, kWaveTaskChunk);
-    auto fetch = [&]() { return wave_next_task(chunk, cursor); };
+    const bool dealt = ntasks / kWaveTaskChunk <= workers;
+    uint32_t tdeal = wave_bcast(blockIdx.x * WPB + uint32_t(w));
+    auto fetch = [&]() {
+        if (!dealt) return wave_next_task(chunk, cursor);
+        const uint32_t r = tdeal;
+        tdeal += workers;  // at most 33 * workers: no wrap
+        return r;
+    };
     // current task: index, query, list start and length, graph arrays
     uint32_t t = fetch(), q = 0, d = 0;
     uint64_t ub = 0;
@@ -1140,7 +1152,7 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
     uint32_t* cur = x.d_cursor + gr.cursor;
     const size_t lds_limit = R.lds_per_block - kStaticLdsReserve;
     if (gr.bucket == 0) {
-        const uint32_t grid = std::min<uint32_t>((nt + 3) / 4, uint32_t(R.num_cus) * 8);
+        const uint32_t grid = std::min<uint32_t>((nt + 3) / 4, uint32_t(R.num_cus) * kWaveBlocksPerCU);
         if (stream_queue_enabled())
             hipLaunchKernelGGL((clique_wave_kernel<K, true>), dim3(grid), dim3(256), 0, s, qrefs, tv, tq, nt, cur,
                                x.d_result);

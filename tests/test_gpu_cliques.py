@@ -219,3 +219,16 @@ def test_kernels_without_probe_queues_are_exact(tmp_path):
     for name, g in graphs.items():
         want = [oracle.run_app(APP[k], g.rowptr, g.col)[1][0] for k in (3, 4, 5)]
         assert got[name] == want, (name, got[name], want)
+
+
+@pytest.mark.parametrize("n,m", [(5, 9), (3000, 9000), (150000, 450000), (260000, 1600000)])
+def test_wave_tasks_dealt_and_from_the_cursor(kzdev, n, m):
+    """Root lists of a handful of waves, of one round, of many rounds dealt
+    out round robin, and long enough (above 32 roots a wave) for the cursor."""
+    kz = kzdev
+    g = kz.gen_erdos_renyi(n, m, 3).oriented()
+    want = oracle.run_app(APP[3], g.rowptr, g.col)[1][0]
+    dg = g.to_device()
+    for _ in range(2):
+        assert dg.count_cliques(3, "persistent") == want
+    dg.release()
