@@ -45,21 +45,28 @@
 #include <cstring>
 #include <map>
 
+#include "kz_core.h"
 #include "kz_device.h"
 #include "kz_kernels.h"
 #include "kz_stream.h"
 
 namespace kz {
 
+// A query's forward graph and its core (kz_core.h): ids >= cbase, csize of
+// them, n1 the highest id; without a core cbase is above every id.
 struct QueryRef {
     const uint64_t* rowptr;
     const uint32_t* col;
+    const uint32_t* core;
+    uint32_t n1, cbase, csize;
 };
 
-// A hub root split over workgroups (bucket above the last bound).
+// A hub root split over workgroups (bucket above the last bound); list
+// entries from index k0 on are in the core.
 struct HubMeta {
     uint32_t u, q, d, W;
     uint64_t slab_off;  // in u64 words
+    uint32_t k0, reserved;
 };
 
 // ------------------------------------------------------------ wave tasks --
@@ -121,10 +128,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
     uint64_t ub = 0;
     const uint64_t* rowptr = nullptr;
     const uint32_t* col = nullptr;
+    const uint32_t* core = nullptr;
+    uint32_t n1 = 0, cbase = 0, csize = 0;
+    auto load_core = [&](uint32_t qi) {
+        core = queries[qi].core;
+        n1 = queries[qi].n1;
+        cbase = queries[qi].cbase;
+        csize = queries[qi].csize;
+    };
     if (t < ntasks) {
         q = task_q ? task_q[t] : 0u;
         rowptr = queries[q].rowptr;
         col = queries[q].col;
+        load_core(q);
         const uint32_t u = task_v[t];
         ub = ldg(rowptr, u);
         d = uint32_t(ldg(rowptr, u + 1) - ub);
@@ -137,22 +153,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
         const uint32_t x = lane < d ? ldg(col, ub + lane) : 0xFFFFFFFFu;
         const uint32_t tn = fetch();
         L[lane] = x;
-        hk[lane] = kEmpty;
-        hk[lane + 64] = kEmpty;
-        if (lane < 32) rs.fb[lane] = 0;
-        rows[lane] = 0;
-        // row descriptors: lane r owns row r
-        // (rows >= d - 1 are empty, so rp[d - 1] is the group total)
-        uint32_t groups = 0, len = 0;
-        uint64_t desc = 0;
+        // rows below k0: streamed or searched; the others come from the core
+        const uint32_t k0 = uint32_t(__popcll(__ballot(lane < d && x < cbase)));
+        const uint32_t nr = k0 < d - 1 ? k0 : d - 1;
+        uint32_t G = 0;
         bool skewed = false;
-        if (lane + 1 < d) skewed = row_desc(rowptr, x, d - 1 - lane, &desc, &groups, &len);
-        rb[lane] = desc;
-        uint32_t excl;
-        const uint32_t G = wave_exclusive_scan(groups, &excl);
-        rp[lane] = excl;
-        wave_lds_sync();
-        if (lane < d) root_insert(rs, x, uint16_t(lane));
+        if (k0) {
+            rows[lane] = 0;
+            // row descriptors: lane r owns row r
+            // (rows >= nr are empty, so rp[nr] is the group total)
+            uint32_t groups = 0, len = 0;
+            uint64_t desc = 0;
+            if (lane < nr) skewed = row_desc(rowptr, x, d - 1 - lane, &desc, &groups, &len);
+            rb[lane] = desc;
+            uint32_t excl;
+            G = wave_exclusive_scan(groups, &excl);
+            rp[lane] = excl;
+            if (G) {
+                hk[lane] = kEmpty;
+                hk[lane + 64] = kEmpty;
+                if (lane < 32) rs.fb[lane] = 0;
+                wave_lds_sync();
+                if (lane < d) root_insert(rs, x, uint16_t(lane));
+            }
+        }
         // next task's query and root (a cursor atomic has returned by now)
         uint32_t qn = q, un = 0;
         if (tn < ntasks) {
@@ -160,13 +184,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
             un = task_v[tn];
         }
         wave_lds_sync();
-        stream_groups<kGroups, (K >= 4), QU>(
-            col, rb, rp, d - 1, G, lane, 64, rs,
-            [&](uint32_t r, uint32_t j, uint64_t) {
-                if (K == 3) acc += 1;
-                else atomicOr(&rows[r], 1ull << j);
-            },
-            nullptr, QU ? sQ[QU ? w : 0] : nullptr);
+        if (k0 + 1 < d) {
+            const uint32_t c = d - k0;
+            unsigned long long wrow = 0;
+            if (c <= 32) {
+                const uint32_t xr = core_num(x, n1, csize), line = core_line(xr);
+                if (c <= 8) wrow = core_rows_short<8>(core, xr, line, k0, c);
+                else if (c <= 16) wrow = core_rows_short<4>(core, xr, line, k0, c);
+                else wrow = core_rows_short<2>(core, xr, line, k0, c);
+                if (K == 3) acc += uint32_t(__popcll(wrow));
+                else if (lane >= k0) rows[lane] = wrow;
+            } else {
+                for (uint32_t i0 = k0 & 32u; i0 < d; i0 += 32)
+                    core_tile(
+                        core, n1, csize, d, k0, i0, 0, [&](uint32_t i) { return L[i]; },
+                        [&](uint32_t i, unsigned long long wd) {
+                            if (K == 3) acc += uint32_t(__popcll(wd));
+                            else rows[i] = wd;
+                        });
+            }
+        } else if (K >= 4 && k0 < d && lane == k0) {
+            rows[lane] = 0;
+        }
+        if (G)
+            stream_groups<kGroups, (K >= 4), QU>(
+                col, rb, rp, nr, G, lane, 64, rs,
+                [&](uint32_t r, uint32_t j, uint64_t) {
+                    if (K == 3) acc += 1;
+                    else atomicOr(&rows[r], 1ull << j);
+                },
+                nullptr, QU ? sQ[QU ? w : 0] : nullptr);
         // next task's list bounds
         const uint64_t* rowptr_n = rowptr;
         const uint32_t* col_n = col;
@@ -182,7 +229,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
         }
         // skewed rows: their (row, candidate) pairs spread over the lanes
         if (__ballot(skewed))
-            search_skewed(col, rb, L, d, 0, d - 1, 0, 1, [&](uint32_t r, uint32_t j, uint64_t) {
+            search_skewed(col, rb, L, d, 0, nr, 0, 1, [&](uint32_t r, uint32_t j, uint64_t) {
                 if (K == 3) acc += 1;
                 else atomicOr(&rows[r], 1ull << j);
             });
@@ -208,6 +255,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void c
         }
         wave_lds_sync();
         t = tn;
+        if (qn != q && tn < ntasks) load_core(qn);
         q = qn;
         rowptr = rowptr_n;
         col = col_n;
@@ -660,15 +708,17 @@ __device__ __forceinline__ void set_row_bit(unsigned long long* rows, uint32_t w
 // caller), streaming the neighbour lists of all rows as 16-byte groups.  rb holds
 // (r1 - r0) row descriptors and rp (r1 - r0 + 1) group prefixes, both LDS
 // scratch; tmp holds one u32 per wave and ctr one u32 (the stream's span
-// counter).  Block-wide; NG groups of 4 entries per lane and span; QU:
-// queued probes, q the workgroup's queues (64 uint2 per wave); TRI: packed
-// rows (word_base).
-template <int K, int NG = kGroups, bool QU = false, bool TRI = false>
+// counter).  stage() builds the set rs (block-wide, ending in a barrier) and
+// is called only if a row is streamed: searched rows do not need it.
+// Block-wide, no barrier at the end; NG groups of 4 entries per lane and
+// span; QU: queued probes, q the workgroup's queues (64 uint2 per wave);
+// TRI: packed rows (word_base).
+template <int K, int NG = kGroups, bool QU = false, bool TRI = false, class Stage>
 __device__ __forceinline__ void build_rows_block(const uint64_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
                                                  const uint32_t* L, uint32_t d, const RootSet& rs, uint32_t r0, uint32_t r1,
                                                  unsigned long long* rows_out, uint32_t ws, unsigned long long* rb,
                                                  uint32_t* rp, uint32_t* tmp, uint32_t* ctr,
-                                                 unsigned long long& acc, uint32_t* q = nullptr) {
+                                                 unsigned long long& acc, uint32_t* q, Stage&& stage) {
     const uint32_t nr = r1 - r0;
     if (threadIdx.x == 0) *ctr = 0;
     for (uint32_t r = threadIdx.x; r <= nr; r += blockDim.x) {
@@ -681,19 +731,50 @@ __device__ __forceinline__ void build_rows_block(const uint64_t* __restrict__ ro
     }
     __syncthreads();
     const uint32_t G = block_exclusive_scan(rp, nr + 1, tmp);
-    stream_groups<NG, (K >= 4), QU>(
-        col, rb, rp, nr, G, threadIdx.x, blockDim.x, rs,
-        [&](uint32_t r, uint32_t j, uint64_t) {
-            if (K == 3) acc += 1;
-            else set_row_bit<TRI>(rows_out, ws, r, j);
-        },
-        ctr, QU ? q + (threadIdx.x >> 6) * 128 : nullptr);
+    if (G) {
+        stage();
+        stream_groups<NG, (K >= 4), QU>(
+            col, rb, rp, nr, G, threadIdx.x, blockDim.x, rs,
+            [&](uint32_t r, uint32_t j, uint64_t) {
+                if (K == 3) acc += 1;
+                else set_row_bit<TRI>(rows_out, ws, r, j);
+            },
+            ctr, QU ? q + (threadIdx.x >> 6) * 128 : nullptr);
+    }
     // skewed rows: each wave searches the candidates of its own rows
     search_skewed(col, rb, L, d, r0, nr, threadIdx.x >> 6, blockDim.x >> 6, [&](uint32_t r, uint32_t j, uint64_t) {
         if (K == 3) acc += 1;
         else set_row_bit<TRI>(rows_out, ws, r, j);
     });
-    __syncthreads();
+}
+
+// Rows [lo, d) of a root from the core: the workgroup's waves take tiles of
+// 32 rows by one 64-candidate word from an LDS counter (ctr, zeroed before a
+// barrier), tile (I, kk) with I <= 2 kk + 1 numbered as pair_coords; tiles
+// below row lo are skipped.  put(i, kk, word) as core_tile.
+template <class Put>
+__device__ __forceinline__ void core_rows_block(const uint32_t* core, uint32_t n1, uint32_t csize, const uint32_t* L,
+                                                uint32_t d, uint32_t lo, uint32_t* ctr, Put&& put) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t nb = (d + 31) >> 5, W = (d + 63) >> 6;
+    const uint32_t k_lo = lo >> 6, base = k_lo * (k_lo + 1);  // tiles of words below lo's hold no row
+    const uint32_t n = (W - 1) * W + nb - base;
+    uint32_t t = 0;
+    if (lane == 0) t = atomicAdd(ctr, 1u);
+    t = wave_bcast(t);
+    while (t < n) {
+        uint32_t tn = 0;
+        if (lane == 0) tn = atomicAdd(ctr, 1u);
+        uint32_t I, kk;
+        pair_coords(base + t, W, &I, &kk);
+        I = wave_bcast(I);
+        kk = wave_bcast(kk);
+        if (32 * I + 32 > lo)
+            core_tile(
+                core, n1, csize, d, lo, 32 * I, kk, [&](uint32_t i) { return L[i]; },
+                [&](uint32_t i, unsigned long long w) { put(i, kk, w); });
+        t = wave_bcast(tn);
+    }
 }
 
 // ----------------------------------------------------------- block tasks --
@@ -740,17 +821,20 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(WPE))) voi
     uint32_t* fb = reinterpret_cast<uint32_t*>(p);
     p += size_t(FW) * 4;
     uint16_t* hv = reinterpret_cast<uint16_t*>(p);
-    __shared__ uint32_t sTask, sTmp[16], sSpan, sTile;
+    __shared__ uint32_t sTask, sTmp[16], sSpan, sTile, sCore;
     const RootSet rs{hk, hv, H - 1, hshift, fb, fshift};
     unsigned long long acc = 0;
     uint32_t qcur = 0xFFFFFFFFu;
     const uint64_t* rowptr = nullptr;
     const uint32_t* col = nullptr;
+    const uint32_t* core = nullptr;
+    uint32_t n1 = 0, cbase = 0, csize = 0;
     TaskChunk chunk(ntasks, gridDim.x, 8);
     while (true) {
         if (threadIdx.x == 0) {
             sTask = thread_next_task(chunk, cursor);
             sTile = 0;
+            sCore = 0;
         }
         __syncthreads();
         const uint32_t t = wave_bcast(sTask);
@@ -761,18 +845,39 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(WPE))) voi
             qcur = q;
             rowptr = queries[q].rowptr;
             col = queries[q].col;
+            core = queries[q].core;
+            n1 = queries[q].n1;
+            cbase = queries[q].cbase;
+            csize = queries[q].csize;
         }
         const uint32_t u = task_v[t];
         const uint64_t ub = ldg(rowptr, u);
         const uint32_t d = wave_bcast(uint32_t(ldg(rowptr, u + 1) - ub));
         for (uint32_t i = threadIdx.x; i < d; i += blockDim.x) L[i] = ldg(col, ub + i);
-        root_clear(rs, H, FW, threadIdx.x, blockDim.x);
-        if (K >= 4)
-            for (uint32_t i = threadIdx.x, n = TRI ? tri_words(d) : d * W; i < n; i += blockDim.x) rows[i] = 0;
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < d; i += blockDim.x) root_insert(rs, L[i], uint16_t(i));
+        // rows below k0 are streamed or searched, the others come from the
+        // core.  Core tiles store whole words (never read below a row's own
+        // word), so only the others are zeroed.
+        const uint32_t k0 = wave_bcast(core_first(L, d, cbase));
+        if (k0) {
+            if (K >= 4)
+                for (uint32_t kk = 0; 64 * kk < d; ++kk) {
+                    const uint32_t n = TRI && 64 * (kk + 1) < k0 ? 64 * (kk + 1) : k0;
+                    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) rows[word_base<TRI>(kk, d) + i] = 0;
+                }
+            build_rows_block<K, NG, QU, TRI>(rowptr, col, L, d, rs, 0, k0, rows, d, rb, rp, sTmp, &sSpan, acc, qu, [&]() {
+                root_clear(rs, H, FW, threadIdx.x, blockDim.x);
+                __syncthreads();
+                for (uint32_t i = threadIdx.x; i < d; i += blockDim.x) root_insert(rs, L[i], uint16_t(i));
+                __syncthreads();
+            });
+        }
+        if (k0 < d)
+            core_rows_block(core, n1, csize, L, d, k0, &sCore, [&](uint32_t i, uint32_t kk, unsigned long long w) {
+                if (K == 3) acc += uint32_t(__popcll(w));
+                else rows[word_base<TRI>(kk, d) + i] = w;
+            });
         __syncthreads();
-        build_rows_block<K, NG, QU, TRI>(rowptr, col, L, d, rs, 0, d, rows, d, rb, rp, sTmp, &sSpan, acc, qu);
         if (K == 4) count_rows_mfma4<TRI, (WPE <= 4)>(rows, d, d, &sTile, acc);
         else if (K == 5) {
             if (W <= 8) count5_edges<TRI>(rows, d, rp, sTmp, &sTile, acc);
@@ -862,11 +967,13 @@ __global__ __launch_bounds__(1024) void hub_rows_kernel(const QueryRef* __restri
             hcur = h;
         }
         const uint32_t r0 = (it - item_prefix[h]) * RPC;
-        const uint32_t r1 = r0 + RPC < d ? r0 + RPC : d;
+        const uint32_t r1 = r0 + RPC < hm.k0 ? r0 + RPC : hm.k0;
         if (K >= 4)
             for (uint32_t i = threadIdx.x; i < (r1 - r0) * hm.W; i += blockDim.x) rbuf[i] = 0;
         __syncthreads();
-        build_rows_block<K, kGroups, QU>(rowptr, col, L, d, rs, r0, r1, rbuf, r1 - r0, rb, rp, sTmp, &sSpan, acc, qu);
+        build_rows_block<K, kGroups, QU>(rowptr, col, L, d, rs, r0, r1, rbuf, r1 - r0, rb, rp, sTmp, &sSpan, acc, qu,
+                                         [] {});
+        __syncthreads();
         if (K >= 4) {
             // the slab is word-major over all d rows of the hub
             const uint32_t nr = r1 - r0;
@@ -879,6 +986,99 @@ __global__ __launch_bounds__(1024) void hub_rows_kernel(const QueryRef* __restri
         __syncthreads();
     }
     if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
+}
+
+// Core rows of the hubs, one wave per tile of 32 rows by one 64-candidate word
+// (core_tile; tile_prefix: exclusive prefix over hubs of (W - 1) W +
+// ceil(d / 32) tiles, numbered as pair_coords), stored to the hub's slab, or
+// counted directly (k = 3).
+template <int K>
+__global__ __launch_bounds__(256) void hub_core_kernel(const QueryRef* __restrict__ queries,
+                                                       const HubMeta* __restrict__ hubs, uint32_t nhubs,
+                                                       const uint32_t* __restrict__ tile_prefix, uint32_t ntiles,
+                                                       uint32_t* __restrict__ cursor,
+                                                       unsigned long long* __restrict__ results,
+                                                       unsigned long long* __restrict__ slab) {
+    unsigned long long acc = 0;
+    uint32_t qcur = 0xFFFFFFFFu;
+    TaskChunk chunk(ntiles, gridDim.x * (blockDim.x >> 6), 8);
+    while (true) {
+        const uint32_t t = wave_next_task(chunk, cursor);
+        if (t >= ntiles) break;
+        const uint32_t h = wave_bcast(row_of(tile_prefix, nhubs, t));
+        const HubMeta hm = hubs[h];
+        if (hm.q != qcur) {
+            if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
+            qcur = hm.q;
+        }
+        uint32_t I, kk;
+        pair_coords(t - tile_prefix[h], hm.W, &I, &kk);
+        I = wave_bcast(I);
+        kk = wave_bcast(kk);
+        if (32 * I + 32 <= hm.k0) continue;
+        const QueryRef Q = queries[hm.q];
+        const uint64_t ub = ldg(Q.rowptr, hm.u);
+        unsigned long long* rows = slab + hm.slab_off + size_t(kk) * hm.d;
+        core_tile(
+            Q.core, Q.n1, Q.csize, hm.d, hm.k0, 32 * I, kk, [&](uint32_t i) { return ldg(Q.col, ub + i); },
+            [&](uint32_t i, unsigned long long w) {
+                if (K == 3) acc += uint32_t(__popcll(w));
+                else rows[i] = w;
+            });
+    }
+    if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
+}
+
+// k0 of every hub: its list entries below the core.
+__global__ void hub_split_kernel(const QueryRef* __restrict__ queries, HubMeta* __restrict__ hubs, uint32_t nhubs) {
+    const uint32_t h = blockIdx.x * blockDim.x + threadIdx.x;
+    if (h >= nhubs) return;
+    const QueryRef Q = queries[hubs[h].q];
+    hubs[h].k0 = lower_bound_global(Q.col + Q.rowptr[hubs[h].u], hubs[h].d, Q.cbase);
+}
+
+// Builds a core's bit rows: one workgroup per row r (vertex n1 - r), in LDS,
+// written out whole lines.
+__global__ __launch_bounds__(256) void core_build_kernel(const uint64_t* __restrict__ rowptr,
+                                                         const uint32_t* __restrict__ col, uint32_t n1, uint32_t size,
+                                                         uint32_t* __restrict__ bm) {
+    extern __shared__ uint32_t srow[];
+    // the last workgroup zeroes the words masked lanes read past the last row
+    const uint32_t r = blockIdx.x;
+    const uint32_t words = r < size ? 32 * (core_line(r + 1) - core_line(r)) : (size / 8 + 256) / 128 * 32;
+    uint32_t* out = bm + 32ull * core_line(r);
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) srow[i] = 0;
+    __syncthreads();
+    if (r < size) {
+        const uint64_t b = rowptr[n1 - r], e = rowptr[n1 - r + 1];
+        for (uint64_t p = b + threadIdx.x; p < e; p += blockDim.x) {
+            const uint32_t x = n1 - col[p];
+            if (x < r) atomicOr(&srow[x >> 5], 1u << (x & 31u));  // forward neighbours are higher ids
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) out[i] = srow[i];
+}
+
+// Sum of d+(v) over up to kCoreSample evenly spaced edges (u, v) of each
+// graph (one workgroup per graph).
+constexpr uint32_t kCoreSample = 16384;
+struct CoreGraph {
+    const uint64_t* rowptr;
+    const uint32_t* col;
+    uint64_t nnz;
+};
+__global__ __launch_bounds__(256) void core_sample_kernel(const CoreGraph* __restrict__ graphs,
+                                                          unsigned long long* __restrict__ sums) {
+    const CoreGraph G = graphs[blockIdx.x];
+    const uint64_t n = G.nnz < kCoreSample ? G.nnz : kCoreSample;
+    unsigned long long s = 0;
+    for (uint64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        const uint32_t v = G.col[i * G.nnz / n];
+        s += G.rowptr[v + 1] - G.rowptr[v];
+    }
+    s = wave_sum_u64(s);
+    if ((threadIdx.x & 63) == 0 && s) atomicAdd(&sums[blockIdx.x], s);
 }
 
 // One wave per hub row: counts the cliques whose second vertex is that row.
@@ -988,6 +1188,8 @@ CliqueJob::~CliqueJob() {
     for (auto& h : hub_items) hipFree(h.second);
     for (auto& h : hub_rows) hipFree(h.second);
     for (auto& h : hub_tiles) hipFree(h.second);
+    for (auto& h : hub_ctiles) hipFree(h.second);
+    for (uint32_t* c : cores) hipFree(c);
 }
 
 // Must match the carving at the top of clique_block_kernel / hub_rows_kernel.
@@ -1086,7 +1288,8 @@ static int set_lds_attrs() {
                          reinterpret_cast<const void*>(&hub_rows_kernel<4>),
                          reinterpret_cast<const void*>(&hub_rows_kernel<5>),
                          reinterpret_cast<const void*>(&hub_rows_kernel<4, true>),
-                         reinterpret_cast<const void*>(&hub_rows_kernel<5, true>)};
+                         reinterpret_cast<const void*>(&hub_rows_kernel<5, true>),
+                         reinterpret_cast<const void*>(&core_build_kernel)};
     for (const void* f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, maxb) != hipSuccess)
             (void)hipGetLastError();
@@ -1235,7 +1438,13 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
         KZ_FAIL(KZ_ERR_UNSUPPORTED, "hub rows need %zu bytes of LDS (limit %zu)", sh.lds, lds_limit);
     const uint32_t grid = std::min<uint32_t>(hp.nitems, uint32_t(R.num_cus) * sh.per_cu);
     const HubMeta* meta = static_cast<const HubMeta*>(x.hub_meta[K]);
-    if (hp.queues)
+    if (hp.nctiles) {
+        const uint32_t cgrid = std::min<uint32_t>((hp.nctiles + 3) / 4, uint32_t(R.num_cus) * 8);
+        hipLaunchKernelGGL(hub_core_kernel<K>, dim3(cgrid), dim3(256), 0, s, qrefs, meta, hp.nhubs, x.hub_ctiles[K],
+                           hp.nctiles, cur + 2 * kCursorStride, x.d_result, K >= 4 ? x.slabs[K] : nullptr);
+    }
+    if (!hp.nitems) {
+    } else if (hp.queues)
         hipLaunchKernelGGL((hub_rows_kernel<K, true>), dim3(grid), dim3(sh.block), sh.lds, s, qrefs, meta, hp.nhubs,
                            x.hub_items[K], hp.nitems, cur, x.d_result, K >= 4 ? x.slabs[K] : nullptr, hp.dmax,
                            hp.wmax, hp.rpc, H, filter_words(hp.dmax, hp.fkey), hp.fkey);
@@ -1257,7 +1466,7 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
 
 // Hub plan for one k: per-hub metadata, item and row prefixes, HBM slab.
 static int prepare_hubs(CliqueJob& x, int k, const std::vector<uint32_t>& hv, const std::vector<uint32_t>& hq,
-                        const std::vector<uint32_t>& hd) {
+                        const std::vector<uint32_t>& hd, hipStream_t st) {
     CliqueJob::HubPlan hp;
     hp.nhubs = uint32_t(hv.size());
     hp.dmax = 0;
@@ -1294,41 +1503,61 @@ static int prepare_hubs(CliqueJob& x, int k, const std::vector<uint32_t>& hv, co
         }
     }
     std::vector<HubMeta> meta(hp.nhubs);
-    std::vector<uint32_t> items(hp.nhubs), rows(hp.nhubs), tiles(hp.nhubs);
-    uint64_t slab = 0, nt = 0;
-    uint32_t ni = 0, nr = 0;
+    uint64_t slab = 0;
     for (uint32_t h = 0; h < hp.nhubs; ++h) {
         const uint32_t d = hd[h];
         const uint32_t W = (d + 63) / 64;
-        const uint64_t nb = (d + 63) / 64;  // 2 x 2 tile blocks: one per pair of 64-bit words
-        meta[h] = HubMeta{hv[h], hq[h], d, W, slab};
+        meta[h] = HubMeta{hv[h], hq[h], d, W, slab, d, 0};
         slab += uint64_t(d) * W;
+    }
+    void* dm = nullptr;
+    KZ_HIP(hipMalloc(&dm, sizeof(HubMeta) * std::max<uint32_t>(1, hp.nhubs)));
+    x.hub_meta[k] = dm;
+    KZ_HIP(hipMemcpyAsync(dm, meta.data(), sizeof(HubMeta) * meta.size(), hipMemcpyHostToDevice, st));
+    if (x.core_bytes) {
+        hipLaunchKernelGGL(hub_split_kernel, dim3((hp.nhubs + 255) / 256), dim3(256), 0, st,
+                           static_cast<const QueryRef*>(x.d_queries), static_cast<HubMeta*>(dm), hp.nhubs);
+        KZ_HIP(hipGetLastError());
+        KZ_HIP(hipMemcpyAsync(meta.data(), dm, sizeof(HubMeta) * meta.size(), hipMemcpyDeviceToHost, st));
+    }
+    KZ_HIP(hipStreamSynchronize(st));
+    // rows below k0 go to the rows kernel in chunks, the others to the core
+    // kernel in tiles
+    std::vector<uint32_t> items(hp.nhubs), rows(hp.nhubs), tiles(hp.nhubs), ctiles(hp.nhubs);
+    uint64_t nt = 0, nc = 0;
+    uint32_t ni = 0, nr = 0;
+    for (uint32_t h = 0; h < hp.nhubs; ++h) {
+        const uint32_t d = hd[h];
+        const uint64_t nb = (d + 63) / 64;  // 2 x 2 tile blocks: one per pair of 64-bit words
         items[h] = ni;
         rows[h] = nr;
         tiles[h] = uint32_t(nt);
-        ni += (d + hp.rpc - 1) / hp.rpc;
+        ctiles[h] = uint32_t(nc);
+        ni += (meta[h].k0 + hp.rpc - 1) / hp.rpc;
         nr += d;
         nt += nb * (nb + 1) / 2;
+        if (meta[h].k0 < d) nc += (nb - 1) * nb + (d + 31) / 32;
     }
-    if (nt >= (uint64_t(1) << 32)) KZ_FAIL(KZ_ERR_UNSUPPORTED, "%llu hub tiles (> 2^32)", (unsigned long long)nt);
+    if (nt >= (uint64_t(1) << 32) || nc >= (uint64_t(1) << 32))
+        KZ_FAIL(KZ_ERR_UNSUPPORTED, "%llu hub tiles (> 2^32)", (unsigned long long)std::max(nt, nc));
     hp.nitems = ni;
     hp.nrows = nr;
     hp.ntiles = uint32_t(nt);
-    void* dm = nullptr;
-    uint32_t *di = nullptr, *dr = nullptr, *dt = nullptr;
-    KZ_HIP(hipMalloc(&dm, sizeof(HubMeta) * std::max<uint32_t>(1, hp.nhubs)));
+    hp.nctiles = uint32_t(nc);
+    uint32_t *di = nullptr, *dr = nullptr, *dt = nullptr, *dc = nullptr;
     KZ_HIP(hipMalloc(&di, 4 * std::max<uint32_t>(1, hp.nhubs)));
-    KZ_HIP(hipMalloc(&dr, 4 * std::max<uint32_t>(1, hp.nhubs)));
-    KZ_HIP(hipMalloc(&dt, 4 * std::max<uint32_t>(1, hp.nhubs)));
-    x.bytes += (sizeof(HubMeta) + 12) * std::max<uint32_t>(1, hp.nhubs);
-    x.hub_meta[k] = dm;
     x.hub_items[k] = di;
+    KZ_HIP(hipMalloc(&dr, 4 * std::max<uint32_t>(1, hp.nhubs)));
     x.hub_rows[k] = dr;
+    KZ_HIP(hipMalloc(&dt, 4 * std::max<uint32_t>(1, hp.nhubs)));
     x.hub_tiles[k] = dt;
-    KZ_HIP(hipMemcpy(dm, meta.data(), sizeof(HubMeta) * meta.size(), hipMemcpyHostToDevice));
+    KZ_HIP(hipMalloc(&dc, 4 * std::max<uint32_t>(1, hp.nhubs)));
+    x.hub_ctiles[k] = dc;
+    x.bytes += (sizeof(HubMeta) + 16) * std::max<uint32_t>(1, hp.nhubs);
     KZ_HIP(hipMemcpy(di, items.data(), 4 * items.size(), hipMemcpyHostToDevice));
     KZ_HIP(hipMemcpy(dr, rows.data(), 4 * rows.size(), hipMemcpyHostToDevice));
     KZ_HIP(hipMemcpy(dt, tiles.data(), 4 * tiles.size(), hipMemcpyHostToDevice));
+    KZ_HIP(hipMemcpy(dc, ctiles.data(), 4 * ctiles.size(), hipMemcpyHostToDevice));
     if (k >= 4) {
         unsigned long long* s = nullptr;
         KZ_HIP(hipMalloc(&s, std::max<uint64_t>(1, slab) * 8));
@@ -1336,6 +1565,111 @@ static int prepare_hubs(CliqueJob& x, int k, const std::vector<uint32_t>& hv, co
         x.slabs[k] = s;
     }
     x.hubplan[k] = hp;
+    return KZ_OK;
+}
+
+// Core size (ids) of a forward graph of n ids and nnz list entries: bit rows
+// of a quarter of the lists' bytes (size^2 / 16 = nnz), at most kCoreMax ids.
+// The rows of lower ids are long and sparse: a root's candidates then touch
+// more 128-byte lines of the bit row than the list itself has.  RMAT-24
+// 4-cliques by size^2 / nnz, 128-512 bucket: 8 / 16 / 32 / 64 / 128 / 512 /
+// 2048: 29.9 / 30.2 / 34.6 / 41.6 / 50.0 / 57.9 / 60.2 ms; the wave bucket
+// goes the other way, 13.2 / 12.2 / 12.0 / 11.8 / 11.5 ms up to 128.
+constexpr uint64_t kCoreBitsPerEntry = 16;
+static uint32_t core_size(uint64_t n, uint64_t nnz) {
+    uint64_t b = 0;
+    for (uint64_t s = kCoreMax; s; s >>= 1)
+        if ((b + s) * (b + s) <= kCoreBitsPerEntry * nnz) b += s;
+    b = std::min<uint64_t>(std::min<uint64_t>(b, n), kCoreMax);
+    return b < 2 ? 0u : uint32_t(b);
+}
+uint64_t clique_core_bytes(uint64_t n, uint64_t nnz) {
+    const uint32_t b = core_size(n, nnz);
+    return b ? core_alloc_bytes(b) : 0;
+}
+
+// The cores of the queries' graphs (one per distinct graph), built on st; the
+// queries' references point at them when st has run.  A graph has none where
+// they would pass core_limit or an eighth of the free device memory, where
+// the allocation fails, or where its roots have many more candidate pairs
+// than its candidates' lists have entries (an orientation that is not by
+// degree can have roots of thousands of candidates with almost empty lists):
+// there the stream is cheaper.  A pair costs about an eighth of a streamed
+// entry.
+constexpr uint64_t kCorePairsPerEntry = 8;
+
+static int build_cores(CliqueJob& x, const std::vector<CliqueQuery>& queries, std::vector<QueryRef>& qr, hipStream_t st) {
+    struct Cand {
+        const CliqueQuery* q;
+        uint64_t nnz = 0, pairs = 0;
+        uint32_t size = 0;
+        const uint32_t* bm = nullptr;
+    };
+    std::map<const uint32_t*, size_t> at;  // by column array
+    std::vector<Cand> cand;
+    for (const CliqueQuery& Q : queries) {
+        if (!Q.core || !Q.fdeg || Q.fdeg->size() < 2 || at.count(Q.col)) continue;
+        Cand c{&Q};
+        for (uint32_t d : *Q.fdeg) {
+            c.nnz += d;
+            c.pairs += uint64_t(d) * d / 2;
+        }
+        c.size = core_size(Q.fdeg->size(), c.nnz);
+        if (!c.size || !c.pairs) continue;
+        at[Q.col] = cand.size();
+        cand.push_back(c);
+    }
+    if (!cand.empty()) {
+        size_t free_b = 0, total_b = 0;
+        KZ_HIP(hipMemGetInfo(&free_b, &total_b));
+        const uint64_t limit = std::min<uint64_t>(x.core_limit, free_b / 8);
+        // sampled list entries behind each graph's edges
+        std::vector<CoreGraph> cg(cand.size());
+        std::vector<unsigned long long> sums(cand.size(), 0);
+        for (size_t i = 0; i < cand.size(); ++i) cg[i] = CoreGraph{cand[i].q->rowptr, cand[i].q->col, cand[i].nnz};
+        struct Tmp {
+            void* p = nullptr;
+            ~Tmp() { (void)hipFree(p); }
+        } dg, ds;
+        KZ_HIP(hipMalloc(&dg.p, sizeof(CoreGraph) * cg.size()));
+        KZ_HIP(hipMalloc(&ds.p, 8 * cg.size()));
+        KZ_HIP(hipMemcpyAsync(dg.p, cg.data(), sizeof(CoreGraph) * cg.size(), hipMemcpyHostToDevice, st));
+        KZ_HIP(hipMemcpyAsync(ds.p, sums.data(), 8 * cg.size(), hipMemcpyHostToDevice, st));
+        hipLaunchKernelGGL(core_sample_kernel, dim3(uint32_t(cg.size())), dim3(256), 0, st,
+                           static_cast<const CoreGraph*>(dg.p), static_cast<unsigned long long*>(ds.p));
+        KZ_HIP(hipGetLastError());
+        KZ_HIP(hipMemcpyAsync(sums.data(), ds.p, 8 * cg.size(), hipMemcpyDeviceToHost, st));
+        KZ_HIP(hipStreamSynchronize(st));
+        for (size_t i = 0; i < cand.size(); ++i) {
+            Cand& c = cand[i];
+            const double entries = double(sums[i]) * double(c.nnz) / double(std::min<uint64_t>(c.nnz, kCoreSample));
+            const uint64_t bytes = core_alloc_bytes(c.size);
+            if (double(c.pairs) > double(kCorePairsPerEntry) * entries || x.core_bytes + bytes > limit) continue;
+            uint32_t* bm = nullptr;
+            if (hipMalloc(&bm, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                continue;
+            }
+            x.cores.push_back(bm);
+            x.core_bytes += bytes;
+            c.bm = bm;
+            hipLaunchKernelGGL(core_build_kernel, dim3(c.size + 1), dim3(256), c.size / 8 + 512, st, c.q->rowptr,
+                               c.q->col, uint32_t(c.q->fdeg->size() - 1), c.size, bm);
+            KZ_HIP(hipGetLastError());
+        }
+        x.bytes += x.core_bytes;
+    }
+    for (size_t i = 0; i < queries.size(); ++i) {
+        qr[i] = QueryRef{queries[i].rowptr, queries[i].col, nullptr, 0, 0xFFFFFFFFu, 0};
+        const auto it = at.find(queries[i].col);
+        if (it == at.end() || !queries[i].core) continue;
+        const Cand& c = cand[it->second];
+        if (!c.bm || c.q->rowptr != queries[i].rowptr) continue;
+        qr[i].core = c.bm;
+        qr[i].n1 = uint32_t(c.q->fdeg->size() - 1);
+        qr[i].csize = c.size;
+        qr[i].cbase = qr[i].n1 + 1 - c.size;
+    }
     return KZ_OK;
 }
 
@@ -1401,6 +1735,20 @@ int clique_job_prepare(CliqueJob& x, const std::vector<CliqueQuery>& queries, co
             hq[at] = qi;
         }
     }
+    // a stream of its own for the preparation and the capture: other threads
+    // may use the library stream meanwhile (the server prepares jobs beside
+    // running queries)
+    hipStream_t main = nullptr;
+    KZ_HIP(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
+    struct StreamFree {
+        hipStream_t s;
+        ~StreamFree() { (void)hipStreamDestroy(s); }
+    } main_free{main};
+    std::vector<QueryRef> qr(std::max<size_t>(1, queries.size()));
+    if (int e = build_cores(x, queries, qr, main)) return e;
+    KZ_HIP(hipMalloc(&x.d_queries, sizeof(QueryRef) * qr.size()));
+    KZ_HIP(hipMemcpyAsync(x.d_queries, qr.data(), sizeof(QueryRef) * qr.size(), hipMemcpyHostToDevice, main));
+    KZ_HIP(hipStreamSynchronize(main));  // the cores are built, the references in place
     x.groups.clear();
     int cursor = 0;
     for (int l = 0; l < kLists; ++l) {
@@ -1438,22 +1786,18 @@ int clique_job_prepare(CliqueJob& x, const std::vector<CliqueQuery>& queries, co
             }
         }
         gr.cursor = cursor;
-        // one cursor line per kernel (hubs: rows and count kernels)
-        cursor += int(kCursorStride) * ((gr.bucket == kNumBuckets - 1) ? 2 : 1);
+        // one cursor line per kernel (hubs: rows, count and core kernels)
+        cursor += int(kCursorStride) * ((gr.bucket == kNumBuckets - 1) ? 3 : 1);
         if (gr.bucket == kNumBuckets - 1) {
             std::vector<uint32_t> v(hv.begin() + long(gr.first), hv.begin() + long(gr.first + gr.count));
             std::vector<uint32_t> q(hq.begin() + long(gr.first), hq.begin() + long(gr.first + gr.count));
             std::vector<uint32_t> d(gr.count);
             for (uint64_t i = 0; i < gr.count; ++i) d[i] = (*queries[q[i]].fdeg)[v[i]];
-            if (int e = prepare_hubs(x, gr.k, v, q, d)) return e;
+            if (int e = prepare_hubs(x, gr.k, v, q, d, main)) return e;
         }
         x.groups.push_back(gr);
     }
     x.ntasks = hv.size();
-    std::vector<QueryRef> qr(std::max<size_t>(1, queries.size()));
-    for (size_t i = 0; i < queries.size(); ++i) qr[i] = QueryRef{queries[i].rowptr, queries[i].col};
-    KZ_HIP(hipMalloc(&x.d_queries, sizeof(QueryRef) * qr.size()));
-    KZ_HIP(hipMemcpy(x.d_queries, qr.data(), sizeof(QueryRef) * qr.size(), hipMemcpyHostToDevice));
     KZ_HIP(hipMalloc(&x.d_task_v, sizeof(uint32_t) * std::max<size_t>(1, hv.size())));
     if (!hv.empty()) KZ_HIP(hipMemcpy(x.d_task_v, hv.data(), sizeof(uint32_t) * hv.size(), hipMemcpyHostToDevice));
     if (queries.size() > 1) {
@@ -1464,14 +1808,6 @@ int clique_job_prepare(CliqueJob& x, const std::vector<CliqueQuery>& queries, co
     KZ_HIP(hipMalloc(&x.d_result, sizeof(unsigned long long) * std::max<size_t>(1, queries.size())));
     x.bytes += sizeof(QueryRef) * qr.size() + 4 * std::max<size_t>(1, hv.size()) * (queries.size() > 1 ? 2 : 1) +
                4 * size_t(std::max(1, cursor)) + 8 * std::max<size_t>(1, queries.size());
-    // capture on a stream of its own: other threads may use the library
-    // stream meanwhile (the server prepares jobs beside running queries)
-    hipStream_t main = nullptr;
-    KZ_HIP(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));
-    struct StreamFree {
-        hipStream_t s;
-        ~StreamFree() { (void)hipStreamDestroy(s); }
-    } main_free{main};
     const size_t nbr = std::max<size_t>(1, x.groups.size());
     std::vector<hipStream_t> br(nbr, nullptr);
     std::vector<hipEvent_t> join(nbr, nullptr);

@@ -119,13 +119,14 @@ static std::shared_ptr<void> wrap_job(CliqueJob* j) {
 }
 
 // Prepared single-graph job for (graph, k), built on first use.
-int graph_job(DeviceGraph& d, int k, CliqueJob** out) {
+int graph_job(DeviceGraph& d, int k, CliqueJob** out, uint64_t core_limit) {
     if (int e = ensure_forward(d)) return e;
     auto& slot = d.clique_exec[k];
     if (!slot) {
         CliqueJob* j = new (std::nothrow) CliqueJob();
         if (!j) KZ_FAIL(KZ_ERR_NOMEM, "clique job");
         slot = wrap_job(j);
+        j->core_limit = core_limit;
         std::vector<CliqueQuery> q = {CliqueQuery{d.fwd_rowptr, d.fwd_col, &d.h_fdeg, k}};
         if (int e = clique_job_prepare(*j, q, graph_buckets(d, k))) {
             slot.reset();

@@ -242,7 +242,12 @@ struct CliqueQuery {
     const std::vector<uint32_t>* fdeg;  // host forward out-degrees
     int k;
     uint32_t root_lo = 0, root_hi = 0xFFFFFFFFu;
+    bool core = true;  // rowptr and col are final: a core bitmap may be built from them
 };
+
+// Device bytes of the core bitmap (kz_core.h) of a forward graph, before the
+// checks that may leave it out.
+uint64_t clique_core_bytes(uint64_t n, uint64_t nnz);
 
 // Prepared persistent execution of a set of queries: task groups per
 // (k, bucket) and the captured hipGraph that runs them all.
@@ -268,7 +273,7 @@ struct CliqueJob {
     // hub roots (last bucket), per k: split into row chunks over many
     // workgroups; rows go to an HBM slab, then one wave counts each row
     struct HubPlan {
-        uint32_t nhubs = 0, dmax = 0, wmax = 0, rpc = 64, nitems = 0, nrows = 0, ntiles = 0;
+        uint32_t nhubs = 0, dmax = 0, wmax = 0, rpc = 64, nitems = 0, nrows = 0, ntiles = 0, nctiles = 0;
         bool queues = false;  // rows kernel with probe queues
         uint32_t fkey = 16;   // filter bits per id of a hub's list
     };
@@ -277,6 +282,10 @@ struct CliqueJob {
     std::map<int, uint32_t*> hub_items;    // exclusive prefix of row chunks per hub
     std::map<int, uint32_t*> hub_rows;     // exclusive prefix of rows per hub
     std::map<int, uint32_t*> hub_tiles;    // exclusive prefix of 32 x 32 count tiles per hub (k = 4)
+    std::map<int, uint32_t*> hub_ctiles;   // exclusive prefix of core row tiles per hub
+    std::vector<uint32_t*> cores;          // core bitmaps, one per graph that has one
+    uint64_t core_limit = ~uint64_t(0);    // most device bytes the cores may take
+    uint64_t core_bytes = 0;               // what they take (part of bytes)
     std::map<int, unsigned long long*> slabs;  // per k, HBM bitmap rows
     uint64_t bytes = 0;                        // device memory this job holds
     hipGraph_t graph = nullptr;
@@ -299,8 +308,8 @@ int clique_job_run(CliqueJob& x, uint64_t* counts, double* device_ms);
 // host_results (pinned, nqueries entries) on the same stream; no wait.
 int clique_job_launch(CliqueJob& x, hipStream_t s, unsigned long long* host_results);
 // Prepared single-graph job for (graph, k), built on first use and kept in
-// the graph (kz_count.hip).
-int graph_job(DeviceGraph& d, int k, CliqueJob** out);
+// the graph (kz_count.hip); core_limit bounds its core bitmap's bytes.
+int graph_job(DeviceGraph& d, int k, CliqueJob** out, uint64_t core_limit = ~uint64_t(0));
 // Motif census of a symmetric resident graph; the relabelled copy and
 // counter slabs are kept in the graph (kz_census.hip).  census_bytes is the
 // device memory that state holds (0 before the first call).

@@ -336,7 +336,7 @@ int kz_paged_count_cliques(kz_paged p, int k, uint64_t* count, kz_paged_stats* s
         st.request_refs += p->batch_refs[b];
         // count the batch's roots on the working rows
         CliqueJob job;
-        std::vector<CliqueQuery> q = {CliqueQuery{p->wrow, p->wcol, &p->h_deg, k, r0, r1}};
+        std::vector<CliqueQuery> q = {CliqueQuery{p->wrow, p->wcol, &p->h_deg, k, r0, r1, false}};
         if (int e = clique_job_prepare(job, q, default_buckets())) return e;
         uint64_t c = 0;
         double ms = 0;

@@ -67,6 +67,7 @@ struct Prepared {
     int busy = 0;        // launched queries or helper work using it
     bool preparing = false;
     bool retried = false;
+    uint64_t core_limit = 0;  // bytes its core bitmap may take
 };
 
 // Work for a helper thread.
@@ -270,7 +271,7 @@ void aux_run(AuxJob& j) {
         j.rc = ensure_forward(d);
     } else if (j.type == kJobPrepare) {
         CliqueJob* job = nullptr;
-        j.rc = graph_job(d, j.p->k, &job);
+        j.rc = graph_job(d, j.p->k, &job, j.p->core_limit);
     } else {
         kz_run_stats st;
         j.q->t_start = t0;
@@ -467,18 +468,29 @@ int admit(kz_server_s* s, SQuery* q, int* free_slot) {
                 f->busy = 0;
             }
         }
+        // a job kept from a direct call is adopted; one whose core bitmap
+        // alone takes it past the budget is prepared again without
+        auto job_of = [&]() { return static_cast<CliqueJob*>(d.clique_exec[q->k].get()); };
+        if (job_of() && job_of()->core_bytes && job_of()->bytes > budget_of(s)) d.clique_exec[q->k].reset();
         const bool cached = bool(d.clique_exec[q->k]);
-        const uint64_t est = cached ? static_cast<CliqueJob*>(d.clique_exec[q->k].get())->bytes
-                                    : estimate_bytes(d, q->kind, q->k);
-        if (est > budget_of(s)) {
+        const uint64_t base = cached ? job_of()->bytes : estimate_bytes(d, q->kind, q->k);
+        if (base > budget_of(s)) {
             finish(s, q, KZ_ERR_BUDGET);
             return 1;
         }
+        // the core bitmap is left out where it does not fit the budget
+        uint64_t core = cached ? 0 : clique_core_bytes(d.n, d.oriented ? d.nnz : d.nnz / 2);
+        if (base + core > budget_of(s)) core = 0;
         if (f) f->busy++;  // the job needs it: not a victim for its room
-        const bool room = make_room(s, est);
+        bool room = make_room(s, base + core);
+        if (!room && core) {
+            core = 0;
+            room = make_room(s, base);
+        }
         if (f) f->busy--;
         if (!room) return no_room();
-        p = reserve(s, q->g, q->kind, q->k, est);
+        p = reserve(s, q->g, q->kind, q->k, base + core);
+        p->core_limit = core;
         if (!cached) {
             aux_submit(s->prep, AuxJob{kJobPrepare, q, p, 0, 0});
             return 0;

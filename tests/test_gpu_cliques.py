@@ -232,3 +232,49 @@ def test_wave_tasks_dealt_and_from_the_cursor(kzdev, n, m):
     for _ in range(2):
         assert dg.count_cliques(3, "persistent") == want
     dg.release()
+
+
+@pytest.mark.parametrize("k", [3, 4, 5])
+def test_core_rows_at_the_edges_of_their_tiles(kzdev, k):
+    """Rows gathered from the core bitmap: roots of 2 .. 1100 candidates in
+    one graph (every shared-load width, 32-row tiles, 64-candidate words, row
+    lines and the hub path), wholly or partly inside the core."""
+    import numpy as np
+
+    kz = kzdev
+    rng = np.random.default_rng(k)
+    sizes = [2, 3, 8, 9, 16, 17, 32, 33, 63, 64, 65, 96, 127, 128, 129, 511, 512, 513, 831, 832, 833, 1023, 1024, 1100]
+    top = 1200  # ids the roots' lists fall on, themselves a random graph
+    src, dst = [], []
+    a, b = np.triu_indices(top, 1)
+    keep = rng.random(len(a)) < 0.03
+    src.append(a[keep] + len(sizes)), dst.append(b[keep] + len(sizes))
+    for r, d in enumerate(sizes):
+        v = rng.choice(top, d, replace=False) + len(sizes)
+        src.append(np.full(d, r)), dst.append(v)
+    for extra in (0, 60000):  # a tail of sparse ids below: the core then covers the top only
+        s, t = np.concatenate(src) + extra, np.concatenate(dst) + extra
+        if extra:
+            s = np.concatenate([s, np.arange(extra)])
+            t = np.concatenate([t, (np.arange(extra) + 1 + rng.integers(0, 40, extra))])
+        g = _forward_graph(kz, s, t)
+        want = oracle.run_app(APP[k], g.rowptr, g.col)[1][0]
+        dg = g.to_device()
+        print(f"[case] core rows k={k} tail={extra}", flush=True)
+        assert dg.count_cliques(k, "persistent") == want
+        assert dg.count_cliques(k, "persistent") == want
+        dg.release()
+
+
+def _forward_graph(kz, src, dst):
+    """The oriented graph u -> v (v > u) of the given pairs, ids kept."""
+    import tempfile
+
+    import numpy as np
+    pairs = np.unique(np.stack([src, dst], 1).astype(np.uint32), axis=0)
+    nv = int(pairs.max()) + 1
+    with tempfile.NamedTemporaryFile(suffix=".dgraph") as f:
+        f.write(np.uint32(nv).tobytes() + np.uint64(len(pairs)).tobytes() + np.zeros(2, np.int32).tobytes())
+        f.write(pairs.tobytes())
+        f.flush()
+        return kz.load_dgraph(f.name)
