@@ -415,37 +415,46 @@ __device__ __forceinline__ void count5_edges(const unsigned long long* rows, uin
 // ------------------------------------------------------- MFMA 4-cliques --
 // With A the d x d 0/1 matrix of the root's DAG (A[i][j] = bit j of row i,
 // j > i), the 4-cliques at the root are sum_{i<j} A[i][j] * |row_i & row_j|
-// = sum_{i,j} A[i][j] * (A A^T)[i][j]: an int8 GEMM masked by A.  The
-// workgroup's waves take 32 x 32 tiles (I, J), J >= I, of A A^T, one
-// v_mfma_i32_32x32x32_i8 per 32 columns; A A^T[i][j] only gathers columns
-// l > j >= 32 J, so column blocks start at J.  Operands come straight from
-// the LDS bitmap: lane l holds row (or column) l % 32 of the tile and the 16
-// bits (l / 32) of the 32-column block, expanded to 16 bytes of 0/1; the
-// k order inside a block is the same for both operands, so any order works.
-// Accumulator r of lane l holds tile row (r / 4) * 8 + (l / 32) * 4 + r % 4,
-// column l % 32.
-typedef int kz_v4i __attribute__((ext_vector_type(4)));
-typedef int kz_v16i __attribute__((ext_vector_type(16)));
+// = sum_{i,j} A[i][j] * (A A^T)[i][j]: a product masked by A.  The waves take
+// 32 x 32 tiles (I, J), J >= I, of A A^T, one FP4 MFMA (32 x 32 x 64) per
+// 64-bit word of the rows; A A^T[i][j] only gathers columns l > j >= 32 J, so
+// words start at J / 2 (a tile of odd J also takes the low half of its first
+// word, whose products are zero: row j has no bit l <= j).
+//
+// Why FP4: a bit of a row word is already in place as a bit of a 4-bit code
+// (E2M1: 1 = 0.5, 2 = 1, 4 = 2), so an operand is the word masked four times,
+// 11 VALU instructions for both operands of 64 columns (int8 operands took 48
+// and bound the count: 92 % VALU busy in the 833-1024 group).  The two sides
+// use codes whose product is 1; the order of the columns is the same for
+// both, so it does not matter which code a column takes.  Products and sums
+// are integers: accumulators start at 2^23 and hold 2^23 + n exactly (n <= d
+// <= 8192), whose low 24 bits are n.  Lane l holds row (or column) l % 32 of
+// the tile and half l / 32 of the word; accumulator r of lane l is tile row
+// (r / 4) * 8 + (l / 32) * 4 + r % 4, column l % 32 (checked on the device
+// over 122,880 sums up to 8192).
+typedef int kz_v8i __attribute__((ext_vector_type(8)));
+typedef float kz_v16f __attribute__((ext_vector_type(16)));
 
-// Bits off .. off + 15 of w as 16 bytes of 0 or 1 (bit off + t in byte t):
-// each nibble is a bit-field extract, a 24-bit multiply spreads its bits 7
-// apart and the mask keeps one per byte.
-__device__ __forceinline__ kz_v4i bits_to_bytes(uint32_t w, uint32_t off) {
-    kz_v4i r;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        r[q] = int(__umul24(__builtin_amdgcn_ubfe(w, off + 4u * uint32_t(q), 4u), 0x00204081u) & 0x01010101u);
-    return r;
+// A's rows: column 4 e + t of the half word as the code 2^t of element e (t <
+// 3), column 4 e + 3 as code 2; B's columns: the codes of the inverse values.
+__device__ __forceinline__ kz_v8i fp4_rows(uint32_t w) {
+    const uint32_t h = w >> 2;
+    return kz_v8i{int(w & 0x11111111u), int(w & 0x22222222u), int(w & 0x44444444u), int(h & 0x22222222u), 0, 0, 0, 0};
+}
+__device__ __forceinline__ kz_v8i fp4_cols(uint32_t w) {
+    const uint32_t h = w >> 2;
+    return kz_v8i{int((w << 2) & 0x44444444u), int(w & 0x22222222u), int(h & 0x11111111u), int(h & 0x22222222u),
+                  0, 0, 0, 0};
 }
 
-// This lane's share of sum_r A[i_r][j] * c[r] over its 16 rows i_r of tile
+// This lane's share of sum_r A[i_r][j] * n[r] over its 16 rows i_r of tile
 // row block I (accumulator r of lane l holds row (r / 4) * 8 + (l / 32) * 4 +
 // r % 4) and its column j: A[i_r][j] read as the 32-bit half of each row's
-// word that holds bit j (entries of A A^T are at most d < 2^24: 24-bit
+// word that holds bit j, n[r] the low 24 bits of the accumulator (24-bit
 // multiply-adds).
 template <bool TRI>
 __device__ __forceinline__ uint32_t mask_tile(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t I,
-                                              uint32_t j, const kz_v16i& c) {
+                                              uint32_t j, const kz_v16f& c) {
     const uint32_t lane = threadIdx.x & 63;
     uint32_t s = 0;
     if (j < d) {
@@ -456,133 +465,97 @@ __device__ __forceinline__ uint32_t mask_tile(const unsigned long long* rows, ui
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const uint32_t ir = ib + (r >> 2) * 8 + (r & 3);
-                s = __umul24(__builtin_amdgcn_ubfe(cw[2 * ir], b5, 1u), uint32_t(c[r])) + s;
+                s = __umul24(__builtin_amdgcn_ubfe(cw[2 * ir], b5, 1u), __float_as_uint(c[r])) + s;
             }
         } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const uint32_t ir = ib + (r >> 2) * 8 + (r & 3);
                 const uint32_t a = ir < d ? __builtin_amdgcn_ubfe(cw[2 * ir], b5, 1u) : 0u;
-                s = __umul24(a, uint32_t(c[r])) + s;
+                s = __umul24(a, __float_as_uint(c[r])) + s;
             }
         }
     }
     return s;
 }
 
-// One 32 x 32 tile (I, J >= I) of A A^T masked by A: this lane's share of
-// sum A[i][j] * (A A^T)[i][j] over the tile.  rows is a word-major bitmap
-// (word kk of row i at rows[word_base<TRI>(kk, ws) + i]) in LDS or in HBM.
-// Every row a tile reads exists in the packed form: rows below 32 (J + 1)
-// from words kk >= J / 2, and rows clamped to d - 1 only in the last word.
-// Call with every lane of the wave.
-template <bool TRI = false>
-__device__ __forceinline__ uint32_t mfma4_tile(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t I,
-                                               uint32_t J) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t nb = (d + 31) >> 5;
-    const uint32_t i = 32 * I + (lane & 31), j = 32 * J + (lane & 31);
-    // rows past d read row d - 1: their products land in tile rows and
-    // columns that the mask below leaves out
-    const uint32_t ic = i < d ? i : d - 1, jc = j < d ? j : d - 1;
-    const uint32_t hs = 16 * (lane >> 5);
-    // one 64-bit word = two 32-column blocks, read once, the next word's
-    // reads issued before this one's products; word J / 2 may start at its
-    // high block (J odd), the last word may end after its low block (nb odd)
-    kz_v16i c;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) c[r] = 0;
-    const uint32_t wend = (nb + 1) >> 1;
-    uint32_t kw = J >> 1;
-    unsigned long long wi = rows[word_base<TRI>(kw, ws) + ic], wj = rows[word_base<TRI>(kw, ws) + jc];
-    if (J & 1u) {
-        const uint32_t hi_i = uint32_t(wi >> 32), hi_j = uint32_t(wj >> 32);
-        ++kw;
-        if (kw < wend) {
-            wi = rows[word_base<TRI>(kw, ws) + ic];
-            wj = rows[word_base<TRI>(kw, ws) + jc];
-        }
-        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(bits_to_bytes(hi_i, hs), bits_to_bytes(hi_j, hs), c, 0, 0, 0);
-    }
-    while (2 * kw + 1 < nb) {
-        const uint32_t lo_i = uint32_t(wi), hi_i = uint32_t(wi >> 32);
-        const uint32_t lo_j = uint32_t(wj), hi_j = uint32_t(wj >> 32);
-        ++kw;
-        if (kw < wend) {
-            wi = rows[word_base<TRI>(kw, ws) + ic];
-            wj = rows[word_base<TRI>(kw, ws) + jc];
-        }
-        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(bits_to_bytes(lo_i, hs), bits_to_bytes(lo_j, hs), c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(bits_to_bytes(hi_i, hs), bits_to_bytes(hi_j, hs), c, 0, 0, 0);
-    }
-    if (2 * kw < nb)
-        c = __builtin_amdgcn_mfma_i32_32x32x32_i8(bits_to_bytes(uint32_t(wi), hs), bits_to_bytes(uint32_t(wj), hs), c,
-                                                  0, 0, 0);
-    return mask_tile<TRI>(rows, ws, d, I, j, c);
-}
-
-// Four 32 x 32 tiles (2 bI + a, 2 bJ + b), a, b in {0, 1}, of A A^T masked
-// by A in one pass over the 64-bit words kw >= bJ (block (bI, bJ), bJ >=
-// bI, of the W x W word blocks).  Each word's operands, the rows of the two
-// I tiles and of the two J tiles, are expanded to bytes once and feed four
-// MFMAs per 32-column half: 12 VALU of expansion per MFMA instead of 24, and
-// half the row reads.  Tile 2 bJ + 1 also takes the low half of word bJ,
-// whose products are zero (row j has no bit l <= j).  Tiles below the
-// diagonal (2 bI + 1 > 2 bJ) or past the last row are computed on clamped
-// rows and left out; a clamped row, d - 1, is empty.  The accumulators take
-// 64 registers: for kernels with a budget of at least 128.
-template <bool TRI>
-__device__ __forceinline__ uint32_t mfma4_block(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t bI,
-                                                uint32_t bJ) {
+// N x N tiles (I0 + a, J0 + b) of A A^T masked by A in one pass over the
+// words kw >= J0 / 2 (I0, J0 multiples of N): this lane's share of the sum.
+// Each word's operands are built once and feed N * N MFMAs, the next word's
+// reads issued before this one's products.  rows is a word-major bitmap (word
+// kk of row i at rows[word_base<TRI>(kk, ws) + i]) in LDS or (HBM, N = 2) in
+// memory, where the mask comes by lane permutes of the first word read, not
+// by 64 loads.  Every row a tile reads exists in the packed form: rows below
+// 32 (J + 1) from words kk >= J / 2, and rows clamped to d - 1 only in the
+// last word.  Tiles below the diagonal or past the last row are computed on
+// clamped rows and left out; a clamped row, d - 1, is empty.  Accumulators:
+// 16 N N registers.  Call with every lane of the wave.
+template <bool TRI, int N, bool HBM = false>
+__device__ __forceinline__ uint32_t mfma4_tiles(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t I0,
+                                                uint32_t J0) {
+    static_assert(!HBM || N == 2, "the mask word needs an even J0");
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t nb = (d + 31) >> 5, W = (d + 63) >> 6;
-    const uint32_t i0 = 64 * bI + (lane & 31), j0 = 64 * bJ + (lane & 31);
-    const uint32_t ic0 = i0 < d ? i0 : d - 1, ic1 = i0 + 32 < d ? i0 + 32 : d - 1;
-    const uint32_t jc0 = j0 < d ? j0 : d - 1, jc1 = j0 + 32 < d ? j0 + 32 : d - 1;
-    const uint32_t hs = 16 * (lane >> 5);
-    kz_v16i c00, c01, c10, c11;
+    const uint32_t* half = reinterpret_cast<const uint32_t*>(rows) + (lane >> 5);
+    uint32_t ic[N], jc[N];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) c00[r] = c01[r] = c10[r] = c11[r] = 0;
-    uint32_t kw = bJ;
-    unsigned long long a0 = rows[word_base<TRI>(kw, ws) + ic0], a1 = rows[word_base<TRI>(kw, ws) + ic1];
-    unsigned long long b0 = rows[word_base<TRI>(kw, ws) + jc0], b1 = rows[word_base<TRI>(kw, ws) + jc1];
-    while (kw < W) {
-        const uint32_t kn = kw + 1;
-        unsigned long long na0 = 0, na1 = 0, nb0 = 0, nb1 = 0;
-        if (kn < W) {
-            const uint32_t base = word_base<TRI>(kn, ws);
-            na0 = rows[base + ic0];
-            na1 = rows[base + ic1];
-            nb0 = rows[base + jc0];
-            nb1 = rows[base + jc1];
-        }
-        {
-            const kz_v4i A0 = bits_to_bytes(uint32_t(a0), hs), A1 = bits_to_bytes(uint32_t(a1), hs);
-            const kz_v4i B0 = bits_to_bytes(uint32_t(b0), hs), B1 = bits_to_bytes(uint32_t(b1), hs);
-            c00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A0, B0, c00, 0, 0, 0);
-            c01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A0, B1, c01, 0, 0, 0);
-            c10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, B0, c10, 0, 0, 0);
-            c11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, B1, c11, 0, 0, 0);
-        }
-        if (2 * kw + 1 < nb) {  // the word's high half holds columns below d
-            const kz_v4i A0 = bits_to_bytes(uint32_t(a0 >> 32), hs), A1 = bits_to_bytes(uint32_t(a1 >> 32), hs);
-            const kz_v4i B0 = bits_to_bytes(uint32_t(b0 >> 32), hs), B1 = bits_to_bytes(uint32_t(b1 >> 32), hs);
-            c00 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A0, B0, c00, 0, 0, 0);
-            c01 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A0, B1, c01, 0, 0, 0);
-            c10 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, B0, c10, 0, 0, 0);
-            c11 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A1, B1, c11, 0, 0, 0);
-        }
-        a0 = na0;
-        a1 = na1;
-        b0 = nb0;
-        b1 = nb1;
-        kw = kn;
+    for (int a = 0; a < N; ++a) {
+        const uint32_t i = 32 * (I0 + uint32_t(a)) + (lane & 31), j = 32 * (J0 + uint32_t(a)) + (lane & 31);
+        ic[a] = 2 * (i < d ? i : d - 1);
+        jc[a] = 2 * (j < d ? j : d - 1);
     }
-    const uint32_t I0 = 2 * bI, J0 = 2 * bJ;
-    uint32_t s = mask_tile<TRI>(rows, ws, d, I0, j0, c00);
-    if (J0 + 1 < nb) s += mask_tile<TRI>(rows, ws, d, I0, j0 + 32, c01);
-    if (I0 + 1 < nb && I0 + 1 <= J0) s += mask_tile<TRI>(rows, ws, d, I0 + 1, j0, c10);
-    if (J0 + 1 < nb && I0 + 1 < nb) s += mask_tile<TRI>(rows, ws, d, I0 + 1, j0 + 32, c11);
+    kz_v16f c[N][N];
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+#pragma unroll
+        for (int b = 0; b < N; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) c[a][b][r] = 8388608.0f;
+    uint32_t kw = J0 >> 1;
+    uint32_t wi[N], wj[N], first[N];
+    auto load = [&](uint32_t k) {
+        const uint32_t base = 2 * word_base<TRI>(k, ws);
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            wi[a] = half[base + ic[a]];
+            wj[a] = half[base + jc[a]];
+        }
+    };
+    load(kw);
+#pragma unroll
+    for (int a = 0; a < N; ++a) first[a] = wi[a];
+    while (kw < W) {
+        kz_v8i A[N], B[N];
+#pragma unroll
+        for (int a = 0; a < N; ++a) {
+            A[a] = fp4_rows(wi[a]);
+            B[a] = fp4_cols(wj[a]);
+        }
+        if (++kw < W) load(kw);
+#pragma unroll
+        for (int a = 0; a < N; ++a)
+#pragma unroll
+            for (int b = 0; b < N; ++b)
+                c[a][b] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A[a], B[b], c[a][b], 4, 4, 0, 0, 0, 0);
+    }
+    uint32_t s = 0;
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+#pragma unroll
+        for (int b = 0; b < N; ++b) {
+            const uint32_t I = I0 + uint32_t(a), J = J0 + uint32_t(b);
+            if (I > J || J >= nb) continue;
+            if constexpr (HBM) {
+                // half b of row i's word J0 / 2 is on lane i % 32 + 32 b
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const uint32_t m = __shfl(first[a], int((lane >> 5) * 4 + 32u * uint32_t(b) + (r >> 2) * 8 + (r & 3)));
+                    s = __umul24(__builtin_amdgcn_ubfe(m, lane & 31u, 1u), __float_as_uint(c[a][b][r])) + s;
+                }
+            } else {
+                s += mask_tile<TRI>(rows, ws, d, I, 32 * J + (lane & 31), c[a][b]);
+            }
+        }
     return s;
 }
 
@@ -595,83 +568,19 @@ __device__ __forceinline__ void tile_coords(uint32_t t, uint32_t* I, uint32_t* J
     *I = t - j * (j + 1) / 2;
 }
 
-// Tiles go to the workgroup's waves from a counter in LDS (ctr, zeroed
-// before a barrier), the next tile's atomic issued ahead: tile t = J (J + 1)
-// / 2 + I, so the costly tiles (small J: the most 64-bit words) come first
-// and the waves finish together.
-// Two 32 x 32 tiles (I, 2 bJ) and (I, 2 bJ + 1), I <= 2 bJ + 1, of A A^T
-// masked by A in one pass over the words kw >= bJ: the row block I operand
-// is expanded once per half for two MFMAs (18 VALU of expansion per MFMA
-// instead of 24); two accumulators (32 registers).  Zero products and
-// clamped rows as in mfma4_block.
-template <bool TRI>
-__device__ __forceinline__ uint32_t mfma4_pair(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t I,
-                                               uint32_t bJ) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t nb = (d + 31) >> 5, W = (d + 63) >> 6;
-    const uint32_t i = 32 * I + (lane & 31), j0 = 64 * bJ + (lane & 31);
-    const uint32_t ic = i < d ? i : d - 1;
-    const uint32_t jc0 = j0 < d ? j0 : d - 1, jc1 = j0 + 32 < d ? j0 + 32 : d - 1;
-    const uint32_t hs = 16 * (lane >> 5);
-    kz_v16i c0, c1;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) c0[r] = c1[r] = 0;
-    uint32_t kw = bJ;
-    unsigned long long a = rows[word_base<TRI>(kw, ws) + ic];
-    unsigned long long b0 = rows[word_base<TRI>(kw, ws) + jc0], b1 = rows[word_base<TRI>(kw, ws) + jc1];
-    while (kw < W) {
-        const uint32_t kn = kw + 1;
-        unsigned long long na = 0, nb0 = 0, nb1 = 0;
-        if (kn < W) {
-            const uint32_t base = word_base<TRI>(kn, ws);
-            na = rows[base + ic];
-            nb0 = rows[base + jc0];
-            nb1 = rows[base + jc1];
-        }
-        {
-            const kz_v4i A = bits_to_bytes(uint32_t(a), hs);
-            c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, bits_to_bytes(uint32_t(b0), hs), c0, 0, 0, 0);
-            c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, bits_to_bytes(uint32_t(b1), hs), c1, 0, 0, 0);
-        }
-        if (2 * kw + 1 < nb) {
-            const kz_v4i A = bits_to_bytes(uint32_t(a >> 32), hs);
-            c0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, bits_to_bytes(uint32_t(b0 >> 32), hs), c0, 0, 0, 0);
-            c1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(A, bits_to_bytes(uint32_t(b1 >> 32), hs), c1, 0, 0, 0);
-        }
-        a = na;
-        b0 = nb0;
-        b1 = nb1;
-        kw = kn;
-    }
-    uint32_t s = 0;
-    if (I <= 2 * bJ) s = mask_tile<TRI>(rows, ws, d, I, j0, c0);
-    if (2 * bJ + 1 < nb) s += mask_tile<TRI>(rows, ws, d, I, j0 + 32, c1);
-    return s;
-}
-
-// (I, bJ) of pair t: pairs come by bJ, I = 0 .. 2 bJ + 1 (0 .. nb - 1 for
-// the last word), so pair t of bJ < W - 1 is t = bJ (bJ + 1) + I.
-__device__ __forceinline__ void pair_coords(uint32_t t, uint32_t W, uint32_t* I, uint32_t* bJ) {
-    if (t >= (W - 1) * W) {
-        *bJ = W - 1;
-        *I = t - (W - 1) * W;
-        return;
-    }
-    uint32_t b = uint32_t((sqrtf(4.0f * float(t) + 1.0f) - 1.0f) * 0.5f);
-    if (b * (b + 1) > t) --b;
-    if ((b + 1) * (b + 2) <= t) ++b;
-    *bJ = b;
-    *I = t - b * (b + 1);
-}
-
-// BLK: tile pairs (mfma4_pair) instead of single tiles, for kernels whose
-// register budget holds their two accumulators.
-template <bool TRI, bool BLK = false>
+// 4-cliques of one root's rows in LDS: tiles go to the workgroup's waves from
+// a counter in LDS (ctr, zeroed before a barrier), the next tile's atomic
+// issued ahead, the costly ones (small J: the most words) first, so that the
+// waves finish together.  N = 2: 2 x 2 tile blocks instead of single tiles,
+// for kernels whose register budget holds their four accumulators (RMAT-24,
+// the two groups of the 512-1024 bucket: single tiles 10.9 ms, pairs 10.5,
+// blocks 9.8; pairs at 6 waves per SIMD spill: 128-512 30.0 -> 33.2).
+template <bool TRI, int N>
 __device__ __forceinline__ void count_rows_mfma4(const unsigned long long* rows, uint32_t ws, uint32_t d,
                                                  uint32_t* ctr, unsigned long long& acc) {
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t nb = (d + 31) >> 5, W = (d + 63) >> 6;
-    const uint32_t ntiles = BLK ? (W - 1) * W + nb : nb * (nb + 1) / 2;
+    const uint32_t nb = (d + 32 * N - 1) / (32 * N);
+    const uint32_t ntiles = nb * (nb + 1) / 2;
     uint32_t tile = 0;
     if (lane == 0) tile = atomicAdd(ctr, 1u);
     tile = wave_bcast(tile);
@@ -679,13 +588,8 @@ __device__ __forceinline__ void count_rows_mfma4(const unsigned long long* rows,
         uint32_t tn = 0;
         if (lane == 0) tn = atomicAdd(ctr, 1u);
         uint32_t I, J;
-        if (BLK) {
-            pair_coords(tile, W, &I, &J);
-            acc += mfma4_pair<TRI>(rows, ws, d, I, J);
-        } else {
-            tile_coords(tile, &I, &J);
-            acc += mfma4_tile<TRI>(rows, ws, d, I, J);
-        }
+        tile_coords(tile, &I, &J);
+        acc += mfma4_tiles<TRI, N>(rows, ws, d, N * wave_bcast(I), N * wave_bcast(J));
         tile = wave_bcast(tn);
     }
 }
@@ -746,6 +650,22 @@ __device__ __forceinline__ void build_rows_block(const uint64_t* __restrict__ ro
         if (K == 3) acc += 1;
         else set_row_bit<TRI>(rows_out, ws, r, j);
     });
+}
+
+// (I, kk) of tile t of 32 rows by one 64-candidate word: tiles come by word,
+// I = 0 .. 2 kk + 1 (0 .. ceil(d / 32) - 1 for the last), so tile t of kk < W
+// - 1 is t = kk (kk + 1) + I.
+__device__ __forceinline__ void pair_coords(uint32_t t, uint32_t W, uint32_t* I, uint32_t* kk) {
+    if (t >= (W - 1) * W) {
+        *kk = W - 1;
+        *I = t - (W - 1) * W;
+        return;
+    }
+    uint32_t b = uint32_t((sqrtf(4.0f * float(t) + 1.0f) - 1.0f) * 0.5f);
+    if (b * (b + 1) > t) --b;
+    if ((b + 1) * (b + 2) <= t) ++b;
+    *kk = b;
+    *I = t - b * (b + 1);
 }
 
 // Rows [lo, d) of a root from the core: the workgroup's waves take tiles of
@@ -878,7 +798,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(WPE))) voi
                 else rows[word_base<TRI>(kk, d) + i] = w;
             });
         __syncthreads();
-        if (K == 4) count_rows_mfma4<TRI, (WPE <= 4)>(rows, d, d, &sTile, acc);
+                if (K == 4) count_rows_mfma4<TRI, (WPE <= 4 ? 2 : 1)>(rows, d, d, &sTile, acc);
         else if (K == 5) {
             if (W <= 8) count5_edges<TRI>(rows, d, rp, sTmp, &sTile, acc);
             else count_rows<K, true, TRI>(rows, d, d, 0, 0, acc, &sTile);
@@ -1002,17 +922,23 @@ __global__ __launch_bounds__(256) void hub_core_kernel(const QueryRef* __restric
     unsigned long long acc = 0;
     uint32_t qcur = 0xFFFFFFFFu;
     TaskChunk chunk(ntiles, gridDim.x * (blockDim.x >> 6), 8);
+    HubMeta hm{};
+    uint32_t h0 = 0, h1 = 0;  // tiles of hub hm: its meta and the search are kept between them
     while (true) {
         const uint32_t t = wave_next_task(chunk, cursor);
         if (t >= ntiles) break;
-        const uint32_t h = wave_bcast(row_of(tile_prefix, nhubs, t));
-        const HubMeta hm = hubs[h];
+        if (t < h0 || t >= h1) {
+            const uint32_t h = wave_bcast(row_of(tile_prefix, nhubs, t));
+            hm = hubs[h];
+            h0 = wave_bcast(tile_prefix[h]);
+            h1 = h + 1 < nhubs ? wave_bcast(tile_prefix[h + 1]) : ntiles;
+        }
         if (hm.q != qcur) {
             if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
             qcur = hm.q;
         }
         uint32_t I, kk;
-        pair_coords(t - tile_prefix[h], hm.W, &I, &kk);
+        pair_coords(t - h0, hm.W, &I, &kk);
         I = wave_bcast(I);
         kk = wave_bcast(kk);
         if (32 * I + 32 <= hm.k0) continue;
@@ -1107,7 +1033,7 @@ __global__ __launch_bounds__(256) void hub_count_kernel(const HubMeta* __restric
 }
 
 // 4-cliques of the hubs on MFMA: one wave per 2 x 2 block of 32 x 32 tiles
-// of a hub's A A^T (mfma4_block), the blocks of every hub (tile_prefix:
+// of a hub's A A^T (mfma4_tiles), the blocks of every hub (tile_prefix:
 // exclusive prefix over hubs of W (W + 1) / 2, W = ceil(d / 64)) taken from
 // one cursor, read from the hub's word-major slab rows in HBM.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void hub_mfma4_kernel(const HubMeta* __restrict__ hubs, uint32_t nhubs,
@@ -1118,18 +1044,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void h
     unsigned long long acc = 0;
     uint32_t qcur = 0xFFFFFFFFu;
     TaskChunk chunk(ntiles, gridDim.x * (blockDim.x >> 6), 8);
+    HubMeta hm{};
+    uint32_t h0 = 0, h1 = 0;  // tiles of hub hm: its meta and the search are kept between them
     while (true) {
         const uint32_t t = wave_next_task(chunk, cursor);
         if (t >= ntiles) break;
-        const uint32_t h = wave_bcast(row_of(tile_prefix, nhubs, t));
-        const HubMeta hm = hubs[h];
+        if (t < h0 || t >= h1) {
+            const uint32_t h = wave_bcast(row_of(tile_prefix, nhubs, t));
+            hm = hubs[h];
+            h0 = wave_bcast(tile_prefix[h]);
+            h1 = h + 1 < nhubs ? wave_bcast(tile_prefix[h + 1]) : ntiles;
+        }
         if (hm.q != qcur) {
             if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
             qcur = hm.q;
         }
         uint32_t I, J;
-        tile_coords(t - tile_prefix[h], &I, &J);
-        acc += mfma4_block<false>(slab + hm.slab_off, hm.d, hm.d, I, J);
+        tile_coords(t - h0, &I, &J);
+        acc += mfma4_tiles<false, 2, true>(slab + hm.slab_off, hm.d, hm.d, 2 * wave_bcast(I), 2 * wave_bcast(J));
     }
     if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
 }
