@@ -18,12 +18,19 @@
 //     so N_l(v), the neighbours of v with label l, is one contiguous segment
 //     whose bounds are two words of a per-vertex table of label offsets
 //     (L + 1 u32 per vertex, written by the same sort);
-//   * one wave per root vertex (the vertices of the root label); domains are
-//     bitmaps in HBM (one per candidate and position, set with atomicOr) and
-//     their sizes come from one popcount pass per level;
-//   * a level's candidates are all known before it runs, so every candidate
-//     of a level is launched back to back into its own bitmaps and the level
-//     synchronises once.
+//   * one wave per root vertex (the vertices of the root label) of more than
+//     kLaneDegree neighbours, one lane per root below: a segment then holds a
+//     few ids, and a wave per root left most of its lanes idle in the same
+//     chain of dependent loads (the run below: 21 -> 10.4 ms; 16 / 64 / 256
+//     neighbours 10.9 / 10.4 / 13.9 ms).  Domains are bitmaps in HBM (one per
+//     candidate and position, set with atomicOr) and their sizes come from
+//     one popcount pass per level;
+//   * a level's candidates are all known before it runs, so one launch per
+//     domain kernel takes every candidate of the level (a grid row each) into
+//     its own bitmaps and the level synchronises once.  A candidate alone has
+//     too few roots to fill the chip and ends on its largest root's wave (60
+//     us a launch, whatever its work: 120 K vertices, 6 labels, 1,900 launches
+//     142 ms a run; one launch per level and kernel 21 ms).
 // Existence rules (labels l0..l3 of pattern positions 0..3; c_l(v) = |N_l(v)|):
 //   edge      (v0-v1): D0 = {v0 : N_l1(v0) non-empty}, D1 = the union of those
 //             N_l1(v0);
@@ -56,6 +63,7 @@
 namespace kz {
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
+constexpr uint32_t kLaneDegree = 64;  // roots of at most this degree run on one lane
 
 // Device state of a labelled graph (kz_graph_set_labels).
 struct FsmState {
@@ -63,7 +71,8 @@ struct FsmState {
     uint32_t* lab = nullptr;    // labels[n]
     uint32_t* lcol = nullptr;   // neighbour lists sorted by (label, id), same rowptr
     uint32_t* loff = nullptr;   // per vertex, L + 1 offsets of the label segments in its row
-    uint32_t* vlist = nullptr;  // vertices grouped by label
+    uint32_t* vlist = nullptr;  // vertices grouped by label, largest degree first
+    uint32_t* groups = nullptr;  // per label: start in vlist, first root of at most kLaneDegree neighbours; then the end
     std::vector<uint32_t> voff;    // host: vlist offsets per label (L + 1)
     uint64_t bytes = 0;
     ~FsmState() {
@@ -71,6 +80,7 @@ struct FsmState {
         hipFree(lcol);
         hipFree(loff);
         hipFree(vlist);
+        hipFree(groups);
     }
 };
 
@@ -145,12 +155,27 @@ __device__ __forceinline__ Seg seg_of(const uint64_t* __restrict__ rowptr, const
     return Seg{b + ldg(o, 0), b + ldg(o, 1)};
 }
 
-__device__ __forceinline__ void mark(uint32_t* bm, uint32_t v) { atomicOr(&bm[v >> 5], 1u << (v & 31)); }
+// Sets v's bit.  Most marks repeat one already set (a vertex joins a domain
+// through every embedding it is in): those are a cached load, not an atomic.
+__device__ __forceinline__ void mark(uint32_t* bm, uint32_t v) {
+    const uint32_t bit = 1u << (v & 31);
+    if (!(ldg(bm, v >> 5) & bit)) atomicOr(&bm[v >> 5], bit);
+}
 
-// Marks every id of lcol[s.b, s.e) except x1, x2 (kNone: none) across the wave.
+// A root runs on one wave (WAVE: the lanes take the entries of its segments)
+// or, when its lists are short, on one lane.
+template <bool WAVE>
+constexpr uint32_t kStep = WAVE ? 64u : 1u;
+template <bool WAVE>
+__device__ __forceinline__ uint32_t sub_lane() {
+    return WAVE ? threadIdx.x & 63 : 0u;
+}
+
+// Marks every id of lcol[s.b, s.e) except x1, x2 (kNone: none).
+template <bool WAVE>
 __device__ __forceinline__ void mark_seg(uint32_t* bm, const uint32_t* __restrict__ lcol, Seg s, uint32_t x1,
                                          uint32_t x2) {
-    for (uint64_t k = s.b + (threadIdx.x & 63); k < s.e; k += 64) {
+    for (uint64_t k = s.b + sub_lane<WAVE>(); k < s.e; k += kStep<WAVE>) {
         const uint32_t w = ldg(lcol, k);
         if (w != x1 && w != x2) mark(bm, w);
     }
@@ -179,148 +204,179 @@ struct FsmArgs {
     const uint32_t* lcol;
     const uint32_t* loff;
     uint32_t L1;  // labels + 1: the offset table's row length
-    const uint32_t* roots;
-    uint32_t nroots;
-    uint32_t l[4];
-    uint32_t* bm;  // 4 bitmaps of W words
+    const uint32_t* vlist;   // vertices grouped by label, largest degree first
+    const uint32_t* groups;  // per label: its start in vlist and its first root for one lane
+    const uint32_t* labels;  // 4 labels per candidate (blockIdx.y)
+    uint32_t* bm;            // 4 bitmaps of W words per candidate
     uint32_t W;
 };
 
-// Running intersection of wave lanes' exclusion sets {x1, x2} over lanes
-// with ok set (i1, i2 uniform; `any` set once a first set was taken).
+// Running intersection {i1, i2} of the exclusion sets {x1, x2} of the entries
+// with ok set (`any` set once a first set was taken): those of the wave's
+// lanes, or the one lane's own.
+template <bool WAVE>
 __device__ __forceinline__ void fold_exclusions(bool ok, uint32_t x1, uint32_t x2, bool& any, uint32_t& i1,
                                                 uint32_t& i2) {
-    const unsigned long long okm = __ballot(ok);
-    if (!okm) return;
-    if (!any) {
-        const int f = __builtin_ctzll(okm);
-        i1 = wave_lane(x1, uint32_t(f));
-        i2 = wave_lane(x2, uint32_t(f));
-        any = true;
+    if constexpr (WAVE) {
+        const unsigned long long okm = __ballot(ok);
+        if (!okm) return;
+        if (!any) {
+            const int f = __builtin_ctzll(okm);
+            i1 = wave_lane(x1, uint32_t(f));
+            i2 = wave_lane(x2, uint32_t(f));
+            any = true;
+        }
+        if (i1 != kNone && __ballot(ok && x1 != i1 && x2 != i1)) i1 = kNone;
+        if (i2 != kNone && __ballot(ok && x1 != i2 && x2 != i2)) i2 = kNone;
+    } else if (ok) {
+        if (!any) {
+            i1 = x1;
+            i2 = x2;
+            any = true;
+        }
+        if (x1 != i1 && x2 != i1) i1 = kNone;
+        if (x1 != i2 && x2 != i2) i2 = kNone;
     }
-    if (i1 != kNone && __ballot(ok && x1 != i1 && x2 != i1)) i1 = kNone;
-    if (i2 != kNone && __ballot(ok && x1 != i2 && x2 != i2)) i2 = kNone;
 }
 
+struct Labels4 {
+    uint32_t l0, l1, l2, l3;
+};
+
+// Adds root v's embeddings of template T to the domains D0 .. D3.
+template <int T, bool WAVE>
+__device__ __forceinline__ void fsm_root(const FsmArgs& a, const Labels4& l, uint32_t* D0, uint32_t v) {
+    constexpr uint32_t kS = kStep<WAVE>;
+    const uint32_t sub = sub_lane<WAVE>();
+    uint32_t* D1 = D0 + a.W;
+    uint32_t* D2 = D0 + 2 * size_t(a.W);
+    uint32_t* D3 = D0 + 3 * size_t(a.W);
+    auto seg = [&](uint32_t x, uint32_t lab) { return seg_of(a.rowptr, a.loff, a.L1, x, lab); };
+    auto any_of = [](bool b) { return WAVE ? __ballot(b) != 0 : b; };
+    if constexpr (T == 1) {  // edge: v = v0
+        const Seg s1 = seg(v, l.l1);
+        if (s1.e > s1.b) {
+            if (sub == 0) mark(D0, v);
+            mark_seg<WAVE>(D1, a.lcol, s1, kNone, kNone);
+        }
+    } else if constexpr (T == 2) {  // wedge: v = v0 (center)
+        const Seg s1 = seg(v, l.l1), s2 = seg(v, l.l2);
+        if (s1.e > s1.b && s2.e - s2.b >= 1 + uint64_t(l.l1 == l.l2)) {
+            if (sub == 0) mark(D0, v);
+            mark_seg<WAVE>(D1, a.lcol, s1, kNone, kNone);
+            mark_seg<WAVE>(D2, a.lcol, s2, kNone, kNone);
+        }
+    } else if constexpr (T == 3) {  // triangle: v = v0, lanes take v1
+        const Seg A = seg(v, l.l2), S1 = seg(v, l.l1);
+        bool any = false;
+        if (A.e > A.b) {
+            for (uint64_t k0 = S1.b; k0 < S1.e; k0 += kS) {
+                const uint64_t k = k0 + sub;
+                bool hit = false;
+                if (k < S1.e) {
+                    const uint32_t v1 = ldg(a.lcol, k);
+                    const Seg B = seg(v1, l.l2);
+                    // walk the shorter list, search the longer
+                    const bool ab = A.e - A.b <= B.e - B.b;
+                    const Seg sm = ab ? A : B, lg = ab ? B : A;
+                    for (uint64_t q = sm.b; q < sm.e; ++q) {
+                        const uint32_t w = ldg(a.lcol, q);
+                        if (seg_has(a.lcol, lg, w)) {
+                            mark(D2, w);
+                            hit = true;
+                        }
+                    }
+                    if (hit) mark(D1, v1);
+                }
+                if (any_of(hit)) any = true;
+            }
+        }
+        if (any && sub == 0) mark(D0, v);
+    } else if constexpr (T == 4) {  // four-chain v2 - v0 - v1 - v3, from the v0 side: v = v0
+        const Seg A2 = seg(v, l.l2), S1 = seg(v, l.l1);
+        const uint64_t s2 = (A2.e - A2.b) - uint64_t(l.l1 == l.l2);
+        bool any = false;
+        uint32_t i1 = kNone, i2 = kNone;
+        if (s2 >= 1) {
+            for (uint64_t k0 = S1.b; k0 < S1.e; k0 += kS) {
+                const uint64_t k = k0 + sub;
+                bool ok = false;
+                uint32_t v1 = kNone, x2 = kNone;
+                if (k < S1.e) {
+                    v1 = ldg(a.lcol, k);
+                    const Seg B3 = seg(v1, l.l3);
+                    const uint64_t s3 = (B3.e - B3.b) - uint64_t(l.l0 == l.l3);
+                    if (s3 >= 1) {
+                        const uint32_t e3 = s3 == 1 ? only_other(a.lcol, B3, v) : kNone;
+                        const uint32_t e2 = s2 == 1 ? only_other(a.lcol, A2, v1) : kNone;
+                        ok = !(s2 == 1 && s3 == 1 && e2 == e3);
+                        x2 = e3;
+                    }
+                    if (ok) mark(D1, v1);
+                }
+                fold_exclusions<WAVE>(ok, v1, x2, any, i1, i2);
+            }
+        }
+        if (any) {
+            if (sub == 0) mark(D0, v);
+            mark_seg<WAVE>(D2, a.lcol, A2, i1, i2);
+        }
+    } else if constexpr (T == 5) {  // four-chain, from the v1 side: v = v1, lanes take v0
+        const Seg B3 = seg(v, l.l3), S0 = seg(v, l.l0);
+        const uint64_t s3 = (B3.e - B3.b) - uint64_t(l.l0 == l.l3);
+        bool any = false;
+        uint32_t j1 = kNone, j2 = kNone;
+        if (s3 >= 1) {
+            for (uint64_t k0 = S0.b; k0 < S0.e; k0 += kS) {
+                const uint64_t k = k0 + sub;
+                bool ok = false;
+                uint32_t v0 = kNone, y2 = kNone;
+                if (k < S0.e) {
+                    v0 = ldg(a.lcol, k);
+                    const Seg A2 = seg(v0, l.l2);
+                    const uint64_t s2 = (A2.e - A2.b) - uint64_t(l.l1 == l.l2);
+                    if (s2 >= 1) {
+                        const uint32_t e2 = s2 == 1 ? only_other(a.lcol, A2, v) : kNone;
+                        const uint32_t e3 = s3 == 1 ? only_other(a.lcol, B3, v0) : kNone;
+                        ok = !(s2 == 1 && s3 == 1 && e2 == e3);
+                        y2 = e2;
+                    }
+                }
+                fold_exclusions<WAVE>(ok, v0, y2, any, j1, j2);
+            }
+        }
+        if (any) mark_seg<WAVE>(D3, a.lcol, B3, j1, j2);
+    } else {  // three-star: v = v1 (center), leaves of labels l0, l2, l3
+        const Seg S0 = seg(v, l.l0), S2 = seg(v, l.l2), S3 = seg(v, l.l3);
+        const uint64_t r0 = 1 + uint64_t(l.l2 == l.l0) + uint64_t(l.l3 == l.l0);
+        const uint64_t r2 = 1 + uint64_t(l.l0 == l.l2) + uint64_t(l.l3 == l.l2);
+        const uint64_t r3 = 1 + uint64_t(l.l0 == l.l3) + uint64_t(l.l2 == l.l3);
+        if (S0.e - S0.b >= r0 && S2.e - S2.b >= r2 && S3.e - S3.b >= r3) {
+            if (sub == 0) mark(D1, v);
+            mark_seg<WAVE>(D0, a.lcol, S0, kNone, kNone);
+            mark_seg<WAVE>(D2, a.lcol, S2, kNone, kNone);
+            mark_seg<WAVE>(D3, a.lcol, S3, kNone, kNone);
+        }
+    }
+}
+
+// Candidate blockIdx.y: its roots of more than kLaneDegree neighbours first,
+// one wave each, then the others, one lane each.
 template <int T>
 __global__ __launch_bounds__(256) void fsm_domain_kernel(FsmArgs a) {
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wid = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const uint32_t wid = wave_bcast(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6));
     const uint32_t nw = gridDim.x * (blockDim.x >> 6);
-    uint32_t* D0 = a.bm;
-    uint32_t* D1 = a.bm + a.W;
-    uint32_t* D2 = a.bm + 2 * size_t(a.W);
-    uint32_t* D3 = a.bm + 3 * size_t(a.W);
-    const uint32_t l0 = a.l[0], l1 = a.l[1], l2 = a.l[2], l3 = a.l[3];
-    for (uint32_t r = wid; r < a.nroots; r += nw) {
-        const uint32_t v = ldg(a.roots, r);
-        if (T == 1) {  // edge: v = v0
-            const Seg s1 = seg_of(a.rowptr, a.loff, a.L1, v, l1);
-            if (s1.e > s1.b) {
-                if (lane == 0) mark(D0, v);
-                mark_seg(D1, a.lcol, s1, kNone, kNone);
-            }
-        } else if (T == 2) {  // wedge: v = v0 (center)
-            const Seg s1 = seg_of(a.rowptr, a.loff, a.L1, v, l1), s2 = seg_of(a.rowptr, a.loff, a.L1, v, l2);
-            if (s1.e > s1.b && s2.e - s2.b >= 1 + uint64_t(l1 == l2)) {
-                if (lane == 0) mark(D0, v);
-                mark_seg(D1, a.lcol, s1, kNone, kNone);
-                mark_seg(D2, a.lcol, s2, kNone, kNone);
-            }
-        } else if (T == 3) {  // triangle: v = v0, lanes take v1
-            const Seg A = seg_of(a.rowptr, a.loff, a.L1, v, l2), S1 = seg_of(a.rowptr, a.loff, a.L1, v, l1);
-            bool any = false;
-            if (A.e > A.b) {
-                for (uint64_t k0 = S1.b; k0 < S1.e; k0 += 64) {
-                    const uint64_t k = k0 + lane;
-                    bool hit = false;
-                    if (k < S1.e) {
-                        const uint32_t v1 = ldg(a.lcol, k);
-                        const Seg B = seg_of(a.rowptr, a.loff, a.L1, v1, l2);
-                        // walk the shorter list, search the longer
-                        const bool ab = A.e - A.b <= B.e - B.b;
-                        const Seg sm = ab ? A : B, lg = ab ? B : A;
-                        for (uint64_t q = sm.b; q < sm.e; ++q) {
-                            const uint32_t w = ldg(a.lcol, q);
-                            if (seg_has(a.lcol, lg, w)) {
-                                mark(D2, w);
-                                hit = true;
-                            }
-                        }
-                        if (hit) mark(D1, v1);
-                    }
-                    if (__ballot(hit)) any = true;
-                }
-            }
-            if (any && lane == 0) mark(D0, v);
-        } else if (T == 4) {  // four-chain v2 - v0 - v1 - v3, from the v0 side: v = v0
-            const Seg A2 = seg_of(a.rowptr, a.loff, a.L1, v, l2), S1 = seg_of(a.rowptr, a.loff, a.L1, v, l1);
-            const uint64_t s2 = (A2.e - A2.b) - uint64_t(l1 == l2);
-            bool any = false;
-            uint32_t i1 = kNone, i2 = kNone;
-            if (s2 >= 1) {
-                for (uint64_t k0 = S1.b; k0 < S1.e; k0 += 64) {
-                    const uint64_t k = k0 + lane;
-                    bool ok = false;
-                    uint32_t v1 = kNone, x2 = kNone;
-                    if (k < S1.e) {
-                        v1 = ldg(a.lcol, k);
-                        const Seg B3 = seg_of(a.rowptr, a.loff, a.L1, v1, l3);
-                        const uint64_t s3 = (B3.e - B3.b) - uint64_t(l0 == l3);
-                        if (s3 >= 1) {
-                            const uint32_t e3 = s3 == 1 ? only_other(a.lcol, B3, v) : kNone;
-                            const uint32_t e2 = s2 == 1 ? only_other(a.lcol, A2, v1) : kNone;
-                            ok = !(s2 == 1 && s3 == 1 && e2 == e3);
-                            x2 = e3;
-                        }
-                        if (ok) mark(D1, v1);
-                    }
-                    fold_exclusions(ok, v1, x2, any, i1, i2);
-                }
-            }
-            if (any) {
-                if (lane == 0) mark(D0, v);
-                mark_seg(D2, a.lcol, A2, i1, i2);
-            }
-        } else if (T == 5) {  // four-chain, from the v1 side: v = v1, lanes take v0
-            const Seg B3 = seg_of(a.rowptr, a.loff, a.L1, v, l3), S0 = seg_of(a.rowptr, a.loff, a.L1, v, l0);
-            const uint64_t s3 = (B3.e - B3.b) - uint64_t(l0 == l3);
-            bool any = false;
-            uint32_t j1 = kNone, j2 = kNone;
-            if (s3 >= 1) {
-                for (uint64_t k0 = S0.b; k0 < S0.e; k0 += 64) {
-                    const uint64_t k = k0 + lane;
-                    bool ok = false;
-                    uint32_t v0 = kNone, y2 = kNone;
-                    if (k < S0.e) {
-                        v0 = ldg(a.lcol, k);
-                        const Seg A2 = seg_of(a.rowptr, a.loff, a.L1, v0, l2);
-                        const uint64_t s2 = (A2.e - A2.b) - uint64_t(l1 == l2);
-                        if (s2 >= 1) {
-                            const uint32_t e2 = s2 == 1 ? only_other(a.lcol, A2, v) : kNone;
-                            const uint32_t e3 = s3 == 1 ? only_other(a.lcol, B3, v0) : kNone;
-                            ok = !(s2 == 1 && s3 == 1 && e2 == e3);
-                            y2 = e2;
-                        }
-                    }
-                    fold_exclusions(ok, v0, y2, any, j1, j2);
-                }
-            }
-            if (any) mark_seg(D3, a.lcol, B3, j1, j2);
-        } else {  // three-star: v = v1 (center), leaves of labels l0, l2, l3
-            const Seg S0 = seg_of(a.rowptr, a.loff, a.L1, v, l0), S2 = seg_of(a.rowptr, a.loff, a.L1, v, l2),
-                      S3 = seg_of(a.rowptr, a.loff, a.L1, v, l3);
-            const uint64_t r0 = 1 + uint64_t(l2 == l0) + uint64_t(l3 == l0);
-            const uint64_t r2 = 1 + uint64_t(l0 == l2) + uint64_t(l3 == l2);
-            const uint64_t r3 = 1 + uint64_t(l0 == l3) + uint64_t(l2 == l3);
-            if (S0.e - S0.b >= r0 && S2.e - S2.b >= r2 && S3.e - S3.b >= r3) {
-                if (lane == 0) mark(D1, v);
-                mark_seg(D0, a.lcol, S0, kNone, kNone);
-                mark_seg(D2, a.lcol, S2, kNone, kNone);
-                mark_seg(D3, a.lcol, S3, kNone, kNone);
-            }
-        }
-    }
+    uint32_t* D0 = a.bm + size_t(blockIdx.y) * 4 * a.W;
+    const uint32_t* lp = a.labels + 4 * blockIdx.y;
+    const Labels4 l{lp[0], lp[1], lp[2], lp[3]};
+    // roots: the vertices of the first label; the three-star and the
+    // four-chain's second pass start from their center / v1
+    const uint32_t* g = a.groups + 2 * (T >= 5 ? l.l1 : l.l0);
+    const uint32_t r0 = g[0], rh = g[1], r1 = g[2];
+    for (uint32_t r = r0 + wid; r < rh; r += nw) fsm_root<T, true>(a, l, D0, ldg(a.vlist, r));
+    for (uint32_t r = rh + 64 * wid; r < r1; r += 64 * nw)
+        if (r + lane < r1) fsm_root<T, false>(a, l, D0, ldg(a.vlist, r + lane));
 }
 
 // sizes[c * 4 + i] += popcount of bitmap i of candidate c (blockIdx.y = c * 4 + i).
@@ -366,21 +422,38 @@ int fsm_set_labels(DeviceGraph& d, const uint32_t* h_lab) {
     }
     F->voff.assign(F->L + 1, 0);
     for (uint32_t l = 0; l < F->L; ++l) F->voff[l + 1] = F->voff[l] + cnt[l];
-    std::vector<uint32_t> vl(std::max<uint32_t>(1, d.n));
+    // vertices by label, within a label by degree, largest first (a counting
+    // sort by degree, then a stable one by label)
+    std::vector<uint32_t> vl(std::max<uint32_t>(1, d.n)), groups(2 * size_t(F->L) + 1, d.n);
     {
-        std::vector<uint32_t> at(F->voff.begin(), F->voff.end() - 1);
-        for (uint32_t v = 0; v < d.n; ++v) vl[at[h_lab[v]]++] = v;
+        uint32_t maxd = 0;
+        for (uint32_t x : d.h_deg) maxd = std::max(maxd, x);
+        std::vector<uint32_t> start(size_t(maxd) + 2, 0), order(d.n);
+        for (uint32_t x : d.h_deg) ++start[maxd - x + 1];
+        for (size_t i = 1; i < start.size(); ++i) start[i] += start[i - 1];
+        for (uint32_t v = 0; v < d.n; ++v) order[start[maxd - d.h_deg[v]]++] = v;
+        std::vector<uint32_t> at(F->voff.begin(), F->voff.end() - 1), heavy(F->L, 0);
+        for (uint32_t v : order) {
+            vl[at[h_lab[v]]++] = v;
+            heavy[h_lab[v]] += d.h_deg[v] > kLaneDegree;
+        }
+        for (uint32_t l = 0; l < F->L; ++l) {
+            groups[2 * l] = F->voff[l];
+            groups[2 * l + 1] = F->voff[l] + heavy[l];
+        }
     }
     const size_t n1 = std::max<uint32_t>(1, d.n);
     const size_t m1 = std::max<uint64_t>(1, d.nnz);
     const size_t offs = size_t(F->L + 1) * n1;
     if (hipMalloc(&F->lab, 4 * n1) != hipSuccess || hipMalloc(&F->vlist, 4 * n1) != hipSuccess ||
-        hipMalloc(&F->lcol, 4 * m1) != hipSuccess || hipMalloc(&F->loff, 4 * offs) != hipSuccess) {
+        hipMalloc(&F->lcol, 4 * m1) != hipSuccess || hipMalloc(&F->loff, 4 * offs) != hipSuccess ||
+        hipMalloc(&F->groups, 4 * groups.size()) != hipSuccess) {
         (void)hipGetLastError();
         KZ_FAIL(KZ_ERR_NOMEM, "labelled lists of %llu entries", (unsigned long long)d.nnz);
     }
-    F->bytes = 8 * n1 + 4 * m1 + 4 * offs;
+    F->bytes = 8 * n1 + 4 * m1 + 4 * offs + 4 * groups.size();
     hipStream_t s = rt().stream;
+    KZ_HIP(hipMemcpyAsync(F->groups, groups.data(), 4 * groups.size(), hipMemcpyHostToDevice, s));
     if (d.n) {
         KZ_HIP(hipMemcpyAsync(F->lab, h_lab, 4 * size_t(d.n), hipMemcpyHostToDevice, s));
         KZ_HIP(hipMemcpyAsync(F->vlist, vl.data(), 4 * size_t(d.n), hipMemcpyHostToDevice, s));
@@ -394,42 +467,26 @@ int fsm_set_labels(DeviceGraph& d, const uint32_t* h_lab) {
     return KZ_OK;
 }
 
-// The domain kernels of one candidate of a level (1 edge .. 5 three-star)
-// with labels l[], into its 4 bitmaps bm[4 * W].
-static void launch_domains(const DeviceGraph& d, const FsmState& F, int level, const uint32_t* l, uint32_t* bm,
-                           uint32_t W, uint32_t grid, hipStream_t s) {
-    FsmArgs a{d.rowptr, F.lcol, F.loff, F.L + 1, nullptr, 0, {0, 0, 0, 0}, bm, W};
-    const int size = level == 1 ? 2 : (level <= 3 ? 3 : 4);
-    for (int i = 0; i < size; ++i) a.l[i] = l[i];
-    // roots: the vertices of the first label; the three-star and the
-    // four-chain's second pass start from their center / v1
-    auto roots = [&](uint32_t lab) {
-        a.roots = F.vlist + F.voff[lab];
-        a.nroots = F.voff[lab + 1] - F.voff[lab];
-    };
+// The domain kernels of nc candidates of a level (1 edge .. 5 three-star)
+// with labels[4 * nc] on the device, into their bitmaps bm[4 * W * nc].
+static void launch_domains(const DeviceGraph& d, const FsmState& F, int level, const uint32_t* labels, uint32_t nc,
+                           uint32_t* bm, uint32_t W, hipStream_t s) {
+    const FsmArgs a{d.rowptr, F.lcol, F.loff, F.L + 1, F.vlist, F.groups, labels, bm, W};
+    // workgroups per candidate: enough for a level of few candidates to fill
+    // the chip, no more than the largest label has roots for
+    uint32_t most = 1;
+    for (uint32_t l = 0; l < F.L; ++l) most = std::max(most, F.voff[l + 1] - F.voff[l]);
+    const uint32_t fill = uint32_t(rt().num_cus) * 8;
+    const dim3 grid(std::min<uint32_t>((most + 3) / 4, std::max<uint32_t>(fill / nc, 64)), nc);
     switch (level) {
-        case 1:
-            roots(l[0]);
-            if (a.nroots) hipLaunchKernelGGL(fsm_domain_kernel<1>, dim3(grid), dim3(256), 0, s, a);
-            break;
-        case 2:
-            roots(l[0]);
-            if (a.nroots) hipLaunchKernelGGL(fsm_domain_kernel<2>, dim3(grid), dim3(256), 0, s, a);
-            break;
-        case 3:
-            roots(l[0]);
-            if (a.nroots) hipLaunchKernelGGL(fsm_domain_kernel<3>, dim3(grid), dim3(256), 0, s, a);
-            break;
+        case 1: hipLaunchKernelGGL(fsm_domain_kernel<1>, grid, dim3(256), 0, s, a); break;
+        case 2: hipLaunchKernelGGL(fsm_domain_kernel<2>, grid, dim3(256), 0, s, a); break;
+        case 3: hipLaunchKernelGGL(fsm_domain_kernel<3>, grid, dim3(256), 0, s, a); break;
         case 4:
-            roots(l[0]);
-            if (a.nroots) hipLaunchKernelGGL(fsm_domain_kernel<4>, dim3(grid), dim3(256), 0, s, a);
-            roots(l[1]);
-            if (a.nroots) hipLaunchKernelGGL(fsm_domain_kernel<5>, dim3(grid), dim3(256), 0, s, a);
+            hipLaunchKernelGGL(fsm_domain_kernel<4>, grid, dim3(256), 0, s, a);
+            hipLaunchKernelGGL(fsm_domain_kernel<5>, grid, dim3(256), 0, s, a);
             break;
-        default:
-            roots(l[1]);
-            if (a.nroots) hipLaunchKernelGGL(fsm_domain_kernel<6>, dim3(grid), dim3(256), 0, s, a);
-            break;
+        default: hipLaunchKernelGGL(fsm_domain_kernel<6>, grid, dim3(256), 0, s, a); break;
     }
 }
 
@@ -447,8 +504,8 @@ int fsm_domains(DeviceGraph& d, int level, const uint32_t* labels, uint32_t* siz
         }
     hipStream_t s = rt().stream;
     const uint32_t W = std::max<uint32_t>(1, (F.n + 31) / 32);
-    uint32_t *bm = nullptr, *sz = nullptr;
-    if (hipMalloc(&bm, 16 * size_t(W)) != hipSuccess || hipMalloc(&sz, 16) != hipSuccess) {
+    uint32_t *bm = nullptr, *sz = nullptr;  // sz: 4 sizes, then the 4 labels
+    if (hipMalloc(&bm, 16 * size_t(W)) != hipSuccess || hipMalloc(&sz, 32) != hipSuccess) {
         (void)hipGetLastError();
         hipFree(bm);
         KZ_FAIL(KZ_ERR_NOMEM, "domain bitmaps of %u vertices", F.n);
@@ -461,8 +518,10 @@ int fsm_domains(DeviceGraph& d, int level, const uint32_t* labels, uint32_t* siz
         }
     } free_on_return{bm, sz};
     KZ_HIP(hipMemsetAsync(bm, 0, 16 * size_t(W), s));
-    KZ_HIP(hipMemsetAsync(sz, 0, 16, s));
-    launch_domains(d, F, level, labels, bm, W, uint32_t(rt().num_cus) * 8, s);
+    uint32_t l[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int i = 0; i < size; ++i) l[4 + i] = labels[i];
+    KZ_HIP(hipMemcpyAsync(sz, l, 32, hipMemcpyHostToDevice, s));
+    launch_domains(d, F, level, sz + 4, 1, bm, W, s);
     const uint32_t pgrid = std::min<uint32_t>((W + 255) / 256, 64);
     hipLaunchKernelGGL(fsm_popcount_kernel, dim3(pgrid, 4), dim3(256), 0, s, bm, W, sz);
     KZ_HIP(hipGetLastError());
@@ -518,24 +577,24 @@ int fsm_mine(DeviceGraph& d, uint32_t threshold, kz_fsm_stats* st, kz_fsm_candid
     // candidates per batch: 4 bitmaps each, at most a quarter of free memory
     const size_t per_cand = 16 * size_t(W);
     const uint32_t batch = uint32_t(std::max<size_t>(1, std::min<size_t>(4096, (free_b / 4) / per_cand)));
-    const uint32_t grid = uint32_t(rt().num_cus) * 8;
+    std::vector<uint32_t> labels;
     auto evaluate = [&](int level, const std::vector<Cand>& cs, std::set<Pat>* table) -> int {
         st->num_candidates[level] = uint32_t(cs.size());
         for (size_t c0 = 0; c0 < cs.size(); c0 += batch) {
             const uint32_t nb = uint32_t(std::min<size_t>(batch, cs.size() - c0));
             if (int e = scratch_reserve(bits, per_cand * nb)) return e;
-            if (int e = scratch_reserve(sizes, 16 * size_t(nb))) return e;
+            if (int e = scratch_reserve(sizes, 32 * size_t(nb))) return e;
             uint32_t* bm = static_cast<uint32_t*>(bits.ptr);
-            uint32_t* sz = static_cast<uint32_t*>(sizes.ptr);
-            KZ_HIP(hipEventRecord(e0, s));
-            KZ_HIP(hipMemsetAsync(bm, 0, per_cand * nb, s));
-            KZ_HIP(hipMemsetAsync(sz, 0, 16 * size_t(nb), s));
+            uint32_t* sz = static_cast<uint32_t*>(sizes.ptr);  // 4 nb sizes, then 4 nb labels
+            labels.assign(8 * size_t(nb), 0);
             for (uint32_t c = 0; c < nb; ++c) {
                 const Pat& p = cs[c0 + c].canon;
-                uint32_t l[4] = {0, 0, 0, 0};
-                for (int i = 0; i < p.size; ++i) l[i] = p.l[i];
-                launch_domains(d, F, level, l, bm + size_t(c) * 4 * W, W, grid, s);
+                for (int i = 0; i < p.size; ++i) labels[4 * size_t(nb) + 4 * c + i] = p.l[i];
             }
+            KZ_HIP(hipEventRecord(e0, s));
+            KZ_HIP(hipMemsetAsync(bm, 0, per_cand * nb, s));
+            KZ_HIP(hipMemcpyAsync(sz, labels.data(), 32 * size_t(nb), hipMemcpyHostToDevice, s));
+            launch_domains(d, F, level, sz + 4 * size_t(nb), nb, bm, W, s);
             const uint32_t pgrid = std::min<uint32_t>((W + 255) / 256, 64);
             hipLaunchKernelGGL(fsm_popcount_kernel, dim3(pgrid, 4 * nb), dim3(256), 0, s, bm, W, sz);
             KZ_HIP(hipGetLastError());

@@ -91,3 +91,20 @@ def test_fsm_errors(kzdev):
         o.set_labels(np.zeros(g.num_vertices, np.uint32))  # symmetric graphs only
     dg.release()
     o.release()
+
+
+@pytest.mark.parametrize("hub", [63, 64, 65, 200])
+def test_fsm_roots_of_one_lane_and_of_one_wave(kzdev, hub):
+    """Roots on both sides of the degree that moves them from a lane to a
+    wave, with more roots of a label than one wave takes at a time."""
+    kz = kzdev
+    rng = np.random.default_rng(hub)
+    n = 260
+    src = np.concatenate([rng.integers(0, n, 500), np.zeros(hub, np.int64), np.full(hub, 1)])
+    dst = np.concatenate([rng.integers(0, n, 500), 2 + rng.permutation(n - 2)[:hub], 2 + rng.permutation(n - 2)[:hub]])
+    g = kz.from_edges(src, dst, n)
+    lab = rng.integers(0, 2, g.num_vertices).astype(np.uint32)
+    dg = g.to_device()
+    dg.set_labels(lab)
+    _check(dg, g.rowptr, g.col, lab, 20, f"hub{hub}")
+    dg.release()
