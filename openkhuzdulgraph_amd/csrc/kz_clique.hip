@@ -281,93 +281,33 @@ __host__ __device__ inline uint32_t tri_words(uint32_t d) {
 
 // 5-cliques through DAG rows i < j (bit j of row i set), word kj = (j+1)/64
 // on: with C = row_i & row_j (ids > j), the adjacent pairs l < m of C, i.e.
-// the sum over l in C of |C & row_l|.  C's wd <= WMAX words stay in
-// registers, so each l costs one row load per word instead of three.  TRI:
-// packed rows (word_base), whose word offsets are then constants.
-template <uint32_t WMAX, bool TRI = false>
+// the sum over l in C of |C & row_l|.  C's wd <= 2 words stay in registers, so
+// each l costs one row load per word.  TRI: packed rows (word_base).
+template <bool TRI = false>
 __device__ __forceinline__ uint32_t count5_pairs(const unsigned long long* rows, uint32_t ws, uint32_t wd,
                                                  const unsigned long long* ri, const unsigned long long* rj,
                                                  uint32_t kj) {
-    unsigned long long c[WMAX];
+    unsigned long long c[2];
 #pragma unroll
-    for (uint32_t k = 0; k < WMAX; ++k)
+    for (uint32_t k = 0; k < 2; ++k)
         c[k] = (k >= kj && k < wd) ? ri[word_base<TRI>(k, ws)] & rj[word_base<TRI>(k, ws)] : 0ull;
-    uint32_t n = 0;  // at most |C|^2 / 2 < 2^19 for wd <= 16
+    uint32_t n = 0;
 #pragma unroll
-    for (uint32_t kk = 0; kk < WMAX; ++kk) {
+    for (uint32_t kk = 0; kk < 2; ++kk) {
         unsigned long long m = c[kk];
         while (m) {
             const unsigned long long* rl = rows + (kk * 64 + uint32_t(__builtin_ctzll(m)));
             m &= m - 1;
             // row l holds ids > l only: its words below kk are empty
 #pragma unroll
-            for (uint32_t k3 = kk; k3 < WMAX; ++k3)
+            for (uint32_t k3 = kk; k3 < 2; ++k3)
                 if (k3 < wd) n += uint32_t(__popcll(c[k3] & rl[word_base<TRI>(k3, ws)]));
         }
     }
     return n;
 }
 
-// Counts the k-cliques of one root's DAG rows i = first, first + stride, ...
-// (wave-cooperative: lanes take the set bits j of row i).  The bitmap is
-// word-major: word kk of row i is rows[kk * ws + i], so the lanes' rows j
-// sit in consecutive words (no LDS bank conflicts) and row i is a broadcast.
-// With ctr (an LDS counter zeroed before a barrier) rows are taken one
-// at a time from it instead (first and stride unused): rows come largest
-// first, so the waves finish together.  kRegC: 5-clique rows of at most
-// 16 words keep row_i & row_j in registers (count5_pairs).
-template <int K, bool kRegC = true, bool TRI = false>
-__device__ __forceinline__ void count_rows(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t first,
-                                           uint32_t stride, unsigned long long& acc, uint32_t* ctr = nullptr) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wd = (d + 63) >> 6;
-    auto next = [&](uint32_t i) -> uint32_t {
-        if (!ctr) return i + stride;
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(ctr, 1u);
-        return wave_bcast(t);
-    };
-    for (uint32_t i = ctr ? next(0) : first; i + 2 < d; i = next(i)) {
-        const unsigned long long* ri = rows + i;
-        const uint32_t k_lo = (i + 1) >> 6;
-        uint32_t total = 0;
-        for (uint32_t k = k_lo; k < wd; ++k) total += __popcll(ri[word_base<TRI>(k, ws)]);
-        total = wave_bcast(total);  // row i is the same in every lane
-        for (uint32_t base = 0; base < total; base += 64) {
-            const uint32_t r = base + lane;
-            if (r >= total) break;
-            uint32_t k = k_lo, rem = r;
-            unsigned long long wv = ri[word_base<TRI>(k, ws)];
-            for (uint32_t c = __popcll(wv); rem >= c; c = __popcll(wv)) {
-                rem -= c;
-                wv = ri[word_base<TRI>(++k, ws)];
-            }
-            const uint32_t j = k * 64 + select_bit(wv, rem);
-            const unsigned long long* rj = rows + j;
-            const uint32_t kj = (j + 1) >> 6;
-            if (K == 4) {
-                for (uint32_t kk = kj; kk < wd; ++kk) acc += __popcll(ri[word_base<TRI>(kk, ws)] & rj[word_base<TRI>(kk, ws)]);
-            } else if (kRegC && wd <= 16) {  // d <= 1024: C in registers
-                if (wd <= 2) acc += count5_pairs<2, TRI>(rows, ws, wd, ri, rj, kj);
-                else if (wd <= 8) acc += count5_pairs<8, TRI>(rows, ws, wd, ri, rj, kj);
-                else acc += count5_pairs<16, TRI>(rows, ws, wd, ri, rj, kj);
-            } else {
-                for (uint32_t kk = kj; kk < wd; ++kk) {
-                    unsigned long long m = ri[word_base<TRI>(kk, ws)] & rj[word_base<TRI>(kk, ws)];
-                    while (m) {
-                        const uint32_t l = kk * 64 + __builtin_ctzll(m);
-                        m &= m - 1;
-                        const unsigned long long* rl = rows + l;
-                        for (uint32_t k3 = (l + 1) >> 6; k3 < wd; ++k3)
-                            acc += __popcll(ri[word_base<TRI>(k3, ws)] & rj[word_base<TRI>(k3, ws)] & rl[word_base<TRI>(k3, ws)]);
-                    }
-                }
-            }
-        }
-    }
-}
-
-// 5-cliques of one root's DAG rows in LDS (d <= 1024 rows, word-major with
+// 5-cliques of one root's DAG rows in LDS (d <= 128 rows, word-major with
 // stride d, or packed: TRI), the workgroup's lanes taking its edges (i, j)
 // 64 at a time from ctr (an LDS counter zeroed before a barrier) in row
 // order, so that rows with fewer than 64 set bits leave no lane idle.  pre:
@@ -404,9 +344,7 @@ __device__ __forceinline__ void count5_edges(const unsigned long long* rows, uin
             }
             const uint32_t j = k * 64 + select_bit(wv, rem);
             const uint32_t kj = (j + 1) >> 6;
-            if (wd <= 2) acc += count5_pairs<2, TRI>(rows, d, wd, ri, rows + j, kj);
-            else if (wd <= 8) acc += count5_pairs<8, TRI>(rows, d, wd, ri, rows + j, kj);
-            else acc += count5_pairs<16, TRI>(rows, d, wd, ri, rows + j, kj);
+            acc += count5_pairs<TRI>(rows, d, wd, ri, rows + j, kj);
         }
         base = wave_bcast(nb);
     }
@@ -591,6 +529,101 @@ __device__ __forceinline__ void count_rows_mfma4(const unsigned long long* rows,
         tile_coords(tile, &I, &J);
         acc += mfma4_tiles<TRI, N>(rows, ws, d, N * wave_bcast(I), N * wave_bcast(J));
         tile = wave_bcast(tn);
+    }
+}
+
+// 5-cliques of a root through its DAG row i: the triangles among row i's r set
+// bits, i.e. with c_0 < c_1 < ... the set bits and A the root's DAG, the sum
+// over s < t of A[c_s][c_t] * |row_i & row_{c_s} & row_{c_t}|.  The r x r
+// product is taken on FP4 MFMA as the 4-clique count's (mfma4_tiles), in 32 x
+// 32 tiles (I, J >= I) of rows and columns gathered through the list c, one
+// operand masked by row i; the mask A[c_s][c_t] comes from the same operand
+// times one-hot columns, in the one or two words that hold the tile's
+// columns.  Against the popcount loops (one lane per edge, a select of its
+// bit and a row read per common neighbour) the work no longer grows with the
+// number of edges but with r^2 / 1024 tiles.
+// c: LDS list of at least d u16 for this wave; rows a word-major bitmap (word
+// kk of row i at rows[word_base<TRI>(kk, ws) + i], read for kk >= i / 64
+// only).  Call with every lane of the wave.
+template <bool TRI>
+__device__ __forceinline__ void count5_row(const unsigned long long* rows, uint32_t ws, uint32_t d, uint32_t i,
+                                           uint16_t* c, unsigned long long& acc) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wd = (d + 63) >> 6;
+    uint32_t r = 0;
+    wave_lds_sync();  // the list's last readers are done
+    for (uint32_t kw = (i + 1) >> 6; kw < wd; ++kw) {
+        const unsigned long long w = rows[word_base<TRI>(kw, ws) + i];
+        const uint32_t lo = wave_bcast(uint32_t(w)), hi = wave_bcast(uint32_t(w >> 32));
+        if ((w >> lane) & 1u) c[r + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u))] = uint16_t(64 * kw + lane);
+        r += uint32_t(__popc(lo) + __popc(hi));
+    }
+    if (r < 3) return;
+    wave_lds_sync();
+    const uint32_t hs = lane >> 5;
+    const uint32_t* half = reinterpret_cast<const uint32_t*>(rows) + hs;
+    const uint32_t wend = (wave_bcast(uint32_t(c[r - 1])) >> 6) + 1;
+    for (uint32_t J = 0; 32 * J < r; ++J) {
+        const uint32_t jj = 32 * J + (lane & 31);
+        const uint32_t cj = c[jj < r ? jj : r - 1];
+        const uint32_t k0 = wave_lane(cj, 0u) >> 6, k1 = wave_lane(cj, 31u) >> 6;
+        const uint32_t one = 1u << (cj & 31u), at = cj >> 5;  // the column's one-hot half word
+        for (uint32_t I = 0; I <= J; ++I) {
+            const uint32_t ii = 32 * I + (lane & 31);
+            const uint32_t ci = c[ii < r ? ii : r - 1];
+            kz_v16f p{}, m{};
+            for (uint32_t kw = k0; kw <= k1; ++kw) {
+                // rows past word kw have no such word
+                const uint32_t base = 2 * word_base<TRI>(kw, ws);
+                uint32_t a = half[base + 2 * ci] & half[base + 2 * i], b = half[base + 2 * cj];
+                a = (ci >> 6) <= kw ? a : 0u;
+                b = (cj >> 6) <= kw ? b : 0u;
+                const kz_v8i A = fp4_rows(a);
+                p = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, fp4_cols(b), p, 4, 4, 0, 0, 0, 0);
+                m = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, fp4_cols(at == 2 * kw + hs ? one : 0u), m, 4, 4, 0,
+                                                                   0, 0, 0);
+            }
+            uint32_t a = 0, b = 0;
+            auto load = [&](uint32_t kw) {
+                const uint32_t base = 2 * word_base<TRI>(kw, ws);
+                a = half[base + 2 * ci] & half[base + 2 * i];
+                b = half[base + 2 * cj];
+            };
+            uint32_t kw = k1 + 1;
+            if (kw < wend) load(kw);
+            while (kw < wend) {
+                const kz_v8i A = fp4_rows(a), B = fp4_cols(b);
+                if (++kw < wend) load(kw);
+                p = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, p, 4, 4, 0, 0, 0, 0);
+            }
+            // exact: at most 16 r <= 2^17 per tile and lane
+            float t = 0.f;
+#pragma unroll
+            for (int k = 0; k < 16; ++k) t = __builtin_fmaf(p[k], m[k], t);
+            acc += uint32_t(t);
+        }
+    }
+}
+
+// The rows of one root in LDS, one per wave at a time from ctr (an LDS counter
+// zeroed before a barrier; the longest rows come first).  [lists, end): free
+// LDS, what the build used: d u16 per wave, and where it holds fewer lists
+// than the workgroup has waves (1024 candidates without probe queues: 15 of
+// 16) the last waves leave the rows to the others.
+template <bool TRI>
+__device__ __forceinline__ void count5_rows(const unsigned long long* rows, uint32_t d, uint16_t* lists, uint16_t* end,
+                                            uint32_t* ctr, unsigned long long& acc) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint16_t* c = lists + wave_bcast(threadIdx.x >> 6) * d;
+    if (c + d > end) return;
+    uint32_t i = 0;
+    if (lane == 0) i = atomicAdd(ctr, 1u);
+    i = wave_bcast(i);
+    while (i + 3 < d) {
+        uint32_t in = 0;
+        if (lane == 0) in = atomicAdd(ctr, 1u);
+        count5_row<TRI>(rows, d, d, i, c, acc);
+        i = wave_bcast(in);
     }
 }
 
@@ -800,8 +833,10 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(WPE))) voi
         __syncthreads();
                 if (K == 4) count_rows_mfma4<TRI, (WPE <= 4 ? 2 : 1)>(rows, d, d, &sTile, acc);
         else if (K == 5) {
-            if (W <= 8) count5_edges<TRI>(rows, d, rp, sTmp, &sTile, acc);
-            else count_rows<K, true, TRI>(rows, d, d, 0, 0, acc, &sTile);
+            // (RMAT-22: up to 128 candidates the edge loop is the faster, 9.4
+            // against 10.0 ms for the two buckets; above, MFMA tiles)
+            if (W <= 2) count5_edges<TRI>(rows, d, rp, sTmp, &sTile, acc);
+            else count5_rows<TRI>(rows, d, reinterpret_cast<uint16_t*>(rb), hv + H, &sTile, acc);
         }
         __syncthreads();
     }
@@ -1007,27 +1042,35 @@ __global__ __launch_bounds__(256) void core_sample_kernel(const CoreGraph* __res
     if ((threadIdx.x & 63) == 0 && s) atomicAdd(&sums[blockIdx.x], s);
 }
 
-// One wave per hub row: counts the cliques whose second vertex is that row.
-template <int K>
-__global__ __launch_bounds__(256) void hub_count_kernel(const HubMeta* __restrict__ hubs, uint32_t nhubs,
-                                                        const uint32_t* __restrict__ row_prefix, uint32_t nrows,
-                                                        uint32_t* __restrict__ cursor,
-                                                        unsigned long long* __restrict__ results,
-                                                        const unsigned long long* __restrict__ slab) {
+// 5-cliques of the hubs, one wave per hub row (count5_row), the rows of every
+// hub (row_prefix: exclusive prefix over hubs) taken from one cursor.  Dynamic
+// LDS: dmax u16 per wave.
+__global__ __launch_bounds__(256) void hub_count5_kernel(const HubMeta* __restrict__ hubs, uint32_t nhubs,
+                                                         const uint32_t* __restrict__ row_prefix, uint32_t nrows,
+                                                         uint32_t* __restrict__ cursor,
+                                                         unsigned long long* __restrict__ results,
+                                                         const unsigned long long* __restrict__ slab, uint32_t dmax) {
+    extern __shared__ uint16_t slist[];
+    uint16_t* c = slist + (threadIdx.x >> 6) * dmax;
     unsigned long long acc = 0;
     uint32_t qcur = 0xFFFFFFFFu;
     TaskChunk chunk(nrows, gridDim.x * (blockDim.x >> 6), 8);
+    HubMeta hm{};
+    uint32_t h0 = 0, h1 = 0;  // rows of hub hm
     while (true) {
         const uint32_t r = wave_next_task(chunk, cursor);
         if (r >= nrows) break;
-        const uint32_t h = row_of(row_prefix, nhubs, r);
-        const HubMeta hm = hubs[h];
+        if (r < h0 || r >= h1) {
+            const uint32_t h = wave_bcast(row_of(row_prefix, nhubs, r));
+            hm = hubs[h];
+            h0 = wave_bcast(row_prefix[h]);
+            h1 = h + 1 < nhubs ? wave_bcast(row_prefix[h + 1]) : nrows;
+        }
         if (hm.q != qcur) {
             if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
             qcur = hm.q;
         }
-        const uint32_t i = r - row_prefix[h];
-        count_rows<K, false>(slab + hm.slab_off, hm.d, hm.d, i, hm.d, acc);
+        count5_row<false>(slab + hm.slab_off, hm.d, hm.d, r - h0, c, acc);
     }
     if (qcur != 0xFFFFFFFFu) flush_query(acc, qcur, results);
 }
@@ -1131,12 +1174,11 @@ static uint32_t filter_words(uint32_t Dmax, uint32_t per_key = 16) {
     return w;
 }
 
-// queue_threads: the workgroup size when it keeps probe queues, else 0;
 // tri: packed rows (k >= 4).
-static size_t block_lds_bytes(int K, uint32_t Dmax, uint32_t W, uint32_t H, uint32_t queue_threads = 0,
+static size_t block_lds_bytes(int K, uint32_t Dmax, uint32_t W, uint32_t H, uint32_t threads, bool queues = false,
                               bool tri = false) {
     const size_t rows = K < 4 ? 0 : tri ? size_t(tri_words(Dmax)) : size_t(Dmax) * W;
-    return rows * 8 + size_t(Dmax) * 8 + size_t(queue_threads) * 8 + size_t(Dmax) * 4 +
+    return rows * 8 + size_t(Dmax) * 8 + (queues ? size_t(threads) * 8 : 0) + size_t(Dmax) * 4 +
            size_t(Dmax + 1) * 4 + size_t(filter_words(Dmax)) * 4 + size_t(H) * 6 + 16;
 }
 
@@ -1151,9 +1193,9 @@ static uint32_t two_per_cu_degree(uint32_t lo, uint32_t hi) {
         uint32_t H, hshift;
         hash_size(d, &H, &hshift);
         const uint32_t W = (d + 63) / 64;
-        const size_t ldst = block_lds_bytes(4, d, W, H, 512, true);
+        const size_t ldst = block_lds_bytes(4, d, W, H, 512, true, true);
         if (ldst + kStaticLdsReserve <= per_block && per_cu(ldst) >= 2)
-            return per_cu(block_lds_bytes(4, d, W, H)) == 1 ? d : 0;
+            return per_cu(block_lds_bytes(4, d, W, H, 512)) == 1 ? d : 0;
     }
     return 0;
 }
@@ -1221,6 +1263,7 @@ static int set_lds_attrs() {
                          reinterpret_cast<const void*>(&hub_rows_kernel<5>),
                          reinterpret_cast<const void*>(&hub_rows_kernel<4, true>),
                          reinterpret_cast<const void*>(&hub_rows_kernel<5, true>),
+                         reinterpret_cast<const void*>(&hub_count5_kernel),
                          reinterpret_cast<const void*>(&core_build_kernel)};
     for (const void* f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, maxb) != hipSuccess)
@@ -1302,7 +1345,7 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
         uint32_t H, hshift;
         hash_size(Dmax, &H, &hshift);
         const uint32_t block = gr.block ? gr.block : x.cfg.block[gr.bucket];
-        const size_t lds = block_lds_bytes(K, Dmax, W, H);
+        const size_t lds = block_lds_bytes(K, Dmax, W, H, block);
         if (lds > lds_limit)
             KZ_FAIL(KZ_ERR_UNSUPPORTED, "bucket %d needs %zu bytes of LDS (limit %zu)", gr.bucket, lds, lds_limit);
         auto groups_per_cu = [&](size_t b) {
@@ -1320,8 +1363,8 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
         // whose count dominates, take packed rows wherever they keep the
         // occupancy (constant word offsets; RMAT-22 128-512 bucket 40.28 ->
         // 39.13 ms).
-        const size_t ldsq = block_lds_bytes(K, Dmax, W, H, block);
-        const size_t ldst = block_lds_bytes(K, Dmax, W, H, block, true);
+        const size_t ldsq = block_lds_bytes(K, Dmax, W, H, block, true);
+        const size_t ldst = block_lds_bytes(K, Dmax, W, H, block, true, true);
         const bool qu = stream_queue_enabled() && ldsq <= lds_limit && groups_per_cu(ldsq) == per_cu;
         const bool tri_fit = K >= 4 && stream_queue_enabled() && ldst <= lds_limit;
         const bool tri2 = tri_fit && block == 512 && per_cu == 1 && groups_per_cu(ldst) >= 2;
@@ -1390,8 +1433,8 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
                            cur + kCursorStride, x.d_result, x.slabs[K]);
     } else if (K >= 5) {
         const uint32_t cgrid = std::min<uint32_t>((hp.nrows + 3) / 4, uint32_t(R.num_cus) * 8);
-        hipLaunchKernelGGL(hub_count_kernel<K>, dim3(cgrid), dim3(256), 0, s, meta, hp.nhubs, x.hub_rows[K], hp.nrows,
-                           cur + kCursorStride, x.d_result, x.slabs[K]);
+        hipLaunchKernelGGL(hub_count5_kernel, dim3(cgrid), dim3(256), 4 * 2 * size_t(hp.dmax), s, meta, hp.nhubs,
+                           x.hub_rows[K], hp.nrows, cur + kCursorStride, x.d_result, x.slabs[K], hp.dmax);
     }
     return KZ_OK;
 }

@@ -278,3 +278,23 @@ def _forward_graph(kz, src, dst):
         f.write(pairs.tobytes())
         f.flush()
         return kz.load_dgraph(f.name)
+
+
+@pytest.mark.parametrize("d,p", [(130, 0.9), (192, 0.5), (257, 0.3), (513, 0.25), (700, 0.35), (1100, 0.1), (160, 1.1)])
+def test_five_cliques_on_mfma_tiles(kzdev, d, p):
+    """5-cliques below one root of d candidates: rows of 0 .. d - 1 set bits
+    (partial tiles, tiles whose columns straddle words, hub rows in HBM)."""
+    import numpy as np
+
+    kz = kzdev
+    rng = np.random.default_rng(d)
+    a, b = np.triu_indices(d, 1)
+    keep = rng.random(len(a)) < p * (1 - 0.9 * a / d)  # long rows first, short ones last
+    src = np.concatenate([np.zeros(d, np.int64), a[keep] + 1])
+    dst = np.concatenate([np.arange(1, d + 1), b[keep] + 1])
+    g = _forward_graph(kz, src, dst)
+    want = oracle.run_app(APP[5], g.rowptr, g.col)[1][0]
+    dg = g.to_device()
+    print(f"[case] five cliques d={d} p={p}", flush=True)
+    assert dg.count_cliques(5, "persistent") == want
+    dg.release()
