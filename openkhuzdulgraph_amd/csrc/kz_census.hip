@@ -74,6 +74,9 @@ struct Ranked {
     uint32_t c4_scratch_keys = 0;    // endpoints per heavy workgroup
     uint32_t c4_max_slots = 0;       // bucket hash slots used (a power of two <= kC4HeavySlots)
     uint32_t c4_direct_bound = 0;    // heavy roots up to this bound first try one unbucketed pass
+    uint32_t c4_dense = 0;           // ranges of the graph when every heavy root counts directly, else 0
+    uint32_t c4_nhist = 0, c4_ranges = 0;  // heavy roots bucketed by range (the first ones), ranges of the graph
+    uint32_t* c4_hist = nullptr;     // their endpoints per range
     uint32_t* c4_scratch = nullptr;  // c4_heavy_grid * c4_scratch_keys endpoints
     uint32_t* cursor = nullptr;      // kCursors task cursors, kCursorStride words apart
     unsigned long long* sums = nullptr;  // 8 accumulators
@@ -81,7 +84,7 @@ struct Ranked {
     CliqueJob k4;
     ~Ranked() {
         for (void* p : {(void*)rowptr, (void*)col, (void*)deg, (void*)frowptr, (void*)fcol, (void*)tasks, (void*)troot,
-                        (void*)tmid, (void*)c4_bound, (void*)c4_tasks, (void*)c4_scratch, (void*)cursor, (void*)sums})
+                        (void*)tmid, (void*)c4_bound, (void*)c4_tasks, (void*)c4_scratch, (void*)c4_hist, (void*)cursor, (void*)sums})
             if (p) (void)hipFree(p);
     }
 };
@@ -255,10 +258,21 @@ constexpr uint32_t kC4MaxBuckets = 4096;
 constexpr uint32_t kC4BucketKeys = 4096;   // mean endpoints per bucket aimed at
 constexpr uint32_t kC4ScratchKeys = 12u << 20;  // per heavy workgroup: 48 MB of endpoints
 constexpr uint32_t kC4BucketMul = 0x85EBCA6Bu;  // bucket hash (the tables use 2654435761)
-constexpr int kC4Unroll = 4;                    // wedge stream loads in flight per lane
 constexpr uint32_t kC4DirectBound = kC4HeavySlots / 2;  // heavy roots counted in one unbucketed pass
 constexpr uint32_t kC4MaxProbe = 64;            // bucket table probe limit
 constexpr uint32_t kAllBuckets = 0xFFFFFFFFu;
+// Direct counting of the heavy roots: 16-bit counters of kC4Range consecutive
+// ids fill the table's LDS, one atomic add per endpoint instead of a hash
+// insert.  Counts stay below 2^16: c(w) <= d(w), and larger degrees use the
+// hash.
+constexpr uint32_t kC4RangeBits = 16, kC4Range = 1u << kC4RangeBits;
+constexpr uint32_t kC4DenseRanges = 4;         // graphs of at most 4 ranges: one wedge stream per range, no scratch
+// Larger graphs: roots above this bound are bucketed by range, the others by
+// hash (a range costs its barriers and load latency however few endpoints it
+// gets; 4.84 M vertices, 74 ranges, heavy kernel by bound 32 / 64 / 128 / 256 /
+// 600 K: 24.9 / 25.1 / 25.8 / 27.0 / 29.3 ms).
+constexpr uint64_t kC4RangeBound = 64u << 10;
+constexpr uint64_t kC4HistBytes = 256u << 20;   // most memory of their range histograms
 
 // b(u) for every vertex (one wave per vertex).
 __global__ void c4_bound_kernel(const uint64_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
@@ -284,39 +298,48 @@ __device__ __forceinline__ uint32_t shfl_u32(uint32_t v, uint32_t l) { return ui
 
 // The wedges u - v - w (v = N(u)[k], k < pre; w in N(v), w < u) of one root,
 // streamed by one wave: groups of 64 neighbours v (k0, k0 + kstep, ...),
-// whose lists are concatenated; each lane walks its own contiguous range of
-// ceil(T / 64) positions of the concatenation (found once per group by a
-// binary search of the list offsets), kC4Unroll loads in flight, moving to
-// the next list when it reaches its offset.  The neighbours are in rank
-// order, i.e. by degree, so a group's lists have similar lengths.  f(w) runs
-// on the lanes holding an endpoint.  `wl` is the wave's LDS: 65 offsets
-// (the last one the total) and 64 list starts (census lists hold fewer
-// than 2^31 entries).
-template <class F>
+// whose lists are concatenated as aligned 16-byte groups of 4 entries; each
+// lane walks its own contiguous range of ceil(T / 64) groups of the
+// concatenation (found once per 64 neighbours by a binary search of the list
+// offsets), kC4Unroll loads in flight, moving to the next list when it
+// reaches its offset.  (Single entries took four loads for a group and
+// fetched each line again from L2 while the wave's other lanes' lines pushed
+// it out of L1: 10.4 ms to stream 2.3 G entries, 3.4 ms with groups, 4 in
+// flight.)  The neighbours are in rank order, i.e. by degree, so
+// their lists have similar lengths.  f(w) runs on the lanes holding an
+// endpoint.  `wl` is the wave's LDS (kC4ListWords): 65 offsets (the last one
+// the total), 64 list starts and 64 ends (census lists hold fewer than 2^31
+// entries; the column array is padded to whole groups).
+constexpr uint32_t kC4ListWords = 193;
+constexpr int kHeavyUnroll = 4;  // loads in flight: one 1024-thread workgroup per CU has the registers
+
+template <int kC4Unroll, class F>
 __device__ __forceinline__ void c4_wave_wedges(const uint64_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
                                                uint64_t ub, uint32_t pre, uint32_t u, uint32_t k0, uint32_t kstep,
                                                uint32_t* wl, F&& f) {
     const uint32_t lane = threadIdx.x & 63;
     uint32_t* soff = wl;
     uint32_t* sstart = wl + 65;
+    uint32_t* send = wl + 129;
     for (uint32_t k = k0; k < pre; k += kstep) {
-        uint32_t vb = 0, dv = 0;
+        uint32_t vb = 0, ve = 0;
         if (k + lane < pre) {
             const uint32_t v = ldg(col, ub + k + lane);
-            const uint64_t b = ldg(rowptr, v);
-            vb = uint32_t(b);
-            dv = uint32_t(ldg(rowptr, v + 1) - b);
+            vb = uint32_t(ldg(rowptr, v));
+            ve = uint32_t(ldg(rowptr, v + 1));
         }
+        const uint32_t dv = ve > vb ? ((ve + 3) >> 2) - (vb >> 2) : 0u;  // groups
         uint32_t incl = dv;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const uint32_t t = uint32_t(__shfl_up(int(incl), d));
             if (lane >= uint32_t(d)) incl += t;
         }
-        const uint32_t T = wave_lane(incl, 63);
+        const uint32_t T = wave_lane(incl, 63u);
         wave_lds_sync();
         soff[lane] = incl - dv;
         sstart[lane] = vb;
+        send[lane] = ve;
         if (lane == 63) soff[64] = T;
         wave_lds_sync();
         const uint32_t q = (T + 63) / 64;
@@ -330,28 +353,38 @@ __device__ __forceinline__ void c4_wave_wedges(const uint64_t* __restrict__ rowp
             if (t < 64 && soff[t] <= p) lo = t;
         }
         uint32_t nxt = soff[lo + 1];
-        uint32_t adr = sstart[lo] - soff[lo];  // col index of position p is adr + p (mod 2^32)
+        uint32_t b = sstart[lo], z = send[lo];
+        uint32_t adr = (b & ~3u) - 4 * soff[lo];  // col index of group p is adr + 4 p (mod 2^32)
         while (p < e) {
-            uint32_t ws[kC4Unroll];
+            u32x4 ws[kC4Unroll];
+            uint32_t first[kC4Unroll], last[kC4Unroll];  // entries [first, last) of the group are the list's
             const uint32_t cnt = min(uint32_t(kC4Unroll), e - p);
 #pragma unroll
             for (int c = 0; c < kC4Unroll; ++c) {
-                ws[c] = 0xFFFFFFFFu;
+                first[c] = last[c] = 0;
+                ws[c] = u32x4{0, 0, 0, 0};
                 if (uint32_t(c) < cnt) {
                     if (p == nxt) {
                         do {
                             ++lo;
                             nxt = soff[lo + 1];
                         } while (nxt == p);
-                        adr = sstart[lo] - soff[lo];
+                        b = sstart[lo];
+                        z = send[lo];
+                        adr = (b & ~3u) - 4 * soff[lo];
                     }
-                    ws[c] = ldg(col, uint64_t(adr + p));
+                    const uint32_t g = adr + 4 * p;
+                    first[c] = b > g ? b - g : 0u;
+                    last[c] = z - g < 4u ? z - g : 4u;
+                    ws[c] = ldg(reinterpret_cast<const u32x4*>(col), g >> 2);
                     ++p;
                 }
             }
 #pragma unroll
             for (int c = 0; c < kC4Unroll; ++c)
-                if (ws[c] < u) f(ws[c]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (uint32_t(t) >= first[c] && uint32_t(t) < last[c] && ws[c][t] < u) f(ws[c][t]);
         }
     }
 }
@@ -389,7 +422,7 @@ __global__ __launch_bounds__(256) void census_c4_wave_kernel(const uint64_t* __r
                                                              uint32_t* __restrict__ cursor,
                                                              unsigned long long* __restrict__ sums) {
     __shared__ uint32_t sKey[4][kC4WaveSlots], sCnt[4][kC4WaveSlots];
-    __shared__ uint32_t sList[4][129];
+    __shared__ uint32_t sList[4][kC4ListWords];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = threadIdx.x >> 6;
     uint32_t* key = sKey[wave];
@@ -411,7 +444,7 @@ __global__ __launch_bounds__(256) void census_c4_wave_kernel(const uint64_t* __r
         uint32_t H, hshift;
         c4_geometry(uint32_t(bound[u]), &H, &hshift);
         // the table is clear: every root clears what it used while summing
-        c4_wave_wedges(rowptr, col, ub, pre, u, 0, 64, sList[wave],
+        c4_wave_wedges<1>(rowptr, col, ub, pre, u, 0, 64, sList[wave],
                        [&](uint32_t w) { c4_hash_add(key, cnt, H - 1, hshift, w); });
         wave_lds_sync();
         for (uint32_t i = lane; i < H; i += 64) {
@@ -435,7 +468,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_block_kernel(const uint64_
                                                                    unsigned long long* __restrict__ sums) {
     __shared__ uint32_t sTask;
     __shared__ uint32_t sKey[kC4Slots], sCnt[kC4Slots];
-    __shared__ uint32_t sList[kC4Block / 64][129];
+    __shared__ uint32_t sList[kC4Block / 64][kC4ListWords];
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t nw = blockDim.x >> 6;
@@ -457,7 +490,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_block_kernel(const uint64_
         uint32_t H, hshift;
         c4_geometry(uint32_t(bound[u]), &H, &hshift);
         // the table is clear: every root clears what it used while summing
-        c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
+        c4_wave_wedges<1>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
                        [&](uint32_t w) { c4_hash_add(sKey, sCnt, H - 1, hshift, w); });
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < H; i += blockDim.x) {
@@ -507,7 +540,15 @@ __device__ void block_exclusive_scan(uint32_t* a, uint32_t P, uint32_t* wave_tot
     __syncthreads();
 }
 
-// Roots with b(u) > kC4BlockBound: one workgroup each.
+// Roots with b(u) > kC4BlockBound: one workgroup each.  In graphs of at most
+// kC4DenseRanges ranges of ids every endpoint has its own counter in LDS: one
+// stream of the wedges per range, no buckets.  In larger graphs the roots
+// above kC4RangeBound are bucketed by range (their sizes per range are part
+// of the prepared state) and each bucket is counted by adding its endpoints
+// and then taking each counter once.  Few buckets (74 for 4.84 M vertices,
+// not 4096) keep the buckets' tail lines in L2, so the scratch is written in
+// whole lines: 39.8 -> 11.5 GB a launch, and no hash inserts, table clears
+// or barriers per 4096 endpoints: 58.9 -> 25.1 ms.  The other roots:
 //   0. b(u) <= kC4DirectBound: one pass counts every endpoint in the LDS
 //      table (at most half full);
 //   1. endpoints are bucketed by a hash into P ~ b(u) / kC4BucketKeys
@@ -528,12 +569,17 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                                                                    uint32_t ntasks, uint32_t* __restrict__ cursor,
                                                                    uint32_t* __restrict__ scratch_slab,
                                                                    uint32_t scratch_keys, uint32_t max_slots,
-                                                                   uint32_t direct_bound,
+                                                                   uint32_t direct_bound, uint32_t dense_ranges,
+                                                                   const uint32_t* __restrict__ hist, uint32_t nhist,
+                                                                   uint32_t nranges,
                                                                    unsigned long long* __restrict__ sums) {
-    __shared__ uint32_t sKey[kC4HeavySlots], sCnt[kC4HeavySlots];
+    __shared__ uint32_t sTab[2 * kC4HeavySlots];  // hash keys and counts, or kC4Range 16-bit counters
+    static_assert(2 * kC4HeavySlots * 2 == kC4Range, "the counters fill the table");
+    uint32_t* sKey = sTab;
+    uint32_t* sCnt = sTab + kC4HeavySlots;
     __shared__ uint32_t sOff[kC4MaxBuckets + 1];
     __shared__ uint32_t sWave[kC4Block / 64];
-    __shared__ uint32_t sList[kC4Block / 64][129];
+    __shared__ uint32_t sList[kC4Block / 64][kC4ListWords];
     __shared__ uint32_t sTask, sB1;
     __shared__ uint32_t sOver[2];  // overflow flag per bucket part, alternating
     uint32_t* scratch = scratch_slab + size_t(blockIdx.x) * scratch_keys;
@@ -543,9 +589,10 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
     unsigned long long acc = 0;
     // the bucket table starts clear and every part clears what it used
     for (uint32_t i = threadIdx.x; i < kC4HeavySlots; i += blockDim.x) {
-        sKey[i] = kEmpty;
+        sKey[i] = dense_ranges ? 0u : kEmpty;
         sCnt[i] = 0;
     }
+    auto count_direct = [&](uint32_t w) { atomicAdd(&sTab[(w & (kC4Range - 1)) >> 1], 1u << (16 * (w & 1u))); };
     if (threadIdx.x == 0) sOver[0] = sOver[1] = 0;
     uint32_t flip = 0;
     while (true) {
@@ -558,6 +605,30 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
         const uint32_t du = uint32_t(ldg(rowptr, u + 1) - ub);
         const uint32_t pre = lower_bound_global(col + ub, du, u);
         const uint64_t bu = bound[u];
+        if (dense_ranges) {
+            // every id has a counter in at most kC4DenseRanges passes
+            for (uint32_t r = 0; r << kC4RangeBits < u; ++r) {
+                if (dense_ranges == 1)
+                    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], count_direct);
+                else
+                    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                        if (w >> kC4RangeBits == r) count_direct(w);
+                    });
+                __syncthreads();
+                const uint32_t ids = min(u - (r << kC4RangeBits), kC4Range);
+                for (uint32_t i = threadIdx.x; 2 * i < ids; i += blockDim.x) {
+                    const uint32_t x = sTab[i];
+                    if (x) {
+                        const uint64_t c0 = x & 0xFFFFu, c1 = x >> 16;
+                        acc += c0 * (c0 - 1) / 2 + c1 * (c1 - 1) / 2;
+                        sTab[i] = 0;
+                    }
+                }
+                __syncthreads();
+            }
+            continue;
+        }
+        const bool ranged = t < nhist;
         uint32_t P = 1, pbits = 0;
         while (P < kC4MaxBuckets && uint64_t(P) * kC4BucketKeys < bu) {
             P <<= 1;
@@ -621,7 +692,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                                 if (kw[c] != kEmpty && part_of(kw[c], parts) == part) add(kw[c]);
                         }
                     } else {
-                        c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                        c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                             if ((b == kAllBuckets || bucket_of(w) == b) && part_of(w, parts) == part) add(w);
                         });
                     }
@@ -650,19 +721,19 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
         // Roots with at most half as many wedges as the table has slots are
         // counted in one pass over the whole table (split only if a probe
         // run grows past the limit).
-        if (bu <= direct_bound && count_bucket(kAllBuckets, nullptr, uint32_t(bu), 2)) continue;
+        if (!ranged && bu <= direct_bound && count_bucket(kAllBuckets, nullptr, uint32_t(bu), 2)) continue;
         // When the scratch holds every bucket at a fixed capacity (1.5 times
         // the mean the bound allows, plus 64), one stream appends each
         // endpoint to its bucket; a bucket that fills up sends the root to
         // the exact path below, which larger roots take directly.
         const uint64_t cap64 = bu * 3 / (2 * uint64_t(P)) + 64;
-        bool exact = cap64 * P > scratch_keys;
+        bool exact = ranged || cap64 * P > scratch_keys;
         if (!exact) {
             const uint32_t cap = uint32_t(cap64);
             for (uint32_t b = threadIdx.x; b < P; b += blockDim.x) sOff[b] = 0;
             if (threadIdx.x == 0) sB1 = 0;  // a bucket filled up
             __syncthreads();
-            c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+            c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                 const uint32_t b = bucket_of(w);
                 const uint32_t pos = atomicAdd(&sOff[b], 1u);
                 if (pos < cap) scratch[b * cap + pos] = w;
@@ -677,15 +748,50 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                 }
         }
         if (!exact) continue;
-        // Exact path: histogram, exclusive scan of the bucket starts, then
-        // rounds of consecutive buckets whose endpoints fit the scratch.
+        // Exact path: histogram (the roots bucketed by range have theirs from
+        // the preparation), exclusive scan of the bucket starts, then rounds
+        // of consecutive buckets whose endpoints fit the scratch.
         __syncthreads();
-        for (uint32_t b = threadIdx.x; b <= P; b += blockDim.x) sOff[b] = 0;
-        __syncthreads();
-        c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
-                       [&](uint32_t w) { atomicAdd(&sOff[bucket_of(w)], 1u); });
+        if (ranged) {
+            P = nranges;
+            for (uint32_t b = threadIdx.x; b < P; b += blockDim.x) sOff[b] = hist[size_t(t) * nranges + b];
+            for (uint32_t i = threadIdx.x; i < kC4HeavySlots; i += blockDim.x) sKey[i] = 0;
+        } else {
+            for (uint32_t b = threadIdx.x; b <= P; b += blockDim.x) sOff[b] = 0;
+            __syncthreads();
+            c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
+                           [&](uint32_t w) { atomicAdd(&sOff[bucket_of(w)], 1u); });
+        }
         __syncthreads();
         block_exclusive_scan(sOff, P, sWave);
+        auto place_of = [&](uint32_t w) { return ranged ? w >> kC4RangeBits : bucket_of(w); };
+        // One range's endpoints, keys[0..k): add, then take each counter once.
+        auto count_range = [&](const uint32_t* keys, uint32_t k) {
+            constexpr int kU = 4;
+            for (uint32_t i0 = threadIdx.x; i0 < k; i0 += kU * blockDim.x) {
+                uint32_t kw[kU];
+#pragma unroll
+                for (int c = 0; c < kU; ++c) kw[c] = i0 + c * blockDim.x < k ? keys[i0 + c * blockDim.x] : kEmpty;
+#pragma unroll
+                for (int c = 0; c < kU; ++c)
+                    if (kw[c] != kEmpty) count_direct(kw[c]);
+            }
+            __syncthreads();
+            for (uint32_t i0 = threadIdx.x; i0 < k; i0 += kU * blockDim.x) {
+                uint32_t kw[kU];
+#pragma unroll
+                for (int c = 0; c < kU; ++c) kw[c] = i0 + c * blockDim.x < k ? keys[i0 + c * blockDim.x] : kEmpty;
+#pragma unroll
+                for (int c = 0; c < kU; ++c)
+                    if (kw[c] != kEmpty) {
+                        const uint32_t sh = 16 * (kw[c] & 1u);
+                        const uint32_t old = atomicAnd(&sTab[(kw[c] & (kC4Range - 1)) >> 1], ~(0xFFFFu << sh));
+                        const uint64_t n = (old >> sh) & 0xFFFFu;
+                        if (n > 1) acc += n * (n - 1) / 2;
+                    }
+            }
+            __syncthreads();
+        };
         uint32_t b0 = 0;
         while (b0 < P) {
             const uint32_t base0 = sOff[b0];
@@ -704,12 +810,26 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
             if (b1 == b0) {
                 // one bucket above the scratch: count it from the wedge stream
                 const uint32_t k = sOff[b0 + 1] - base0;
-                count_bucket(b0, nullptr, k, ~0u);
+                if (ranged) {
+                    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                        if (w >> kC4RangeBits == b0) count_direct(w);
+                    });
+                    __syncthreads();
+                    for (uint32_t i = threadIdx.x; 2 * i < kC4Range; i += blockDim.x) {
+                        const uint64_t c0 = sTab[i] & 0xFFFFu, c1 = sTab[i] >> 16;
+                        if (c0 > 1) acc += c0 * (c0 - 1) / 2;
+                        if (c1 > 1) acc += c1 * (c1 - 1) / 2;
+                        sTab[i] = 0;
+                    }
+                    __syncthreads();
+                } else {
+                    count_bucket(b0, nullptr, k, ~0u);
+                }
                 b0 += 1;
                 continue;
             }
-            c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
-                const uint32_t b = bucket_of(w);
+            c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                const uint32_t b = place_of(w);
                 if (b >= b0 && b < b1) scratch[atomicAdd(&sOff[b], 1u) - base0] = w;
             });
             __syncthreads();
@@ -717,13 +837,39 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
             for (uint32_t b = b0; b < b1; ++b) {
                 const uint32_t s0 = b == b0 ? base0 : sOff[b - 1];
                 const uint32_t k = sOff[b] - s0;
-                if (k > 1) count_bucket(b, scratch + (s0 - base0), k, ~0u);
+                if (k < 2) continue;
+                if (ranged) count_range(scratch + (s0 - base0), k);
+                else count_bucket(b, scratch + (s0 - base0), k, ~0u);
             }
             b0 = b1;
+        }
+        if (ranged) {
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < kC4HeavySlots; i += blockDim.x) sKey[i] = kEmpty;
         }
     }
     const unsigned long long x = wave_sum_u64(acc);
     if (lane == 0 && x) atomicAdd(&sums[6], x);
+}
+
+// Endpoints per range of the first heavy roots (one workgroup per root).
+__global__ __launch_bounds__(kC4Block) void census_c4_hist_kernel(const uint64_t* __restrict__ rowptr,
+                                                                  const uint32_t* __restrict__ col,
+                                                                  const uint32_t* __restrict__ tasks, uint32_t nranges,
+                                                                  uint32_t* __restrict__ hist) {
+    __shared__ uint32_t sHist[kC4MaxBuckets];
+    __shared__ uint32_t sList[kC4Block / 64][kC4ListWords];
+    const uint32_t wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const uint32_t u = wave_bcast(tasks[blockIdx.x]);
+    const uint64_t ub = ldg(rowptr, u);
+    const uint32_t du = uint32_t(ldg(rowptr, u + 1) - ub);
+    const uint32_t pre = lower_bound_global(col + ub, du, u);
+    for (uint32_t i = threadIdx.x; i < nranges; i += blockDim.x) sHist[i] = 0;
+    __syncthreads();
+    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
+                   [&](uint32_t w) { atomicAdd(&sHist[w >> kC4RangeBits], 1u); });
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < nranges; i += blockDim.x) hist[size_t(blockIdx.x) * nranges + i] = sHist[i];
 }
 
 static void hash_geometry(uint32_t Dmax, uint32_t* H, uint32_t* hshift) {
@@ -891,7 +1037,40 @@ static int prepare_c4(Ranked& R) {
         while (h < kC4HeavySlots && h < want) h <<= 1;
         R.c4_max_slots = h;
     }
-    if (R.n_c4_heavy) {
+    // heavy roots: direct counters over the whole graph when it has few
+    // ranges; otherwise the largest roots are bucketed by range
+    uint32_t maxdeg = 0;
+    if (n) KZ_HIP(hipMemcpy(&maxdeg, R.deg + (n - 1), 4, hipMemcpyDeviceToHost));  // ranked by degree
+    R.c4_ranges = (n + kC4Range - 1) >> kC4RangeBits;
+    // (any KZ_C4_* knob leaves direct counters to KZ_C4_RANGE_BOUND, which
+    // buckets the roots above it by range in a graph of any size)
+    uint64_t range_bound = kC4RangeBound;
+    const char* rb = std::getenv("KZ_C4_RANGE_BOUND");
+    if (rb) range_bound = std::strtoull(rb, nullptr, 10);
+    const bool knobs = rb || std::getenv("KZ_C4_DIRECT_BOUND") || std::getenv("KZ_C4_SCRATCH_KEYS") ||
+                       std::getenv("KZ_C4_BUCKET_SLOTS");
+    if (R.n_c4_heavy && maxdeg < (1u << 16) && (!knobs || rb)) {
+        if (R.c4_ranges <= kC4DenseRanges && !knobs) {
+            R.c4_dense = R.c4_ranges;
+        } else if (R.c4_ranges <= kC4MaxBuckets) {
+            const uint64_t most = kC4HistBytes / (4ull * R.c4_ranges);
+            while (R.c4_nhist < R.n_c4_heavy && R.c4_nhist < most && b[heavy[R.c4_nhist]] > range_bound &&
+                   b[heavy[R.c4_nhist]] < (uint64_t(1) << 32))
+                ++R.c4_nhist;
+            // (bucket offsets are 32-bit: a larger first root leaves all to the hash)
+        }
+        if (R.c4_nhist) {
+            KZ_HIP(hipMalloc(&R.c4_hist, 4ull * R.c4_nhist * R.c4_ranges));
+            R.bytes += 4ull * R.c4_nhist * R.c4_ranges;
+            hipLaunchKernelGGL(census_c4_hist_kernel, dim3(R.c4_nhist), dim3(kC4Block), 0, s, R.rowptr, R.col,
+                               R.c4_tasks + R.n_c4_wave + R.n_c4_block, R.c4_ranges, R.c4_hist);
+            KZ_HIP(hipGetLastError());
+            KZ_HIP(hipStreamSynchronize(s));
+        }
+    }
+    if (R.n_c4_heavy && R.c4_dense) {
+        R.c4_heavy_grid = std::min<uint32_t>(uint32_t(rt_.num_cus), R.n_c4_heavy);
+    } else if (R.n_c4_heavy) {
         size_t free_b = 0, total_b = 0;
         KZ_HIP(hipMemGetInfo(&free_b, &total_b));
         const size_t per_wg = size_t(R.c4_scratch_keys) * 4;
@@ -1002,7 +1181,7 @@ static int run_census(Ranked& R, uint64_t* sums, double* device_ms) {
         hipLaunchKernelGGL(census_c4_heavy_kernel, dim3(R.c4_heavy_grid), dim3(kC4Block), 0, s, R.rowptr, R.col,
                            R.c4_tasks + R.n_c4_wave + R.n_c4_block, R.c4_bound, R.n_c4_heavy,
                            R.cursor + 4 * kCursorStride, R.c4_scratch, R.c4_scratch_keys, R.c4_max_slots,
-                           R.c4_direct_bound, R.sums);
+                           R.c4_direct_bound, R.c4_dense, R.c4_hist, R.c4_nhist, R.c4_ranges, R.sums);
     if (R.n_c4_block)
         hipLaunchKernelGGL(census_c4_block_kernel, dim3(std::min<uint32_t>(R.n_c4_block, uint32_t(rt_.num_cus) * 2)),
                            dim3(kC4Block), 0, s, R.rowptr, R.col, R.c4_tasks + R.n_c4_wave, R.c4_bound, R.n_c4_block,

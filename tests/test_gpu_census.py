@@ -84,3 +84,25 @@ def test_census_rejects_oriented_graph(kzdev):
     with pytest.raises(kz.KzError):
         dg.motif_census()
     dg.release()
+
+
+@pytest.mark.parametrize("n,knobs", [
+    (60000, {}), (66000, {}), (150000, {}),  # counters of every id: one range, two, three
+    (400000, {}),  # seven ranges: bucketed by range above the default bound
+    (400000, {"KZ_C4_RANGE_BOUND": "4096"}),
+    (400000, {"KZ_C4_RANGE_BOUND": "4096", "KZ_C4_SCRATCH_KEYS": "9000"}),  # rounds of ranges
+    (400000, {"KZ_C4_RANGE_BOUND": "4096", "KZ_C4_SCRATCH_KEYS": "300"}),  # ranges above the scratch
+])
+def test_census_direct_counters(kzdev, monkeypatch, n, knobs):
+    """Heavy roots counted in one counter per id, by range."""
+    kz = kzdev
+    g = kz.gen_chung_lu(n, 5 * n, 2.2, 6000, n)
+    want = oracle.motif_census(g.rowptr, g.col)
+    for k, v in knobs.items():
+        monkeypatch.setenv(k, v)
+    print(f"[case] census n={n} {knobs}", flush=True)
+    dg = g.to_device()
+    got = dg.motif_census()
+    again = dg.motif_census()
+    dg.release()
+    assert got == want and again == want
