@@ -28,7 +28,7 @@ HIPCC = str(ROCM / "bin" / "hipcc")
 ARCH = "gfx950"
 
 HOST_SOURCES = ["kz_graph_host.cpp"]
-HIP_SOURCES = ["kz_runtime.hip", "kz_clique.hip", "kz_plan.hip", "kz_count.hip", "kz_setops.hip", "kz_workload.hip",
+HIP_SOURCES = ["kz_runtime.hip", "kz_clique.hip", "kz_plan.hip", "kz_plan3.hip", "kz_count.hip", "kz_setops.hip", "kz_workload.hip",
                "kz_census.hip", "kz_server.hip",
                "kz_gpugen.hip", "kz_fsm.hip", "kz_paged.hip"]
 

@@ -49,6 +49,7 @@ struct DeviceGraph {
     uint64_t nnz = 0;
     uint32_t max_degree = 0;
     int oriented = 0;
+    int symmetric = 0;  // every edge both ways: 1 yes, 2 no, 0 not checked yet (kz_plan3.hip)
     uint64_t* rowptr = nullptr;
     uint32_t* col = nullptr;
     uint32_t* deg = nullptr;

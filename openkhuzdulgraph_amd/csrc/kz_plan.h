@@ -16,6 +16,10 @@ int plan_validate(const PlanDesc& p);
 // Plain level-by-level execution of a plan on a resident graph.
 int plan_execute(DeviceGraph& g, const PlanDesc& p, bool count_only_last, uint64_t* raw_counts, kz_run_stats* st);
 
+// Counting plans of pattern size 3 in closed form (kz_plan3.hip); *taken is
+// clear when plan_execute has to run the plan.
+int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw_counts, kz_run_stats* st, bool* taken);
+
 // Order code of matched vertices m[0..s) (dense ranks, base s digits).
 static inline __host__ __device__ uint32_t order_code(const uint32_t* m, int s) {
     uint32_t code = 0, pw = 1;

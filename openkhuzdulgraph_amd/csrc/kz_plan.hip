@@ -1319,7 +1319,10 @@ int kz_count_plan(kz_graph g, const kz_plan_desc* plan, uint64_t* raw_counts, ui
     kz_run_stats st;
     std::memset(&st, 0, sizeof(st));
     uint64_t tmp[KZ_MAX_AGGREGATORS] = {0};
-    if (int e = plan_execute(g->g, *plan, false, tmp, &st)) return e;
+    bool taken = false;
+    if (int e = plan3_execute(g->g, *plan, tmp, &st, &taken)) return e;
+    if (!taken)
+        if (int e = plan_execute(g->g, *plan, false, tmp, &st)) return e;
     for (uint32_t i = 0; i < plan->num_aggregators; ++i) raw_counts[i] = tmp[i];
     st.wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (stats) *stats = st;
