@@ -1439,6 +1439,23 @@ static int launch_group(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s)
     return KZ_OK;
 }
 
+static int launch_group_k(CliqueJob& x, const CliqueJob::Group& gr, hipStream_t s) {
+    return gr.k == 3 ? launch_group<3>(x, gr, s) : gr.k == 4 ? launch_group<4>(x, gr, s) : launch_group<5>(x, gr, s);
+}
+
+static void launch_resets(CliqueJob& x, hipStream_t s) {
+    hipLaunchKernelGGL(reset_u32_kernel, dim3(1), dim3(256), 0, s, x.d_cursor, x.ncursor);
+    hipLaunchKernelGGL(reset_u64_kernel, dim3(1), dim3(256), 0, s, x.d_result, int(std::max<uint32_t>(1, x.nqueries)));
+}
+
+// The resets and every group's kernels, one after another.
+static int launch_all(CliqueJob& x, hipStream_t s) {
+    launch_resets(x, s);
+    for (const CliqueJob::Group& gr : x.groups)
+        if (int e = launch_group_k(x, gr, s)) return e;
+    return KZ_OK;
+}
+
 // Hub plan for one k: per-hub metadata, item and row prefixes, HBM slab.
 static int prepare_hubs(CliqueJob& x, int k, const std::vector<uint32_t>& hv, const std::vector<uint32_t>& hq,
                         const std::vector<uint32_t>& hd, hipStream_t st) {
@@ -1783,37 +1800,39 @@ int clique_job_prepare(CliqueJob& x, const std::vector<CliqueQuery>& queries, co
     KZ_HIP(hipMalloc(&x.d_result, sizeof(unsigned long long) * std::max<size_t>(1, queries.size())));
     x.bytes += sizeof(QueryRef) * qr.size() + 4 * std::max<size_t>(1, hv.size()) * (queries.size() > 1 ? 2 : 1) +
                4 * size_t(std::max(1, cursor)) + 8 * std::max<size_t>(1, queries.size());
-    const size_t nbr = std::max<size_t>(1, x.groups.size());
+    x.ncursor = std::max(1, cursor);
+    if (x.once) {  // launched kernel by kernel on the caller's stream
+        x.ready = true;
+        return KZ_OK;
+    }
+    // branch streams and events only where the groups run beside each other
+    const size_t nbr = cfg.serial ? 0 : x.groups.size();
     std::vector<hipStream_t> br(nbr, nullptr);
     std::vector<hipEvent_t> join(nbr, nullptr);
-    hipEvent_t fork;
+    hipEvent_t fork = nullptr;
     for (size_t i = 0; i < nbr; ++i) {
         KZ_HIP(hipStreamCreateWithFlags(&br[i], hipStreamNonBlocking));
         KZ_HIP(hipEventCreateWithFlags(&join[i], hipEventDisableTiming));
     }
-    KZ_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+    if (!cfg.serial) KZ_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
     // the launches' errors are read after the capture: start from none
     (void)hipGetLastError();
     KZ_HIP(hipStreamBeginCapture(main, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(reset_u32_kernel, dim3(1), dim3(256), 0, main, x.d_cursor, std::max(1, cursor));
-    hipLaunchKernelGGL(reset_u64_kernel, dim3(1), dim3(256), 0, main, x.d_result,
-                       int(std::max<size_t>(1, queries.size())));
-    KZ_HIP(hipEventRecord(fork, main));
     int e = KZ_OK;
-    // serial: one chain on the main stream; otherwise one branch per group
-    for (size_t i = 0; i < x.groups.size() && e == KZ_OK; ++i) {
-        hipStream_t s = cfg.serial ? main : br[i];
-        if (!cfg.serial) KZ_HIP(hipStreamWaitEvent(s, fork, 0));
-        const CliqueJob::Group& gr = x.groups[i];
-        if (gr.k == 3) e = launch_group<3>(x, gr, s);
-        else if (gr.k == 4) e = launch_group<4>(x, gr, s);
-        else e = launch_group<5>(x, gr, s);
-    }
-    if (!cfg.serial)
+    if (cfg.serial) {
+        e = launch_all(x, main);
+    } else {
+        launch_resets(x, main);
+        KZ_HIP(hipEventRecord(fork, main));
+        for (size_t i = 0; i < x.groups.size() && e == KZ_OK; ++i) {
+            KZ_HIP(hipStreamWaitEvent(br[i], fork, 0));
+            e = launch_group_k(x, x.groups[i], br[i]);
+        }
         for (size_t i = 0; i < x.groups.size(); ++i) {
             KZ_HIP(hipEventRecord(join[i], br[i]));
             KZ_HIP(hipStreamWaitEvent(main, join[i], 0));
         }
+    }
     hipGraph_t graph;
     KZ_HIP(hipStreamEndCapture(main, &graph));
     if (e == KZ_OK) {
@@ -1827,7 +1846,7 @@ int clique_job_prepare(CliqueJob& x, const std::vector<CliqueQuery>& queries, co
         hipStreamDestroy(br[i]);
         hipEventDestroy(join[i]);
     }
-    hipEventDestroy(fork);
+    if (fork) hipEventDestroy(fork);
     if (e) {
         hipGraphDestroy(graph);
         return e;
@@ -1851,7 +1870,12 @@ int clique_job_run(CliqueJob& x, uint64_t* counts, double* device_ms) {
     KZ_HIP(hipEventCreate(&a));
     KZ_HIP(hipEventCreate(&b));
     KZ_HIP(hipEventRecord(a, R.stream));
-    KZ_HIP(hipGraphLaunch(x.exec, R.stream));
+    if (x.once) {
+        if (int e = launch_all(x, R.stream)) return e;
+        KZ_HIP(hipGetLastError());
+    } else {
+        KZ_HIP(hipGraphLaunch(x.exec, R.stream));
+    }
     KZ_HIP(hipEventRecord(b, R.stream));
     std::vector<unsigned long long> res(std::max<uint32_t>(1, x.nqueries));
     KZ_HIP(hipMemcpyAsync(res.data(), x.d_result, sizeof(unsigned long long) * res.size(), hipMemcpyDeviceToHost,

@@ -261,6 +261,8 @@ struct CliqueJob {
         int cursor = 0;
     };
     bool ready = false;
+    bool once = false;  // set before the preparation: run once, kernel by kernel, without a captured graph
+    int ncursor = 0;    // u32 cursor words
     BucketCfg cfg{};
     uint32_t nqueries = 0;
     uint64_t ntasks = 0;

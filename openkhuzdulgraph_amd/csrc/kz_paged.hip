@@ -16,9 +16,13 @@
 //   * the lists of the highest-degree vertices (total degree >= the
 //     threshold, largest first, as many as cache_bytes holds) are kept in
 //     an HBM cache;
-//   * roots are cut into batches of consecutive ids whose undeduplicated
-//     list entries, d+(u) + sum over w in N+(u) of d+(w), fit the working
-//     buffer (list_bytes);
+//   * roots are cut into batches of consecutive ids whose lists -- the
+//     roots' own and their forward neighbours', each once -- fit the working
+//     buffer (list_bytes).  (Cut by their entries without deduplication, an
+//     RMAT-18 graph with an eighth of its lists in HBM took 1,300 batches of
+//     0.66 ms, nearly all of it launches and preparation: 860 ms a count;
+//     cut this way 840 batches, and launched without a captured graph each:
+//     245 ms);
 //   * per batch: a request kernel stamps every vertex the batch touches
 //     (the roots and their forward neighbours) with the batch number -- the
 //     deduplication --, the stamped vertices are compacted into a request
@@ -183,31 +187,71 @@ int kz_paged_create(const kz_csr* g, const kz_paged_cfg* cfg, kz_paged* out) {
         for (uint64_t i = g->rowptr[v]; i < g->rowptr[v + 1]; ++i)
             __atomic_fetch_add(&indeg[g->col[i]], 1u, __ATOMIC_RELAXED);
     }
-    // batches of consecutive roots whose undeduplicated list entries fit
+    // batches of consecutive roots whose distinct lists fit: greedy, in
+    // pieces of the root range with a batch stamp per vertex each (graphs of
+    // more than kPlanEdges entries a piece are cut in parallel; a batch does
+    // not cross a piece)
     const uint64_t cap = cfg->list_bytes / 4;
-    std::vector<uint64_t> cost(n);
-#pragma omp parallel for schedule(dynamic, 4096)
-    for (int64_t u = 0; u < int64_t(n); ++u) {
-        uint64_t c = p->h_deg[u];
-        for (uint64_t i = g->rowptr[u]; i < g->rowptr[u + 1]; ++i) c += p->h_deg[g->col[i]];
-        cost[u] = c;
-    }
-    uint64_t acc = 0, refs = 0;
-    for (uint32_t u = 0; u < n; ++u) {
-        if (cost[u] > cap)
-            KZ_FAIL(KZ_ERR_BUDGET, "root %u needs %llu list entries, more than list_bytes holds (%llu)", u,
-                    (unsigned long long)cost[u], (unsigned long long)cap);
-        if (acc + cost[u] > cap) {
-            p->batch_end.push_back(u);
-            p->batch_refs.push_back(refs);
-            acc = refs = 0;
+    constexpr uint64_t kPlanEdges = 16u << 20;
+    const uint32_t pieces =
+        uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(omp_get_max_threads()), m / kPlanEdges)));
+    struct Piece {
+        std::vector<uint32_t> end;
+        std::vector<uint64_t> refs;
+        uint64_t too_big = 0;  // entries of the first root that does not fit alone
+        uint32_t root = 0;
+    };
+    std::vector<Piece> plan(pieces);
+#pragma omp parallel for schedule(static, 1)
+    for (int64_t q = 0; q < int64_t(pieces); ++q) {
+        // pieces of about equal entries
+        auto start_of = [&](uint64_t i) {
+            return uint32_t(std::lower_bound(g->rowptr, g->rowptr + n, m / pieces * i) - g->rowptr);
+        };
+        const uint32_t u0 = q ? start_of(uint64_t(q)) : 0u, u1 = q + 1 < int64_t(pieces) ? start_of(uint64_t(q) + 1) : n;
+        Piece& P = plan[q];
+        std::vector<uint32_t> stamp(n, 0);
+        uint32_t epoch = 1;
+        uint64_t acc = 0, refs = 0;
+        for (uint32_t u = u0; u < u1; ++u) {
+            // entries root u adds to the batch
+            auto added = [&]() {
+                uint64_t c = stamp[u] == epoch ? 0 : p->h_deg[u];
+                for (uint64_t i = g->rowptr[u]; i < g->rowptr[u + 1]; ++i)
+                    if (stamp[g->col[i]] != epoch) c += p->h_deg[g->col[i]];
+                return c;
+            };
+            uint64_t c = added();
+            if (acc + c > cap) {
+                if (u > u0 && refs) {
+                    P.end.push_back(u);
+                    P.refs.push_back(refs);
+                }
+                ++epoch;
+                acc = refs = 0;
+                c = added();
+                if (c > cap) {
+                    P.too_big = c;
+                    P.root = u;
+                    break;
+                }
+            }
+            stamp[u] = epoch;
+            for (uint64_t i = g->rowptr[u]; i < g->rowptr[u + 1]; ++i) stamp[g->col[i]] = epoch;
+            acc += c;
+            refs += 1 + p->h_deg[u];
         }
-        acc += cost[u];
-        refs += 1 + p->h_deg[u];
+        if (refs) {
+            P.end.push_back(u1);
+            P.refs.push_back(refs);
+        }
     }
-    if (n) {
-        p->batch_end.push_back(n);
-        p->batch_refs.push_back(refs);
+    for (const Piece& P : plan) {
+        if (P.too_big)
+            KZ_FAIL(KZ_ERR_BUDGET, "root %u needs %llu list entries, more than list_bytes holds (%llu)", P.root,
+                    (unsigned long long)P.too_big, (unsigned long long)cap);
+        p->batch_end.insert(p->batch_end.end(), P.end.begin(), P.end.end());
+        p->batch_refs.insert(p->batch_refs.end(), P.refs.begin(), P.refs.end());
     }
     // cache: total degree >= threshold, largest first, while it fits
     std::vector<uint32_t> cand;
@@ -336,6 +380,7 @@ int kz_paged_count_cliques(kz_paged p, int k, uint64_t* count, kz_paged_stats* s
         st.request_refs += p->batch_refs[b];
         // count the batch's roots on the working rows
         CliqueJob job;
+        job.once = true;
         std::vector<CliqueQuery> q = {CliqueQuery{p->wrow, p->wcol, &p->h_deg, k, r0, r1, false}};
         if (int e = clique_job_prepare(job, q, default_buckets())) return e;
         uint64_t c = 0;
