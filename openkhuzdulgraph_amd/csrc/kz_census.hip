@@ -26,8 +26,8 @@
 //   2. one pass over vertices and F edges for the degree / t(e) sums.
 //   3. 4-cycles, each counted once from its highest-ranked vertex u: wedges
 //      u - v - w with v, w ranked below u (prefixes of the sorted relabelled
-//      lists) increment c(w) in a per-workgroup dense counter array in HBM,
-//      which also records the touched w; then sum C(c(w), 2) and clear.
+//      lists) count c(w) in LDS -- a hash of the endpoints for roots of few,
+//      one counter per id for the others --; then sum C(c(w), 2).
 //   4. 4-cliques: the persistent clique kernels on F.
 
 #include <hipcub/hipcub.hpp>
@@ -245,9 +245,7 @@ __global__ __launch_bounds__(256) void census_sums_kernel(const uint64_t* __rest
 // Roots are split by their wedge bound b(u) = sum of d(v) over v in N(u)
 // below u (c4_bound_kernel): b <= kC4WaveBound one wave per root with a
 // per-wave LDS hash of the endpoints; b <= kC4BlockBound one workgroup per
-// root with a workgroup hash; above it the workgroup buckets the root's
-// endpoints by a hash (an LDS histogram, then a scatter into an HBM scratch
-// region, bucket after bucket) and counts each bucket in the LDS hash.
+// root with a workgroup hash; above it census_c4_heavy_kernel.
 constexpr uint32_t kC4WaveSlots = 1024;    // per-wave hash: keys and counts, 8 KB
 constexpr uint32_t kC4WaveBound = kC4WaveSlots / 2;
 constexpr uint32_t kC4Slots = 8192;        // workgroup hash of the block kernel, 64 KB

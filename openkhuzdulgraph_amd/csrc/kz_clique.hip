@@ -11,29 +11,30 @@
 // (k-1)-cliques inside the out-neighbourhood N+(u).
 //
 // MI355X design (no counterpart in the reference):
-//   * one task = one root vertex u of one query (graph, k).  N+(u) is staged
-//     in LDS with an open-addressing hash (vertex id -> index);
-//   * the induced DAG on N+(u) is built as bitmap rows: row i holds bit j
-//     (j > i) iff N+(u)[j] is in N+(N+(u)[i]).  The lists N+(N+(u)[i]) of all
-//     rows are read as ONE stream of aligned 16-byte groups of 4 entries: an
-//     LDS prefix scan of the rows' group counts maps each lane's group index
-//     to (row, group), every lane keeps several independent 16-byte loads in
-//     flight and probes the hash with each entry (a wave walking one row at
-//     a time is bound by dependent load latency).  Rows whose list is much
-//     longer than their remaining candidates binary-search the candidates
-//     in the list instead;
-//   * cliques are counted with wave64 AND + popcount over the rows: k=4 sums
-//     popc(row_i & row_j) over DAG edges (i, j); k=5 descends one level more;
-//     k=3 counts the matches directly;
+//   * one task = one root vertex u of one query (graph, k).  The induced DAG on
+//     N+(u) is built as bitmap rows: row i holds bit j (j > i) iff N+(u)[j] is
+//     in N+(N+(u)[i]);
+//   * rows of candidates among the graph's highest ids come from the core
+//     bitmap (kz_core.h): one gathered load per 64 candidates and a compare;
+//   * the lists of the other rows are read as ONE stream of aligned 16-byte
+//     groups of 4 entries, probed in an LDS hash of N+(u) (vertex id ->
+//     index): an LDS prefix scan of the rows' group counts maps each lane's
+//     group index to (row, group), every lane keeps several independent
+//     16-byte loads in flight (a wave walking one row at a time is bound by
+//     dependent load latency).  Rows whose list is much longer than their
+//     remaining candidates binary-search the candidates in the list instead;
+//   * cliques are counted on the rows: k=4 and, above 128 candidates, k=5 as
+//     masked products on FP4 MFMA; k=5 below that edge by edge with popcounts;
+//     the wave bucket with one 64-bit row per lane; k=3 by the rows' bits;
 //   * tasks are bucketed by |N+(u)| with runtime bounds (autotunable): the
 //     first bucket (<= 64) runs one task per wave with one u64 row per
 //     candidate, the middle buckets one task per workgroup with rows in LDS,
 //     and roots above the last bound ("hubs") are split over many
-//     workgroups: a rows kernel builds chunks of rows into an HBM slab, then
-//     a count kernel takes one row per wave;
+//     workgroups: their rows go to an HBM slab, then a count kernel takes
+//     tile blocks (k = 4) or rows (k = 5) of all hubs;
 //   * every (k, bucket) is a persistent kernel pulling tasks, largest first,
-//     from a device atomic cursor; all of them are captured in one hipGraph
-//     with parallel branches, replayed per run.  A batch of many graphs and
+//     from a device atomic cursor; all of them are captured in one hipGraph,
+//     replayed per run.  A batch of many graphs and
 //     patterns is the same graph with tasks tagged by query.
 // Per-lane uint64 partial counts are reduced per wave and added to the
 // query's result with one 64-bit atomic when the wave moves to another
