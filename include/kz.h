@@ -358,8 +358,9 @@ int kz_fsm_domains(kz_graph g, uint32_t level, const uint32_t* labels, uint32_t*
 /* ---- Serving --------------------------------------------------------------
  * A server runs queries on resident graphs from a worker thread.  Queries
  * are admitted in arrival order while the device memory of the prepared
- * executions the server keeps (root task lists, bitmap slabs, census
- * copies) stays within hbm_budget bytes; idle prepared executions are
+ * executions the server keeps (root task lists, core bitmaps, bitmap slabs,
+ * census copies) stays within hbm_budget bytes (a core bitmap is left out
+ * where it does not fit); idle prepared executions are
  * released, least recently used first, to make room, and a query whose own
  * execution exceeds the budget fails with KZ_ERR_BUDGET.  Admitted queries
  * are launched as soon as they are prepared, up to max_inflight at once on
@@ -499,7 +500,10 @@ int kz_plan_clique(int k, kz_plan_desc* out);
  * are computed before use, sizes in range, last size has no scatter). */
 int kz_plan_validate(const kz_plan_desc* plan);
 
-/* Execute a plan with the plain level-by-level form.  raw_counts[a] gets the
+/* Execute a plan with the plain level-by-level form, or, for counting plans of
+ * size 3 over N(m_0) and N(m_1) on graphs that are oriented or store every
+ * edge both ways, in closed form from the graph's triangle count (which keeps
+ * what kz_count_cliques keeps with the graph).  raw_counts[a] gets the
  * uint64 sum of aggregator a (mod 2^64), before multiplicity division, as
  * Aggregator<EdgeId>::evaluate returns it (include/engine.h:628-645). */
 int kz_count_plan(kz_graph g, const kz_plan_desc* plan, uint64_t* raw_counts, uint32_t num_counts,
