@@ -208,6 +208,12 @@ typedef struct kz_run_stats {
  * forward out-degree still exceeds 8192 is counted by the plain form. */
 int kz_count_cliques(kz_graph g, int k, int method, uint64_t* count, kz_run_stats* stats);
 
+/* Device bytes a graph keeps for its persistent k-clique counts: out3[0] the
+ * degree-oriented copy of a symmetric graph (0 for an oriented one), out3[1]
+ * the prepared execution of this k (0 before the first count), of which
+ * out3[2] its core bitmap (0: it runs without one). */
+int kz_clique_kept_bytes(kz_graph g, int k, uint64_t* out3);
+
 /* Degree buckets of the persistent form: root tasks with |N+(u)| <= bound[0]
  * run one per wave (bound[0] <= 64); up to bound[1..3] one per workgroup
  * with bitmap rows in LDS (bound[3] <= 1024); larger ones keep rows in HBM.
@@ -359,10 +365,12 @@ int kz_fsm_domains(kz_graph g, uint32_t level, const uint32_t* labels, uint32_t*
  * A server runs queries on resident graphs from a worker thread.  Queries
  * are admitted in arrival order while the device memory of the prepared
  * executions the server keeps (root task lists, core bitmaps, bitmap slabs,
- * census copies) stays within hbm_budget bytes (a core bitmap is left out
- * where it does not fit); idle prepared executions are
- * released, least recently used first, to make room, and a query whose own
- * execution exceeds the budget fails with KZ_ERR_BUDGET.  Admitted queries
+ * census copies) stays within hbm_budget bytes; idle prepared executions are
+ * released, cheapest to rebuild first, to make room, and a query whose own
+ * execution exceeds the budget fails with KZ_ERR_BUDGET.  A clique
+ * execution's core bitmap only takes what is then left of the budget:
+ * nothing is released for it, and an execution whose bitmap does not fit
+ * runs without one.  Admitted queries
  * are launched as soon as they are prepared, up to max_inflight at once on
  * separate streams, so the device does not idle while queries wait
  * (continuous batching); two queries that need the same prepared execution

@@ -413,6 +413,13 @@ class DeviceGraph:
         self.last_stats = st.as_dict()
         return int(out.value)
 
+    def clique_kept_bytes(self, k: int) -> dict:
+        """Device bytes kept for k-clique counts: the oriented copy of a
+        symmetric graph, the prepared execution, its core bitmap."""
+        out = (C.c_uint64 * 3)()
+        check(lib().kz_clique_kept_bytes(self._h, k, out))
+        return {"forward": int(out[0]), "execution": int(out[1]), "core": int(out[2])}
+
     def tune_buckets(self, k: int, reps: int = 2) -> dict:
         """Autotune the degree-bucket thresholds of the persistent form."""
         cfg = _ffi.kz_bucket_cfg()

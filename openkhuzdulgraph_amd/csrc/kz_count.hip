@@ -189,6 +189,15 @@ int kz_count_cliques(kz_graph g, int k, int method, uint64_t* count, kz_run_stat
     return KZ_OK;
 }
 
+int kz_clique_kept_bytes(kz_graph g, int k, uint64_t* out3) {
+    if (!g || !out3 || k < 3 || k > 5) KZ_FAIL(KZ_ERR_INVALID, "bad argument");
+    const CliqueJob* j = static_cast<const CliqueJob*>(g->g.clique_exec[k].get());
+    out3[0] = g->g.fwd_bytes;
+    out3[1] = j ? j->bytes : 0;
+    out3[2] = j ? j->core_bytes : 0;
+    return KZ_OK;
+}
+
 int kz_clique_get_buckets(kz_graph g, int k, kz_bucket_cfg* out) {
     if (!g || !out || k < 3 || k > 5) KZ_FAIL(KZ_ERR_INVALID, "bad argument");
     to_abi(graph_buckets(g->g, k), out);

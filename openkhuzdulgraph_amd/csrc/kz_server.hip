@@ -209,12 +209,15 @@ uint64_t free_device_bytes() {
     return f;
 }
 
-// Frees idle prepared executions, lowest GreedyDual priority first, until
 // `need` more bytes fit in the budget and in the device's free memory.
-// Returns whether they fit.
+bool has_room(const kz_server_s* s, uint64_t need) {
+    return s->in_use + need <= budget_of(s) && (!need || free_device_bytes() >= need + kFreeMargin);
+}
+
+// Frees idle prepared executions, lowest GreedyDual priority first, until
+// `need` more bytes fit.  Returns whether they do.
 bool make_room(kz_server_s* s, uint64_t need) {
-    const uint64_t B = budget_of(s);
-    while (s->in_use + need > B || (need && free_device_bytes() < need + kFreeMargin)) {
+    while (!has_room(s, need)) {
         Prepared* victim = nullptr;
         for (Prepared* p : s->prepared)
             if (releasable(s, p) && (!victim || p->H < victim->H)) victim = p;
@@ -362,10 +365,12 @@ void collect_aux(kz_server_s* s, std::vector<SQuery*>* gone) {
         Prepared* p = j.p;
         const kz_graph g = p->g;
         DeviceGraph& d = g->g;
-        if (j.rc && (j.rc == KZ_ERR_NOMEM || j.rc == KZ_ERR_DEVICE) && !p->retried && release_idle(s, p)) {
+        if (j.rc && (j.rc == KZ_ERR_NOMEM || j.rc == KZ_ERR_DEVICE) && !p->retried &&
+            (release_idle(s, p) || p->core_limit)) {
             // out of device memory despite the estimate: once more, with
-            // every idle execution released
+            // every idle execution released and without a core bitmap
             p->retried = true;
+            p->core_limit = 0;
             aux_submit(s->prep, j);
             continue;
         }
@@ -468,30 +473,31 @@ int admit(kz_server_s* s, SQuery* q, int* free_slot) {
                 f->busy = 0;
             }
         }
-        // a job kept from a direct call is adopted; one whose core bitmap
-        // alone takes it past the budget is prepared again without
-        auto job_of = [&]() { return static_cast<CliqueJob*>(d.clique_exec[q->k].get()); };
-        if (job_of() && job_of()->core_bytes && job_of()->bytes > budget_of(s)) d.clique_exec[q->k].reset();
-        const bool cached = bool(d.clique_exec[q->k]);
-        const uint64_t base = cached ? job_of()->bytes : estimate_bytes(d, q->kind, q->k);
+        // A job kept from a direct call is adopted.  Room is made for the job
+        // without its core bitmap; the bitmap is an extra that takes what is
+        // then left of the budget and that nothing is released for.  A kept
+        // job whose bitmap does not fit is prepared again without it (its
+        // other bytes are known exactly).
+        CliqueJob* kept = static_cast<CliqueJob*>(d.clique_exec[q->k].get());
+        const uint64_t base = kept ? kept->bytes - kept->core_bytes : estimate_bytes(d, q->kind, q->k);
+        uint64_t core = kept ? kept->core_bytes : clique_core_bytes(d.n, d.oriented ? d.nnz : d.nnz / 2);
         if (base > budget_of(s)) {
             finish(s, q, KZ_ERR_BUDGET);
             return 1;
         }
-        // the core bitmap is left out where it does not fit the budget
-        uint64_t core = cached ? 0 : clique_core_bytes(d.n, d.oriented ? d.nnz : d.nnz / 2);
-        if (base + core > budget_of(s)) core = 0;
         if (f) f->busy++;  // the job needs it: not a victim for its room
-        bool room = make_room(s, base + core);
-        if (!room && core) {
-            core = 0;
-            room = make_room(s, base);
-        }
+        const bool room = make_room(s, base);
         if (f) f->busy--;
         if (!room) return no_room();
+        // (a kept bitmap is in device memory already: only the budget counts)
+        if (core && !(kept ? s->in_use + base + core <= budget_of(s) : has_room(s, base + core))) {
+            core = 0;
+            d.clique_exec[q->k].reset();
+            kept = nullptr;
+        }
         p = reserve(s, q->g, q->kind, q->k, base + core);
         p->core_limit = core;
-        if (!cached) {
+        if (!kept) {
             aux_submit(s->prep, AuxJob{kJobPrepare, q, p, 0, 0});
             return 0;
         }

@@ -126,3 +126,70 @@ def test_queries_are_admitted_during_a_census_and_a_preparation(kzdev):
         assert rq["status"] == 0 and rq["counts"][0] == want_small
         assert rb["status"] == 0 and rb["counts"][0] == want_big
         assert big_running, (rq, rb)
+
+
+def _big_chunglu(kz):
+    return kz.gen_chung_lu(20000, 400000, 2.2, 2000, 12)
+
+
+def test_a_kept_job_whose_core_does_not_fit_beside_the_forward_copy(kzdev):
+    """A symmetric graph counted directly first keeps its forward copy and a
+    4-clique job with a core bitmap.  A budget that holds both without the
+    bitmap serves the query, one that holds the bitmap too adopts the job."""
+    kz = kzdev
+    g = _big_chunglu(kz)
+    want = oracle.run_app(APP[4], g.rowptr, g.col)[1][0]
+    for slack, core_kept in ((0, True), (-1, False)):
+        dg = g.to_device()
+        assert dg.count_cliques(4) == want
+        kept = dg.clique_kept_bytes(4)
+        assert kept["forward"] and kept["core"] and kept["execution"] > kept["core"], kept
+        budget = kept["forward"] + kept["execution"] + slack
+        print(f"[case] server budget {budget} on {kept}", flush=True)
+        with kz.Server(hbm_budget=budget, max_inflight=2) as srv:
+            for _ in range(2):
+                res = srv.poll(srv.submit(dg, "clique", 4), wait=True)
+                assert res["status"] == 0 and res["counts"][0] == want, res
+            now = dg.clique_kept_bytes(4)  # no query in flight
+            assert now["core"] == (kept["core"] if core_kept else 0), now
+        # without the bitmap it does not fit either: refused as before
+        if not core_kept:
+            dg2 = g.to_device()
+            assert dg2.count_cliques(4) == want
+            with kz.Server(hbm_budget=kept["forward"] + kept["execution"] - kept["core"] - 1, max_inflight=2) as srv:
+                res = srv.poll(srv.submit(dg2, "clique", 4), wait=True)
+                assert res["status"] == kz._ffi.KZ_ERR_BUDGET, res
+            dg2.release()
+        dg.release()
+
+
+def test_a_core_bitmap_evicts_no_prepared_execution(kzdev):
+    """Room for two executions but not for the second one's core bitmap: the
+    first one stays prepared and the second runs without a bitmap."""
+    kz = kzdev
+    a, b = kz.gen_rmat(12, 16, seed=4).oriented(), _big_chunglu(kz).oriented()
+    wa = oracle.run_app(APP[4], a.rowptr, a.col)[1][0]
+    wb = oracle.run_app(APP[4], b.rowptr, b.col)[1][0]
+    kept = {}
+    for name, g, want in (("a", a, wa), ("b", b, wb)):
+        probe = g.to_device()
+        assert probe.count_cliques(4) == want
+        kept[name] = probe.clique_kept_bytes(4)
+        probe.release()
+    assert kept["a"]["core"] and kept["b"]["core"], kept
+    # an execution on an oriented graph without hubs is admitted at 8 bytes a
+    # vertex and 1 MB, then held at its real size
+    assert max(a.max_degree, b.max_degree) <= 1024
+    budget = 8 * b.num_vertices + (1 << 20) + kept["b"]["core"] + kept["a"]["execution"] // 2
+    assert kept["a"]["execution"] // 2 < kept["b"]["core"], kept
+    da, db = a.to_device(), b.to_device()
+    print(f"[case] server cores {kept}, budget {budget}", flush=True)
+    with kz.Server(hbm_budget=budget, max_inflight=2) as srv:
+        ra = srv.poll(srv.submit(da, "clique", 4), wait=True)
+        rb = srv.poll(srv.submit(db, "clique", 4), wait=True)
+        assert ra["counts"][0] == wa and rb["counts"][0] == wb, (ra, rb)
+        now = da.clique_kept_bytes(4), db.clique_kept_bytes(4)  # no query in flight
+    assert now[0] == kept["a"], "the first execution was released or lost its bitmap"
+    assert now[1]["execution"] and now[1]["core"] == 0, now
+    da.release()
+    db.release()
