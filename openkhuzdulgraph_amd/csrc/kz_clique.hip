@@ -1583,15 +1583,16 @@ uint64_t clique_core_bytes(uint64_t n, uint64_t nnz) {
 
 // The cores of the queries' graphs (one per distinct graph), built on st; the
 // queries' references point at them when st has run.  A graph has none where
-// they would pass core_limit or an eighth of the free device memory, where
-// the allocation fails, or where its roots have many more candidate pairs
+// they would pass core_limit or an eighth of the device memory that the job's
+// own `need` bytes leave free, where the allocation fails, or where its roots have many more candidate pairs
 // than its candidates' lists have entries (an orientation that is not by
 // degree can have roots of thousands of candidates with almost empty lists):
 // there the stream is cheaper.  A pair costs about an eighth of a streamed
 // entry.
 constexpr uint64_t kCorePairsPerEntry = 8;
 
-static int build_cores(CliqueJob& x, const std::vector<CliqueQuery>& queries, std::vector<QueryRef>& qr, hipStream_t st) {
+static int build_cores(CliqueJob& x, const std::vector<CliqueQuery>& queries, std::vector<QueryRef>& qr, uint64_t need,
+                       hipStream_t st) {
     struct Cand {
         const CliqueQuery* q;
         uint64_t nnz = 0, pairs = 0;
@@ -1612,10 +1613,10 @@ static int build_cores(CliqueJob& x, const std::vector<CliqueQuery>& queries, st
         at[Q.col] = cand.size();
         cand.push_back(c);
     }
-    if (!cand.empty()) {
+    if (!cand.empty() && x.core_limit) {
         size_t free_b = 0, total_b = 0;
         KZ_HIP(hipMemGetInfo(&free_b, &total_b));
-        const uint64_t limit = std::min<uint64_t>(x.core_limit, free_b / 8);
+        const uint64_t limit = std::min<uint64_t>(x.core_limit, (free_b - std::min<uint64_t>(free_b, need)) / 8);
         // sampled list entries behind each graph's edges
         std::vector<CoreGraph> cg(cand.size());
         std::vector<unsigned long long> sums(cand.size(), 0);
@@ -1738,7 +1739,13 @@ int clique_job_prepare(CliqueJob& x, const std::vector<CliqueQuery>& queries, co
         ~StreamFree() { (void)hipStreamDestroy(s); }
     } main_free{main};
     std::vector<QueryRef> qr(std::max<size_t>(1, queries.size()));
-    if (int e = build_cores(x, queries, qr, main)) return e;
+    // task lists and hub slabs, allocated after the cores
+    uint64_t need = 8 * ntask + (1u << 20);
+    for (int k = 4; k <= 5; ++k) {
+        const auto& hubs = cnt[(k - 3) * kNumBuckets + kNumBuckets - 1];
+        for (size_t d = 0; d < hubs.size(); ++d) need += hubs[d] * (8 * d * ((d + 63) / 64));
+    }
+    if (int e = build_cores(x, queries, qr, need, main)) return e;
     KZ_HIP(hipMalloc(&x.d_queries, sizeof(QueryRef) * qr.size()));
     KZ_HIP(hipMemcpyAsync(x.d_queries, qr.data(), sizeof(QueryRef) * qr.size(), hipMemcpyHostToDevice, main));
     KZ_HIP(hipStreamSynchronize(main));  // the cores are built, the references in place
