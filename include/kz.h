@@ -303,6 +303,10 @@ int kz_paged_release(kz_paged p);
  * (KZ_ERR_INVALID). */
 #define KZ_CENSUS_PATTERNS 8
 int kz_motif_census(kz_graph g, uint64_t* counts, kz_run_stats* stats);
+/* Device bytes a graph keeps for its census: out2[0] all of them (0 before the
+ * first one), out2[1] those it can do without (its 4-clique execution's core
+ * bitmap, histograms of its largest roots). */
+int kz_census_kept_bytes(kz_graph g, uint64_t* out2);
 
 /* ---------------------------------------------- labelled pattern mining -- */
 
@@ -367,10 +371,10 @@ int kz_fsm_domains(kz_graph g, uint32_t level, const uint32_t* labels, uint32_t*
  * executions the server keeps (root task lists, core bitmaps, bitmap slabs,
  * census copies) stays within hbm_budget bytes; idle prepared executions are
  * released, cheapest to rebuild first, to make room, and a query whose own
- * execution exceeds the budget fails with KZ_ERR_BUDGET.  A clique
- * execution's core bitmap only takes what is then left of the budget:
- * nothing is released for it, and an execution whose bitmap does not fit
- * runs without one.  Admitted queries
+ * execution exceeds the budget fails with KZ_ERR_BUDGET.  Core
+ * bitmaps and the histograms of a census only take what is then left of the
+ * budget: nothing is released for them, and an execution that has no room
+ * for them runs without.  Admitted queries
  * are launched as soon as they are prepared, up to max_inflight at once on
  * separate streams, so the device does not idle while queries wait
  * (continuous batching); two queries that need the same prepared execution

@@ -420,6 +420,12 @@ class DeviceGraph:
         check(lib().kz_clique_kept_bytes(self._h, k, out))
         return {"forward": int(out[0]), "execution": int(out[1]), "core": int(out[2])}
 
+    def census_kept_bytes(self) -> dict:
+        """Device bytes kept for the census, and those of its optional parts."""
+        out = (C.c_uint64 * 2)()
+        check(lib().kz_census_kept_bytes(self._h, out))
+        return {"state": int(out[0]), "extra": int(out[1])}
+
     def tune_buckets(self, k: int, reps: int = 2) -> dict:
         """Autotune the degree-bucket thresholds of the persistent form."""
         cfg = _ffi.kz_bucket_cfg()

@@ -259,6 +259,7 @@ _SIGS = {
     "kz_server_poll": (C.c_int, [C.c_void_p, C.c_uint64, C.c_int, C.POINTER(kz_query_result)]),
     "kz_server_stop": (C.c_int, [C.c_void_p]),
     "kz_clique_kept_bytes": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_uint64)]),
+    "kz_census_kept_bytes": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64)]),
     "kz_clique_get_buckets": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(kz_bucket_cfg)]),
     "kz_clique_set_buckets": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(kz_bucket_cfg)]),
     "kz_clique_tune": (C.c_int, [C.c_void_p, C.c_int, C.c_uint32, C.POINTER(kz_bucket_cfg), C.POINTER(C.c_double)]),

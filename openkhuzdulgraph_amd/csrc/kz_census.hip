@@ -81,6 +81,9 @@ struct Ranked {
     uint32_t* cursor = nullptr;      // kCursors task cursors, kCursorStride words apart
     unsigned long long* sums = nullptr;  // 8 accumulators
     uint64_t bytes = 0;           // device memory held (with the 4-clique job)
+    // the parts it runs without where they do not fit, included in bytes: the
+    // 4-clique job's core bitmap and the range histograms
+    uint64_t extra_bytes = 0;
     CliqueJob k4;
     ~Ranked() {
         for (void* p : {(void*)rowptr, (void*)col, (void*)deg, (void*)frowptr, (void*)fcol, (void*)tasks, (void*)troot,
@@ -1057,8 +1060,8 @@ static int build_ranked(DeviceGraph& g, Ranked& R) {
 // 4-cycle pass: wedge bounds, the three root lists (largest bound first),
 // and the heavy kernel's endpoint scratch (one region per workgroup, one
 // workgroup per CU, fewer when the regions would take more than a quarter
-// of free memory).
-static int prepare_c4(Ranked& R) {
+// of free memory).  *ranged: the heavy roots worth bucketing by range.
+static int prepare_c4(Ranked& R, uint32_t* ranged) {
     const Runtime& rt_ = rt();
     hipStream_t s = rt_.stream;
     const uint32_t n = R.n;
@@ -1118,23 +1121,15 @@ static int prepare_c4(Ranked& R) {
     if (rb) range_bound = std::strtoull(rb, nullptr, 10);
     const bool knobs = rb || std::getenv("KZ_C4_DIRECT_BOUND") || std::getenv("KZ_C4_SCRATCH_KEYS") ||
                        std::getenv("KZ_C4_BUCKET_SLOTS");
+    *ranged = 0;
     if (R.n_c4_heavy && maxdeg < (1u << 16) && (!knobs || rb)) {
         if (R.c4_ranges <= kC4DenseRanges && !knobs) {
             R.c4_dense = R.c4_ranges;
         } else if (R.c4_ranges <= kC4MaxBuckets) {
-            const uint64_t most = kC4HistBytes / (4ull * R.c4_ranges);
-            while (R.c4_nhist < R.n_c4_heavy && R.c4_nhist < most && b[heavy[R.c4_nhist]] > range_bound &&
-                   b[heavy[R.c4_nhist]] < (uint64_t(1) << 32))
-                ++R.c4_nhist;
+            while (*ranged < R.n_c4_heavy && b[heavy[*ranged]] > range_bound &&
+                   b[heavy[*ranged]] < (uint64_t(1) << 32))
+                ++*ranged;
             // (bucket offsets are 32-bit: a larger first root leaves all to the hash)
-        }
-        if (R.c4_nhist) {
-            KZ_HIP(hipMalloc(&R.c4_hist, 4ull * R.c4_nhist * R.c4_ranges));
-            R.bytes += 4ull * R.c4_nhist * R.c4_ranges;
-            hipLaunchKernelGGL(census_c4_hist_kernel, dim3(R.c4_nhist), dim3(kC4Block), 0, s, R.rowptr, R.col,
-                               R.c4_tasks + R.n_c4_wave + R.n_c4_block, R.c4_ranges, R.c4_hist);
-            KZ_HIP(hipGetLastError());
-            KZ_HIP(hipStreamSynchronize(s));
         }
     }
     if (R.n_c4_heavy && R.c4_dense) {
@@ -1154,8 +1149,33 @@ static int prepare_c4(Ranked& R) {
     return KZ_OK;
 }
 
-// Task lists, per-edge arrays, the 4-cycle pass and the 4-clique job.
-static int prepare_passes(Ranked& R) {
+// Range histograms of the first `ranged` heavy roots, as many as `limit` bytes
+// and kC4HistBytes hold; the others, and all where the allocation fails, are
+// bucketed by hash.
+static int prepare_c4_hist(Ranked& R, uint32_t ranged, uint64_t limit) {
+    const uint64_t per_root = 4ull * R.c4_ranges;
+    if (!ranged || !per_root) return KZ_OK;
+    const uint32_t nhist = uint32_t(std::min<uint64_t>(ranged, std::min(kC4HistBytes, limit) / per_root));
+    if (!nhist) return KZ_OK;
+    if (hipMalloc(&R.c4_hist, per_root * nhist) != hipSuccess) {
+        (void)hipGetLastError();
+        R.c4_hist = nullptr;
+        return KZ_OK;
+    }
+    hipStream_t s = rt().stream;
+    hipLaunchKernelGGL(census_c4_hist_kernel, dim3(nhist), dim3(kC4Block), 0, s, R.rowptr, R.col,
+                       R.c4_tasks + R.n_c4_wave + R.n_c4_block, R.c4_ranges, R.c4_hist);
+    KZ_HIP(hipGetLastError());
+    KZ_HIP(hipStreamSynchronize(s));
+    R.c4_nhist = nhist;
+    R.extra_bytes += per_root * nhist;
+    R.bytes += per_root * nhist;
+    return KZ_OK;
+}
+
+// Task lists, per-edge arrays, the 4-cycle pass and the 4-clique job; its core
+// bitmap and the range histograms take at most extra_limit bytes.
+static int prepare_passes(Ranked& R, uint64_t extra_limit) {
     const Runtime& rt_ = rt();
     std::vector<uint32_t> small, large;
     for (uint32_t v = 0; v < R.n; ++v) {
@@ -1186,20 +1206,23 @@ static int prepare_passes(Ranked& R) {
     KZ_HIP(hipMalloc(&R.cursor, 4 * kCursors * kCursorStride));
     KZ_HIP(hipMalloc(&R.sums, 8 * 8));
     R.bytes += 8 * (2 * std::max<uint64_t>(1, R.fnnz) + all.size() + 8);
-    if (int e = prepare_c4(R)) return e;
+    uint32_t ranged = 0;
+    if (int e = prepare_c4(R, &ranged)) return e;
     std::vector<CliqueQuery> q = {CliqueQuery{R.frowptr, R.fcol, &R.h_fdeg, 4}};
+    R.k4.core_limit = extra_limit;
     if (int e = clique_job_prepare(R.k4, q, default_buckets())) return e;
     R.bytes += R.k4.bytes;
-    return KZ_OK;
+    R.extra_bytes = R.k4.core_bytes;
+    return prepare_c4_hist(R, ranged, extra_limit - R.k4.core_bytes);
 }
 
-static int census_state(DeviceGraph& g, Ranked** out) {
+static int census_state(DeviceGraph& g, uint64_t extra_limit, Ranked** out) {
     if (!g.census) {
         Ranked* R = new (std::nothrow) Ranked();
         if (!R) KZ_FAIL(KZ_ERR_NOMEM, "census state");
         std::shared_ptr<void> holder(R, [](void* p) { delete static_cast<Ranked*>(p); });
         if (int e = build_ranked(g, *R)) return e;
-        if (int e = prepare_passes(*R)) return e;
+        if (int e = prepare_passes(*R, extra_limit)) return e;
         g.census = holder;
     }
     *out = static_cast<Ranked*>(g.census.get());
@@ -1283,11 +1306,17 @@ uint64_t census_bytes(const DeviceGraph& d) {
     return d.census ? static_cast<const Ranked*>(d.census.get())->bytes : 0;
 }
 
-int motif_census(DeviceGraph& d, uint64_t* counts, kz_run_stats* stats) {
+uint64_t census_extra_bytes(const DeviceGraph& d) {
+    return d.census ? static_cast<const Ranked*>(d.census.get())->extra_bytes : 0;
+}
+
+uint64_t census_extra_estimate(const DeviceGraph& d) { return clique_core_bytes(d.n, d.nnz / 2) + kC4HistBytes; }
+
+int motif_census(DeviceGraph& d, uint64_t* counts, kz_run_stats* stats, uint64_t extra_limit) {
     if (d.oriented) KZ_FAIL(KZ_ERR_INVALID, "the census needs a symmetric graph");
     auto t0 = std::chrono::steady_clock::now();
     Ranked* R = nullptr;
-    if (int e = census_state(d, &R)) return e;
+    if (int e = census_state(d, extra_limit, &R)) return e;
     uint64_t S[8];
     double ms = 0;
     if (int e = run_census(*R, S, &ms)) return e;
@@ -1326,6 +1355,13 @@ int motif_census(DeviceGraph& d, uint64_t* counts, kz_run_stats* stats) {
 }
 
 }  // namespace kz
+
+extern "C" int kz_census_kept_bytes(kz_graph g, uint64_t* out2) {
+    if (!g || !out2) KZ_FAIL(KZ_ERR_INVALID, "null argument");
+    out2[0] = kz::census_bytes(g->g);
+    out2[1] = kz::census_extra_bytes(g->g);
+    return KZ_OK;
+}
 
 extern "C" int kz_motif_census(kz_graph g, uint64_t* counts, kz_run_stats* stats) {
     if (!g || !counts) KZ_FAIL(KZ_ERR_INVALID, "null argument");

@@ -314,9 +314,13 @@ int clique_job_launch(CliqueJob& x, hipStream_t s, unsigned long long* host_resu
 int graph_job(DeviceGraph& d, int k, CliqueJob** out, uint64_t core_limit = ~uint64_t(0));
 // Motif census of a symmetric resident graph; the relabelled copy and
 // counter slabs are kept in the graph (kz_census.hip).  census_bytes is the
-// device memory that state holds (0 before the first call).
-int motif_census(DeviceGraph& d, uint64_t* counts, kz_run_stats* stats);
+// device memory that state holds (0 before the first call), of which
+// census_extra_bytes are parts it can be built without; extra_limit bounds
+// them when it is built (census_extra_estimate: the most they take).
+int motif_census(DeviceGraph& d, uint64_t* counts, kz_run_stats* stats, uint64_t extra_limit = ~uint64_t(0));
 uint64_t census_bytes(const DeviceGraph& d);
+uint64_t census_extra_bytes(const DeviceGraph& d);
+uint64_t census_extra_estimate(const DeviceGraph& d);
 int clique_workload(const CliqueView& gv, uint64_t* out6);
 // Forward part of a graph for the clique kernels: the graph itself when it
 // is degree-oriented, else its orientation by (degree, id) rank, built once

@@ -67,7 +67,7 @@ struct Prepared {
     int busy = 0;        // launched queries or helper work using it
     bool preparing = false;
     bool retried = false;
-    uint64_t core_limit = 0;  // bytes its core bitmap may take
+    uint64_t extra_limit = 0;  // bytes its optional parts (a core bitmap, census histograms) may take
 };
 
 // Work for a helper thread.
@@ -274,11 +274,11 @@ void aux_run(AuxJob& j) {
         j.rc = ensure_forward(d);
     } else if (j.type == kJobPrepare) {
         CliqueJob* job = nullptr;
-        j.rc = graph_job(d, j.p->k, &job, j.p->core_limit);
+        j.rc = graph_job(d, j.p->k, &job, j.p->extra_limit);
     } else {
         kz_run_stats st;
         j.q->t_start = t0;
-        j.rc = motif_census(d, j.q->res.counts, &st);
+        j.rc = motif_census(d, j.q->res.counts, &st, j.p->extra_limit);
     }
     if (j.rc) j.err = get_error();
     j.ms = ms_between(t0, Clock::now());
@@ -366,11 +366,11 @@ void collect_aux(kz_server_s* s, std::vector<SQuery*>* gone) {
         const kz_graph g = p->g;
         DeviceGraph& d = g->g;
         if (j.rc && (j.rc == KZ_ERR_NOMEM || j.rc == KZ_ERR_DEVICE) && !p->retried &&
-            (release_idle(s, p) || p->core_limit)) {
+            (release_idle(s, p) || p->extra_limit)) {
             // out of device memory despite the estimate: once more, with
             // every idle execution released and without a core bitmap
             p->retried = true;
-            p->core_limit = 0;
+            p->extra_limit = 0;
             aux_submit(s->prep, j);
             continue;
         }
@@ -398,6 +398,7 @@ void collect_aux(kz_server_s* s, std::vector<SQuery*>* gone) {
             // a HIP runtime error (as preparations, once more; a lasting
             // one fails the second run too)
             j.q->retried = true;
+            p->extra_limit = 0;
             aux_submit(s->census, AuxJob{kJobCensus, j.q, p, 0, 0});
             continue;
         }
@@ -432,16 +433,25 @@ int admit(kz_server_s* s, SQuery* q, int* free_slot) {
     if (q->kind == KZ_QUERY_CENSUS) {
         if (s->census.pending) return 0;
         if (!p) {
-            const bool cached = bool(d.census);
-            const uint64_t est = cached ? census_bytes(d) : estimate_bytes(d, q->kind, 0);
-            if (est > budget_of(s)) {
+            // a copy kept from a direct call is adopted with its real size;
+            // its optional parts as for clique executions below
+            bool kept = bool(d.census);
+            const uint64_t base = kept ? census_bytes(d) - census_extra_bytes(d) : estimate_bytes(d, q->kind, 0);
+            if (base > budget_of(s)) {
                 finish(s, q, KZ_ERR_BUDGET);
                 return 1;
             }
-            if (!make_room(s, est)) return no_room();
-            p = reserve(s, q->g, q->kind, 0, est);
-            // a copy kept from a direct call is adopted with its real size
-            if (cached) p->preparing = false;
+            if (!make_room(s, base)) return no_room();
+            const uint64_t left = budget_of(s) - s->in_use - base;
+            uint64_t extra = kept ? census_extra_bytes(d) : std::min(census_extra_estimate(d), left);
+            if (extra > left || (!kept && !has_room(s, base + extra))) extra = 0;
+            if (kept && extra != census_extra_bytes(d)) {
+                d.census.reset();
+                kept = false;
+            }
+            p = reserve(s, q->g, q->kind, 0, base + extra);
+            p->extra_limit = extra;
+            if (kept) p->preparing = false;
         } else {
             p->busy++;
         }
@@ -496,7 +506,7 @@ int admit(kz_server_s* s, SQuery* q, int* free_slot) {
             kept = nullptr;
         }
         p = reserve(s, q->g, q->kind, q->k, base + core);
-        p->core_limit = core;
+        p->extra_limit = core;
         if (!kept) {
             aux_submit(s->prep, AuxJob{kJobPrepare, q, p, 0, 0});
             return 0;

@@ -193,3 +193,55 @@ def test_a_core_bitmap_evicts_no_prepared_execution(kzdev):
     assert now[1]["execution"] and now[1]["core"] == 0, now
     da.release()
     db.release()
+
+
+def test_a_census_whose_optional_parts_do_not_fit(kzdev, monkeypatch):
+    """The census copy's core bitmap and range histograms are left out where
+    the budget has no room for them, in a copy kept from a direct call and in
+    one that the server builds; the copy then stays with the server."""
+    kz = kzdev
+    monkeypatch.setenv("KZ_C4_RANGE_BOUND", "4096")  # histograms at this size
+    monkeypatch.setenv("KZ_C4_SCRATCH_KEYS", "9000")  # a scratch below the server's estimate
+    g = kz.gen_chung_lu(300000, 1500000, 2.2, 5000, 21)
+    want = oracle.motif_census(g.rowptr, g.col)
+    dg = g.to_device()
+    assert dg.motif_census() == want
+    full = dg.census_kept_bytes()
+    dg.release()
+    assert full["extra"] > 1 << 20, full
+    cases = [  # budget, counted directly before, optional bytes kept
+        (full["state"], True, full["extra"]),
+        (full["state"] - 1, True, 0),
+        (full["state"] - full["extra"], True, 0),
+        (0, False, full["extra"]),
+    ]
+    for budget, direct, extra in cases:
+        dg = g.to_device()
+        if direct:
+            assert dg.motif_census() == want
+        print(f"[case] server census, budget {budget}, kept {direct}, of {full}", flush=True)
+        with kz.Server(hbm_budget=budget, max_inflight=2) as srv:
+            for _ in range(2):
+                res = srv.poll(srv.submit(dg, "census", 0), wait=True)
+                assert res["status"] == 0 and res["counts"] == want, res
+                now = dg.census_kept_bytes()  # no query in flight
+                assert now["state"] - now["extra"] == full["state"] - full["extra"], (now, full)
+                assert now["extra"] == extra, (now, full)
+        dg.release()
+    # a budget for the server's own upper estimate alone: no optional part
+    n, m = g.num_vertices, g.num_entries
+    col = 4 * ((m + 3) // 4 * 4 + 4)
+    cus = kz.device_info()["compute_units"]
+    need = 8 * (n + 1) * 3 + 3 * col + 16 * n * cus + 8 * n + (1 << 20)
+    for budget, extra in ((need, False), (need - 1, None)):
+        dg = g.to_device()
+        print(f"[case] server census, budget {budget}", flush=True)
+        with kz.Server(hbm_budget=budget, max_inflight=2) as srv:
+            res = srv.poll(srv.submit(dg, "census", 0), wait=True)
+            if extra is None:
+                assert res["status"] == kz._ffi.KZ_ERR_BUDGET, res
+            else:
+                assert res["status"] == 0 and res["counts"] == want, res
+                now = dg.census_kept_bytes()
+                assert now["state"] and now["extra"] == 0, now
+        dg.release()
