@@ -287,6 +287,16 @@ typedef struct kz_paged_stats {
     uint64_t cached_vertices;  /* lists the cache holds                  */
 } kz_paged_stats;
 int kz_paged_create(const kz_csr* oriented, const kz_paged_cfg* cfg, kz_paged* out);
+/* The root batches that kz_paged_create cuts for list_bytes, on the host alone
+ * (to size list_bytes beforehand): batch i is the roots up to batch_end[i],
+ * with batch_refs[i] list references before deduplication; both arrays (may
+ * be null) hold num_vertices entries at most.  Roots are cut in pieces of
+ * about piece_entries list entries (0: as kz_paged_create) that no batch
+ * crosses, with 4 bytes of host memory per vertex and working thread, never
+ * more than the lists' own size and at least one vertex array.
+ * KZ_ERR_BUDGET: a root's own lists exceed list_bytes. */
+int kz_paged_plan(const kz_csr* oriented, uint64_t list_bytes, uint64_t piece_entries, uint32_t* batch_end,
+                  uint64_t* batch_refs, uint32_t* num_batches);
 /* Exact k-clique count (k = 3..5), as kz_count_cliques. */
 int kz_paged_count_cliques(kz_paged p, int k, uint64_t* count, kz_paged_stats* stats);
 int kz_paged_release(kz_paged p);

@@ -236,6 +236,8 @@ _SIGS = {
                                       C.POINTER(C.c_void_p)]),
     "kz_graph_download": (C.c_int, [C.c_void_p, C.POINTER(kz_csr)]),
     "kz_graph_orient": (C.c_int, [C.c_void_p, C.POINTER(C.c_void_p)]),
+    "kz_paged_plan": (C.c_int, [C.POINTER(kz_csr), C.c_uint64, C.c_uint64, C.POINTER(C.c_uint32),
+                                C.POINTER(C.c_uint64), C.POINTER(C.c_uint32)]),
     "kz_paged_create": (C.c_int, [C.POINTER(kz_csr), C.POINTER(kz_paged_cfg), C.POINTER(C.c_void_p)]),
     "kz_paged_count_cliques": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_uint64), C.POINTER(kz_paged_stats)]),
     "kz_paged_release": (C.c_int, [C.c_void_p]),

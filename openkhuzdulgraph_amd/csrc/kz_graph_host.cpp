@@ -25,6 +25,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "kz_internal.h"
@@ -169,11 +170,119 @@ static int clean_symmetric(uint64_t m, uint32_t n_hint, EdgeFn edge, kz_csr* out
     return KZ_OK;
 }
 
+// Batches of the paged form: consecutive roots whose distinct lists fit
+// list_bytes, greedy within pieces of the root range of about piece_entries
+// list entries each, cut in parallel; a batch does not cross a piece.  Each
+// working thread stamps the vertices its batch has counted (4 bytes a vertex,
+// freed on return): pieces are bounded so that all stamps together take no
+// more than the lists do, which the caller allocates once more afterwards.
+// The pieces, and so the batches, depend on the graph only.
+int paged_cut(const kz_csr& g, uint64_t list_bytes, uint64_t piece_entries, std::vector<uint32_t>* batch_end,
+              std::vector<uint64_t>* batch_refs) {
+    constexpr uint64_t kMaxPieces = 64;
+    const uint32_t n = g.num_vertices;
+    const uint64_t m = g.num_entries, cap = list_bytes / 4;
+    if (!n) return KZ_OK;
+    const uint64_t pieces = std::max<uint64_t>(
+        1, std::min({m / std::max<uint64_t>(1, piece_entries), m / n, kMaxPieces}));
+    struct Piece {
+        std::vector<uint32_t> end;
+        std::vector<uint64_t> refs;
+        uint64_t too_big = 0;  // entries of the first root that does not fit alone
+        uint32_t root = 0;
+        bool nomem = false;
+    };
+    std::vector<Piece> plan(pieces);
+    int threads = int(std::min<uint64_t>(pieces, uint64_t(omp_get_max_threads())));
+    uint32_t* stamps = static_cast<uint32_t*>(std::calloc(size_t(n) * size_t(threads), 4));
+    if (!stamps && threads > 1) stamps = static_cast<uint32_t*>(std::calloc(size_t(n) * size_t(threads = 1), 4));
+    if (!stamps) KZ_FAIL(KZ_ERR_NOMEM, "batch stamps of %u vertices", n);
+    std::vector<uint32_t> epochs(threads, 0);
+    auto degree = [&](uint32_t v) { return g.rowptr[v + 1] - g.rowptr[v]; };
+    auto start_of = [&](uint64_t i) {
+        return uint32_t(std::lower_bound(g.rowptr, g.rowptr + n, m / pieces * i) - g.rowptr);
+    };
+    auto cut = [&](Piece& P, uint32_t u0, uint32_t u1, uint32_t* stamp, uint32_t& epoch) {
+        uint64_t acc = 0, refs = 0;
+        ++epoch;
+        for (uint32_t u = u0; u < u1; ++u) {
+            const uint64_t b = g.rowptr[u], e = g.rowptr[u + 1];
+            // entries root u adds to the batch
+            auto added = [&]() {
+                uint64_t c = stamp[u] == epoch ? 0 : e - b;
+                for (uint64_t i = b; i < e; ++i)
+                    if (stamp[g.col[i]] != epoch) c += degree(g.col[i]);
+                return c;
+            };
+            uint64_t c = added();
+            if (acc + c > cap) {
+                if (refs) {
+                    P.end.push_back(u);
+                    P.refs.push_back(refs);
+                }
+                ++epoch;
+                acc = refs = 0;
+                c = added();
+                if (c > cap) {
+                    P.too_big = c;
+                    P.root = u;
+                    return;
+                }
+            }
+            stamp[u] = epoch;
+            for (uint64_t i = b; i < e; ++i) stamp[g.col[i]] = epoch;
+            acc += c;
+            refs += 1 + (e - b);
+        }
+        if (refs) {
+            P.end.push_back(u1);
+            P.refs.push_back(refs);
+        }
+    };
+#pragma omp parallel for schedule(dynamic, 1) num_threads(threads)
+    for (int64_t q = 0; q < int64_t(pieces); ++q) {
+        const int t = omp_get_thread_num();
+        // no exception leaves a parallel region
+        try {
+            cut(plan[q], q ? start_of(uint64_t(q)) : 0u, q + 1 < int64_t(pieces) ? start_of(uint64_t(q) + 1) : n,
+                stamps + size_t(t) * n, epochs[t]);
+        } catch (const std::bad_alloc&) {
+            plan[q].nomem = true;
+        }
+    }
+    std::free(stamps);
+    for (const Piece& P : plan) {
+        if (P.nomem) KZ_FAIL(KZ_ERR_NOMEM, "root batches");
+        if (P.too_big)
+            KZ_FAIL(KZ_ERR_BUDGET, "root %u needs %llu list entries, more than list_bytes holds (%llu)", P.root,
+                    (unsigned long long)P.too_big, (unsigned long long)cap);
+        batch_end->insert(batch_end->end(), P.end.begin(), P.end.end());
+        batch_refs->insert(batch_refs->end(), P.refs.begin(), P.refs.end());
+    }
+    return KZ_OK;
+}
+
 }  // namespace kz
 
 using namespace kz;
 
 extern "C" {
+
+int kz_paged_plan(const kz_csr* g, uint64_t list_bytes, uint64_t piece_entries, uint32_t* batch_end,
+                  uint64_t* batch_refs, uint32_t* num_batches) {
+    if (!g || !g->rowptr || (g->num_entries && !g->col) || !num_batches) KZ_FAIL(KZ_ERR_INVALID, "null argument");
+    try {
+        std::vector<uint32_t> end;
+        std::vector<uint64_t> refs;
+        if (int e = paged_cut(*g, list_bytes, piece_entries ? piece_entries : kPagedPieceEntries, &end, &refs)) return e;
+        if (batch_end) std::copy(end.begin(), end.end(), batch_end);
+        if (batch_refs) std::copy(refs.begin(), refs.end(), batch_refs);
+        *num_batches = uint32_t(end.size());
+        return KZ_OK;
+    } catch (const std::bad_alloc&) {
+        KZ_FAIL(KZ_ERR_NOMEM, "root batches");
+    }
+}
 
 const char* kz_last_error(void) { return kz::get_error(); }
 

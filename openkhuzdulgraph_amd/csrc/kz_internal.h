@@ -48,6 +48,12 @@ bool csr_alloc(kz_csr* g, uint32_t n, uint64_t entries, bool labels);
 // draw r32 picks the first i with cdf[i+1] > (r32 + 0.5) * cdf[n] / 2^32.
 int chung_lu_cdf(uint32_t n, uint64_t num_draws, double exponent, uint32_t max_weight, std::vector<double>* cdf);
 
+// The paged form's batches of consecutive roots (kz_paged_plan): ends and list
+// references before deduplication.
+constexpr uint64_t kPagedPieceEntries = 1u << 20;
+int paged_cut(const kz_csr& g, uint64_t list_bytes, uint64_t piece_entries, std::vector<uint32_t>* batch_end,
+              std::vector<uint64_t>* batch_refs);
+
 }  // namespace kz
 
 #define KZ_FAIL(code, ...)           \

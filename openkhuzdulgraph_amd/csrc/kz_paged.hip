@@ -160,9 +160,7 @@ struct kz_paged_s {
 
 using namespace kz;
 
-extern "C" {
-
-int kz_paged_create(const kz_csr* g, const kz_paged_cfg* cfg, kz_paged* out) {
+static int paged_create(const kz_csr* g, const kz_paged_cfg* cfg, kz_paged* out) {
     if (!g || !cfg || !out || !g->rowptr || (g->num_entries && !g->col)) KZ_FAIL(KZ_ERR_INVALID, "null argument");
     if (!g->oriented) KZ_FAIL(KZ_ERR_INVALID, "the paged form takes a degree-oriented graph (kz_orient_by_degree)");
     if (int e = ensure_ready()) return e;
@@ -187,72 +185,8 @@ int kz_paged_create(const kz_csr* g, const kz_paged_cfg* cfg, kz_paged* out) {
         for (uint64_t i = g->rowptr[v]; i < g->rowptr[v + 1]; ++i)
             __atomic_fetch_add(&indeg[g->col[i]], 1u, __ATOMIC_RELAXED);
     }
-    // batches of consecutive roots whose distinct lists fit: greedy, in
-    // pieces of the root range with a batch stamp per vertex each (graphs of
-    // more than kPlanEdges entries a piece are cut in parallel; a batch does
-    // not cross a piece)
     const uint64_t cap = cfg->list_bytes / 4;
-    constexpr uint64_t kPlanEdges = 16u << 20;
-    const uint32_t pieces =
-        uint32_t(std::max<uint64_t>(1, std::min<uint64_t>(uint64_t(omp_get_max_threads()), m / kPlanEdges)));
-    struct Piece {
-        std::vector<uint32_t> end;
-        std::vector<uint64_t> refs;
-        uint64_t too_big = 0;  // entries of the first root that does not fit alone
-        uint32_t root = 0;
-    };
-    std::vector<Piece> plan(pieces);
-#pragma omp parallel for schedule(static, 1)
-    for (int64_t q = 0; q < int64_t(pieces); ++q) {
-        // pieces of about equal entries
-        auto start_of = [&](uint64_t i) {
-            return uint32_t(std::lower_bound(g->rowptr, g->rowptr + n, m / pieces * i) - g->rowptr);
-        };
-        const uint32_t u0 = q ? start_of(uint64_t(q)) : 0u, u1 = q + 1 < int64_t(pieces) ? start_of(uint64_t(q) + 1) : n;
-        Piece& P = plan[q];
-        std::vector<uint32_t> stamp(n, 0);
-        uint32_t epoch = 1;
-        uint64_t acc = 0, refs = 0;
-        for (uint32_t u = u0; u < u1; ++u) {
-            // entries root u adds to the batch
-            auto added = [&]() {
-                uint64_t c = stamp[u] == epoch ? 0 : p->h_deg[u];
-                for (uint64_t i = g->rowptr[u]; i < g->rowptr[u + 1]; ++i)
-                    if (stamp[g->col[i]] != epoch) c += p->h_deg[g->col[i]];
-                return c;
-            };
-            uint64_t c = added();
-            if (acc + c > cap) {
-                if (u > u0 && refs) {
-                    P.end.push_back(u);
-                    P.refs.push_back(refs);
-                }
-                ++epoch;
-                acc = refs = 0;
-                c = added();
-                if (c > cap) {
-                    P.too_big = c;
-                    P.root = u;
-                    break;
-                }
-            }
-            stamp[u] = epoch;
-            for (uint64_t i = g->rowptr[u]; i < g->rowptr[u + 1]; ++i) stamp[g->col[i]] = epoch;
-            acc += c;
-            refs += 1 + p->h_deg[u];
-        }
-        if (refs) {
-            P.end.push_back(u1);
-            P.refs.push_back(refs);
-        }
-    }
-    for (const Piece& P : plan) {
-        if (P.too_big)
-            KZ_FAIL(KZ_ERR_BUDGET, "root %u needs %llu list entries, more than list_bytes holds (%llu)", P.root,
-                    (unsigned long long)P.too_big, (unsigned long long)cap);
-        p->batch_end.insert(p->batch_end.end(), P.end.begin(), P.end.end());
-        p->batch_refs.insert(p->batch_refs.end(), P.refs.begin(), P.refs.end());
-    }
+    if (int e = paged_cut(*g, cfg->list_bytes, kPagedPieceEntries, &p->batch_end, &p->batch_refs)) return e;
     // cache: total degree >= threshold, largest first, while it fits
     std::vector<uint32_t> cand;
     for (uint32_t v = 0; v < n; ++v)
@@ -328,6 +262,16 @@ int kz_paged_create(const kz_csr* g, const kz_paged_cfg* cfg, kz_paged* out) {
     *out = p;
     p = nullptr;  // handed over
     return KZ_OK;
+}
+
+extern "C" {
+
+int kz_paged_create(const kz_csr* g, const kz_paged_cfg* cfg, kz_paged* out) {
+    try {
+        return paged_create(g, cfg, out);
+    } catch (const std::bad_alloc&) {
+        KZ_FAIL(KZ_ERR_NOMEM, "paged graph host arrays");
+    }
 }
 
 int kz_paged_count_cliques(kz_paged p, int k, uint64_t* count, kz_paged_stats* stats) {

@@ -179,3 +179,83 @@ def test_golden_fixture_digests():
         assert f"{g.digest():016x}" == e["digest"], name
         assert g.num_vertices == e["num_vertices"] and g.num_entries == e["num_entries"]
         g.check()
+
+
+def _paged_plan(raw, list_bytes, piece_entries):
+    n = raw.num_vertices
+    end, refs, nb = np.zeros(max(1, n), np.uint32), np.zeros(max(1, n), np.uint64), C.c_uint32()
+    rc = _ffi.lib().kz_paged_plan(C.byref(raw), list_bytes, piece_entries, end.ctypes.data_as(C.POINTER(C.c_uint32)),
+                                  refs.ctypes.data_as(C.POINTER(C.c_uint64)), C.byref(nb))
+    return rc, end[:nb.value].tolist(), refs[:nb.value].tolist()
+
+
+def _paged_plan_want(g, list_bytes, piece_entries):
+    """Greedy batches of distinct lists within pieces of the root range."""
+    n, m, cap = g.num_vertices, g.num_entries, list_bytes // 4
+    rp, col = g.rowptr.astype(np.int64), g.col
+    pieces = max(1, min(m // piece_entries, m // n, 64))
+    starts = [0] + [int(np.searchsorted(rp[:-1], m // pieces * i)) for i in range(1, pieces)] + [n]
+    end, refs = [], []
+    for u0, u1 in zip(starts, starts[1:]):
+        seen, acc, r = set(), 0, 0
+        for u in range(u0, u1):
+            own = {u, *col[rp[u]:rp[u + 1]].tolist()}
+            c = sum(int(rp[v + 1] - rp[v]) for v in own - seen)
+            if acc + c > cap:
+                if r:
+                    end.append(u), refs.append(r)
+                seen, acc, r = set(), 0, 0
+                c = sum(int(rp[v + 1] - rp[v]) for v in own)
+                if c > cap:
+                    return None
+            seen |= own
+            acc += c
+            r += 1 + int(rp[u + 1] - rp[u])
+        if r:
+            end.append(u1), refs.append(r)
+    return end, refs
+
+
+@pytest.mark.parametrize("piece", [1 << 40, 5000, 1000, 100])
+def test_paged_batches_are_the_greedy_cut_of_each_piece(piece):
+    g = kz.gen_rmat(11, 12, seed=5).oriented()
+    for list_bytes in (4 * g.num_entries, g.num_entries, g.num_entries // 3):
+        want = _paged_plan_want(g, list_bytes, piece)
+        rc, end, refs = _paged_plan(g._raw, list_bytes, piece)
+        if want is None:
+            assert rc == _ffi.KZ_ERR_BUDGET
+            continue
+        assert rc == 0 and (end, refs) == want
+        assert end[-1] == g.num_vertices and sum(refs) == g.num_vertices + g.num_entries
+    # a root that does not fit alone, in whichever piece it is
+    rc, _, _ = _paged_plan(g._raw, 4 * g.max_degree - 4, piece)
+    assert rc == _ffi.KZ_ERR_BUDGET
+    empty = _ffi.kz_csr()
+    empty.rowptr = (C.c_uint64 * 1)(0)
+    assert _paged_plan(empty, 64, piece) == (0, [], [])
+
+
+def test_paged_batches_do_not_depend_on_the_thread_count():
+    prog = ("import ctypes as C, openkhuzdulgraph_amd as kz\n"
+            "from tests.test_graph_host import _paged_plan\n"
+            "g = kz.gen_rmat(12, 16, seed=2).oriented()\n"
+            "print(_paged_plan(g._raw, g.num_entries, 3000))\n")
+    outs = {subprocess.run([sys.executable, "-c", prog], env=dict(os.environ, OMP_NUM_THREADS=t), check=True,
+                           capture_output=True, text=True, cwd=GOLDEN.parent.parent).stdout for t in ("1", "3", "8")}
+    assert len(outs) == 1 and len(outs.pop()) > 100
+
+
+def test_paged_batches_report_missing_host_memory():
+    """No exception or abort where the vertex stamps cannot be allocated."""
+    prog = ("import ctypes as C, resource\n"
+            "from openkhuzdulgraph_amd import _ffi\n"
+            "L = _ffi.lib()\n"
+            "n = 60_000_000\n"
+            "raw = _ffi.kz_csr()\n"
+            "raw.num_vertices, raw.rowptr = n, (C.c_uint64 * (n + 1))()\n"
+            "used = int(open('/proc/self/statm').read().split()[0]) * resource.getpagesize()\n"
+            "resource.setrlimit(resource.RLIMIT_AS, (used + (64 << 20),) * 2)\n"
+            "nb = C.c_uint32()\n"
+            "print(L.kz_paged_plan(C.byref(raw), 1 << 20, 0, None, None, C.byref(nb)))\n")
+    out = subprocess.run([sys.executable, "-c", prog], capture_output=True, text=True, cwd=GOLDEN.parent.parent)
+    assert out.returncode == 0 and out.stdout.strip() == str(_ffi.KZ_ERR_NOMEM), out.stderr
