@@ -49,7 +49,9 @@ struct DeviceGraph {
     uint64_t nnz = 0;
     uint32_t max_degree = 0;
     int oriented = 0;
-    int symmetric = 0;  // every edge both ways: 1 yes, 2 no, 0 not checked yet (kz_plan3.hip)
+    // no self-loops, and every edge upwards (oriented) or both ways: 1 yes,
+    // 2 no, 0 not checked yet (kz_plan3.hip; a resident graph does not change)
+    int plan3 = 0;
     uint64_t* rowptr = nullptr;
     uint32_t* col = nullptr;
     uint32_t* deg = nullptr;

@@ -123,7 +123,8 @@ void add_members(Weights& w, uint32_t pred, int code, bool oriented, uint64_t ti
 int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats* st, bool* taken) {
     *taken = false;
     const char* env = std::getenv("KZ_PLAN_FLAT");  // =0: the general path (for comparisons)
-    if (p.pattern_size != 3 || (env && env[0] == '0') || g.n == 0 || plan_validate(p) != KZ_OK) return KZ_OK;
+    if (p.pattern_size != 3 || (env && env[0] == '0') || g.n == 0 || g.plan3 == 2 || plan_validate(p) != KZ_OK)
+        return KZ_OK;
     auto nbr = [](const kz_set_ref& r) { return r.kind == KZ_SET_NBR; };
     Weights w[KZ_MAX_AGGREGATORS];
     // size 1: order code 0
@@ -179,6 +180,10 @@ int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats
             }
         }
     }
+    // (the largest forward degree of an oriented graph is its own; a symmetric
+    // graph's is known once its forward copy is built)
+    const uint32_t fwd_max = g.oriented ? g.max_degree : g.fwd_ready ? g.fwd_max : 0u;
+    if (members && fwd_max > kMaxBitmapDegree) return KZ_OK;
     hipStream_t s = rt().stream;
     DeviceWords dev;
     if (hipMalloc(&dev.p, 8 * (kSums + 1)) != hipSuccess) {
@@ -195,7 +200,7 @@ int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats
         KZ_HIP(hipEventRecord(e0, s));
         KZ_HIP(hipMemcpyAsync(dev.p, h, sizeof(h), hipMemcpyHostToDevice, s));
         hipLaunchKernelGGL(split_sums_kernel, dim3(grid), dim3(256), 0, s, g.rowptr, g.col, g.n, g.oriented, dev.p);
-        if (!g.oriented && !g.symmetric)
+        if (!g.oriented && !g.plan3)
             hipLaunchKernelGGL(reverse_check_kernel, dim3(uint32_t(rt().num_cus) * 8), dim3(256), 0, s, g.rowptr, g.col,
                                g.n, dev.p + kSums);
         KZ_HIP(hipGetLastError());
@@ -209,8 +214,8 @@ int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (e) return e;
-    if (!g.oriented && !g.symmetric) g.symmetric = h[kSums] == 0 && h[kSumS] == h[kSumF] ? 1 : 2;
-    if (h[kBad] || (!g.oriented && g.symmetric != 1)) return KZ_OK;
+    if (!g.plan3) g.plan3 = !h[kBad] && !h[kSums] && (g.oriented || h[kSumS] == h[kSumF]) ? 1 : 2;
+    if (g.plan3 == 2) return KZ_OK;
     uint64_t T = 0;
     double t_ms = 0;
     if (members) {

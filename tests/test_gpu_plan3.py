@@ -89,18 +89,57 @@ GRAPHS = {
 }
 
 
+QUALIFY = {"rmat_sym", "rmat_oriented", "chunglu_sym", "star", "complete"}  # no self-loop, upwards or both ways
+
+
+def _closed(p, oriented):
+    """Whether plan p has the closed form: the operations and counts of the
+    order codes that its scatters reach, restated from the plan alone."""
+    scatters = [p.lists[0].outs[o].pred for o in range(p.lists[0].num_outs)
+                if p.lists[0].outs[o].kind == _ffi.KZ_OUT_SCATTER]
+    reached = [c for c, bit in ((1, 0), (2, 2)) if any((s >> bit) & 1 for s in scatters)]
+    for code in reached:
+        if oriented and code == 1:
+            continue
+        lst = p.lists[p.type_table[2][code]]
+        ops = [lst.ops[j] for j in range(lst.num_ops)]
+        if any(r.kind != _ffi.KZ_SET_NBR for op in ops for r in (op.lhs, op.rhs)):
+            return False
+        for o in range(lst.num_outs):
+            src = lst.outs[o].src
+            if src.kind == _ffi.KZ_SET_NBR:
+                whole = src.a
+            else:
+                op = ops[src.b]
+                alone = op.lhs.a == op.rhs.a if op.op == _ffi.KZ_OP_INTERSECT else op.lhs.a != op.rhs.a
+                whole = op.lhs.a if alone else None
+            if oriented and whole == 1:
+                return False
+    return True
+
+
+def _took_closed_form(stats):
+    return stats["peak_bytes"] == 8 * 7 and stats["launches"] in (1, 2) and stats["chunks"] == 1
+
+
 @pytest.mark.parametrize("name", sorted(GRAPHS))
 def test_size3_plans_equal_the_interpreter_and_the_executor(kzdev, monkeypatch, name):
     kz = kzdev
     g = GRAPHS[name](kz)
     dg = g.to_device()
     rng = np.random.default_rng(len(name))
+    taken = 0
     for i in range(30):
         p = _plan(rng, outside=i % 5 == 4)
         print(f"[case] plan3 {name} {i}", flush=True)
         want = oracle.run_plan(p, g.rowptr, g.col)
         assert dg.count_plan(p) == want, (name, i)
+        closed = name in QUALIFY and _closed(p, g.oriented_flag)
+        assert _took_closed_form(dg.last_stats) == closed, (name, i, dg.last_stats)
+        taken += closed
         monkeypatch.setenv("KZ_PLAN_FLAT", "0")
         assert dg.count_plan(p) == want, (name, i)
+        assert not _took_closed_form(dg.last_stats)
         monkeypatch.delenv("KZ_PLAN_FLAT")
+    assert taken >= 5 if name in QUALIFY else taken == 0
     dg.release()
