@@ -262,16 +262,18 @@ constexpr uint32_t kC4BucketMul = 0x85EBCA6Bu;  // bucket hash (the tables use 2
 constexpr uint32_t kC4DirectBound = kC4HeavySlots / 2;  // heavy roots counted in one unbucketed pass
 constexpr uint32_t kC4MaxProbe = 64;            // bucket table probe limit
 constexpr uint32_t kAllBuckets = 0xFFFFFFFFu;
-// Direct counting of the heavy roots: 16-bit counters of kC4Range consecutive
-// ids fill the table's LDS, one atomic add per endpoint instead of a hash
-// insert.  Counts stay below 2^16: c(w) <= d(w), and larger degrees use the
-// hash.
-constexpr uint32_t kC4RangeBits = 16, kC4Range = 1u << kC4RangeBits;
-constexpr uint32_t kC4DenseRanges = 4;         // graphs of at most 4 ranges: one wedge stream per range, no scratch
+// Direct counting of the heavy roots: the 32-bit counters of kC4Range
+// consecutive ids fill the table's LDS, one atomic add per endpoint instead of
+// a hash insert.
+constexpr uint32_t kC4RangeBits = 15, kC4Range = 1u << kC4RangeBits;
+// Graphs of at most kC4DenseRanges ranges: one wedge stream per range, no
+// scratch (a census of 99 K vertices, 4 ranges, takes 4.15 ms bucketed and 4.25
+// ms in four streams, 60 K in two streams 2.37 against 2.75 bucketed).
+constexpr uint32_t kC4DenseRanges = 2;
 // Larger graphs: roots above this bound are bucketed by range, the others by
 // hash (a range costs its barriers and load latency however few endpoints it
-// gets; 4.84 M vertices, 74 ranges, heavy kernel by bound 32 / 64 / 128 / 256 /
-// 600 K: 24.9 / 25.1 / 25.8 / 27.0 / 29.3 ms).
+// gets; 4.84 M vertices, 148 ranges, a census by bound 16 / 32 / 64 / 128 / 256
+// K: 55.1 / 53.2 / 52.2 / 52.3 / 53.1 ms).
 constexpr uint64_t kC4RangeBound = 64u << 10;
 constexpr uint64_t kC4HistBytes = 256u << 20;   // most memory of their range histograms
 
@@ -617,10 +619,10 @@ __device__ void block_exclusive_scan(uint32_t* a, uint32_t P, uint32_t* wave_tot
 // stream of the wedges per range, no buckets.  In larger graphs the roots
 // above kC4RangeBound are bucketed by range (their sizes per range are part
 // of the prepared state) and each bucket is counted by adding its endpoints
-// and then taking each counter once.  Few buckets (74 for 4.84 M vertices,
-// not 4096) keep the buckets' tail lines in L2, so the scratch is written in
-// whole lines: 39.8 -> 11.5 GB a launch, and no hash inserts, table clears
-// or barriers per 4096 endpoints: 58.9 -> 25.1 ms.  The other roots:
+// and then taking each counter once.  Few buckets (148 for 4.84 M vertices,
+// not 4096) keep the buckets' tail lines in L2, so the scratch is written
+// mostly in whole lines: 39.8 -> 13.2 GB a launch, and no hash inserts, table
+// clears or barriers per 4096 endpoints: 58.9 -> 27.2 ms.  The other roots:
 //   0. b(u) <= kC4DirectBound: one pass counts every endpoint in the LDS
 //      table (at most half full);
 //   1. endpoints are bucketed by a hash into P ~ b(u) / kC4BucketKeys
@@ -645,8 +647,8 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                                                                    const uint32_t* __restrict__ hist, uint32_t nhist,
                                                                    uint32_t nranges,
                                                                    unsigned long long* __restrict__ sums) {
-    __shared__ uint32_t sTab[2 * kC4HeavySlots];  // hash keys and counts, or kC4Range 16-bit counters
-    static_assert(2 * kC4HeavySlots * 2 == kC4Range, "the counters fill the table");
+    __shared__ uint32_t sTab[2 * kC4HeavySlots];  // hash keys and counts, or kC4Range counters
+    static_assert(2 * kC4HeavySlots == kC4Range, "the counters fill the table");
     uint32_t* sKey = sTab;
     uint32_t* sCnt = sTab + kC4HeavySlots;
     __shared__ uint32_t sOff[kC4MaxBuckets + 1];
@@ -664,7 +666,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
         sKey[i] = dense_ranges ? 0u : kEmpty;
         sCnt[i] = 0;
     }
-    auto count_direct = [&](uint32_t w) { atomicAdd(&sTab[(w & (kC4Range - 1)) >> 1], 1u << (16 * (w & 1u))); };
+    auto count_direct = [&](uint32_t w) { atomicAdd(&sTab[w & (kC4Range - 1)], 1u); };
     if (threadIdx.x == 0) sOver[0] = sOver[1] = 0;
     uint32_t flip = 0;
     while (true) {
@@ -688,11 +690,10 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                     });
                 __syncthreads();
                 const uint32_t ids = min(u - (r << kC4RangeBits), kC4Range);
-                for (uint32_t i = threadIdx.x; 2 * i < ids; i += blockDim.x) {
-                    const uint32_t x = sTab[i];
-                    if (x) {
-                        const uint64_t c0 = x & 0xFFFFu, c1 = x >> 16;
-                        acc += c0 * (c0 - 1) / 2 + c1 * (c1 - 1) / 2;
+                for (uint32_t i = threadIdx.x; i < ids; i += blockDim.x) {
+                    const uint64_t c = sTab[i];
+                    if (c) {
+                        acc += c * (c - 1) / 2;
                         sTab[i] = 0;
                     }
                 }
@@ -856,9 +857,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
 #pragma unroll
                 for (int c = 0; c < kU; ++c)
                     if (kw[c] != kEmpty) {
-                        const uint32_t sh = 16 * (kw[c] & 1u);
-                        const uint32_t old = atomicAnd(&sTab[(kw[c] & (kC4Range - 1)) >> 1], ~(0xFFFFu << sh));
-                        const uint64_t n = (old >> sh) & 0xFFFFu;
+                        const uint64_t n = atomicExch(&sTab[kw[c] & (kC4Range - 1)], 0u);
                         if (n > 1) acc += n * (n - 1) / 2;
                     }
             }
@@ -887,10 +886,9 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                         if (w >> kC4RangeBits == b0) count_direct(w);
                     });
                     __syncthreads();
-                    for (uint32_t i = threadIdx.x; 2 * i < kC4Range; i += blockDim.x) {
-                        const uint64_t c0 = sTab[i] & 0xFFFFu, c1 = sTab[i] >> 16;
-                        if (c0 > 1) acc += c0 * (c0 - 1) / 2;
-                        if (c1 > 1) acc += c1 * (c1 - 1) / 2;
+                    for (uint32_t i = threadIdx.x; i < kC4Range; i += blockDim.x) {
+                        const uint64_t c = sTab[i];
+                        if (c > 1) acc += c * (c - 1) / 2;
                         sTab[i] = 0;
                     }
                     __syncthreads();
@@ -1111,8 +1109,6 @@ static int prepare_c4(Ranked& R, uint32_t* ranged) {
     }
     // heavy roots: direct counters over the whole graph when it has few
     // ranges; otherwise the largest roots are bucketed by range
-    uint32_t maxdeg = 0;
-    if (n) KZ_HIP(hipMemcpy(&maxdeg, R.deg + (n - 1), 4, hipMemcpyDeviceToHost));  // ranked by degree
     R.c4_ranges = (n + kC4Range - 1) >> kC4RangeBits;
     // (any KZ_C4_* knob leaves direct counters to KZ_C4_RANGE_BOUND, which
     // buckets the roots above it by range in a graph of any size)
@@ -1122,7 +1118,7 @@ static int prepare_c4(Ranked& R, uint32_t* ranged) {
     const bool knobs = rb || std::getenv("KZ_C4_DIRECT_BOUND") || std::getenv("KZ_C4_SCRATCH_KEYS") ||
                        std::getenv("KZ_C4_BUCKET_SLOTS");
     *ranged = 0;
-    if (R.n_c4_heavy && maxdeg < (1u << 16) && (!knobs || rb)) {
+    if (R.n_c4_heavy && (!knobs || rb)) {
         if (R.c4_ranges <= kC4DenseRanges && !knobs) {
             R.c4_dense = R.c4_ranges;
         } else if (R.c4_ranges <= kC4MaxBuckets) {

@@ -87,8 +87,8 @@ def test_census_rejects_oriented_graph(kzdev):
 
 
 @pytest.mark.parametrize("n,knobs", [
-    (60000, {}), (66000, {}), (150000, {}),  # counters of every id: one range, two, three
-    (400000, {}),  # seven ranges: bucketed by range above the default bound
+    (25000, {}), (60000, {}),  # counters of every id: one range, two
+    (66000, {}), (150000, {}), (400000, {}),  # more ranges: bucketed by range above the default bound
     (400000, {"KZ_C4_RANGE_BOUND": "4096"}),
     (400000, {"KZ_C4_RANGE_BOUND": "4096", "KZ_C4_SCRATCH_KEYS": "9000"}),  # rounds of ranges
     (400000, {"KZ_C4_RANGE_BOUND": "4096", "KZ_C4_SCRATCH_KEYS": "300"}),  # ranges above the scratch
@@ -106,3 +106,19 @@ def test_census_direct_counters(kzdev, monkeypatch, n, knobs):
     again = dg.motif_census()
     dg.release()
     assert got == want and again == want
+
+
+def test_census_counts_above_16_bits(kzdev):
+    """Two vertices with 70,000 common neighbours: one counter reaches 70,000,
+    in a graph that is bucketed by range."""
+    kz = kzdev
+    k = 70000
+    leaves = np.arange(2, k + 2, dtype=np.uint32)
+    g = kz.from_edges(np.repeat(np.array([0, 1], np.uint32), k), np.concatenate([leaves, leaves]), k + 2)
+    print(f"[case] census K(2,{k})", flush=True)
+    dg = g.to_device()
+    got = dg.motif_census()
+    dg.release()
+    # induced: wedges (two leaves at a hub, the hubs at a leaf), no 3-path
+    # (hub - leaf - hub - leaf closes a 4-cycle), stars of three leaves
+    assert got == [k * (k - 1) + k, 0, 0, k * (k - 1) * (k - 2) // 3, k * (k - 1) // 2, 0, 0, 0]
