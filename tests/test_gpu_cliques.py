@@ -236,9 +236,11 @@ def test_wave_tasks_dealt_and_from_the_cursor(kzdev, n, m):
 
 @pytest.mark.parametrize("k", [3, 4, 5])
 def test_core_rows_at_the_edges_of_their_tiles(kzdev, k):
-    """Rows gathered from the core bitmap: roots of 2 .. 1100 candidates in
-    one graph (every shared-load width, 32-row tiles, 64-candidate words, row
-    lines and the hub path), wholly or partly inside the core."""
+    """Roots of 2 .. 1100 candidates in one graph (every shared-load width,
+    32-row tiles, 64-candidate words, row lines and the hub path): with a tail
+    of sparse ids below they are inside the core bitmap but for a few
+    candidates, without it the graph has too many candidate pairs for one and
+    streams all rows."""
     import numpy as np
 
     kz = kzdev
@@ -263,7 +265,61 @@ def test_core_rows_at_the_edges_of_their_tiles(kzdev, k):
         print(f"[case] core rows k={k} tail={extra}", flush=True)
         assert dg.count_cliques(k, "persistent") == want
         assert dg.count_cliques(k, "persistent") == want
+        assert (dg.clique_kept_bytes(k)["core"] > 0) == (extra > 0)
         dg.release()
+
+
+# (candidates below the core, candidates in it) of one root: every bucket, on
+# both sides of 32 rows, 64 candidates and the hub rows' chunks
+CORE_SPLITS = [
+    (0, 2), (1, 1), (2, 0), (1, 7), (8, 8), (31, 33), (32, 32), (33, 31), (63, 1), (1, 63), (64, 0),
+    (31, 40), (32, 64), (33, 95), (63, 2), (64, 64), (65, 63), (127, 1),
+    (64, 66), (65, 200), (128, 256), (129, 383), (300, 212), (511, 1),
+    (64, 449), (65, 600), (128, 703), (129, 704), (512, 512), (513, 511), (700, 324), (1000, 24),
+    (64, 1000), (65, 1036), (512, 700), (600, 600), (1100, 30), (1, 1100),
+]
+
+
+@pytest.mark.parametrize("k", [3, 4, 5])
+def test_roots_partly_inside_the_core(kzdev, k):
+    """Root lists split at given positions between streamed rows and rows from
+    the core bitmap: the lower ids of a list outside the core, the others in
+    it."""
+    import numpy as np
+    from math import isqrt
+
+    kz = kzdev
+    rng = np.random.default_rng(k)
+    top, roots = 2400, len(CORE_SPLITS)
+    a, b = np.triu_indices(top, 1)
+    keep = rng.random(len(a)) < 0.0245
+    # 80 ids, half of them at either end of the list ids, are all joined and
+    # come up often in the lists: cliques that hold ids of both kinds
+    keep |= ((a < 40) | (a >= top - 40)) & ((b < 40) | (b >= top - 40))
+    a, b = a[keep] + roots, b[keep] + roots
+    n, nnz = roots + top, len(a) + sum(map(sum, CORE_SPLITS))
+    size = isqrt(16 * nnz)  # the core's ids: bit rows of a quarter of the lists' bytes
+    below, inside = np.arange(roots, n - size), np.arange(n - size, n)
+    src, dst = [a], [b]
+
+    def some(joined, others, count):
+        few = min(count // 2, len(joined))
+        return [rng.choice(joined, few, replace=False), rng.choice(others, count - few, replace=False)]
+
+    for r, (x, y) in enumerate(CORE_SPLITS):
+        ids = np.concatenate(some(below[:40], below[40:], x) + some(inside[-40:], inside[:-40], y))
+        src.append(np.full(x + y, r)), dst.append(ids)
+    g = _forward_graph(kz, np.concatenate(src), np.concatenate(dst))
+    assert g.num_vertices == n and g.num_entries == nnz
+    want = oracle.run_app(APP[k], g.rowptr, g.col)[1][0]
+    dg = g.to_device()
+    print(f"[case] roots split by the core k={k} size={size} of {n}", flush=True)
+    for _ in range(2):
+        assert dg.count_cliques(k, "persistent") == want
+    q = 128  # bytes of the bitmap: row r takes ceil(r / 1024) lines, then the lines masked lanes read past it
+    lines = sum((r + 1023) // 1024 for r in range(size))
+    assert dg.clique_kept_bytes(k)["core"] == q * lines + (size // 8 + 256) // q * q
+    dg.release()
 
 
 def _forward_graph(kz, src, dst):
