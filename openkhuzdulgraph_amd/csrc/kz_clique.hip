@@ -365,12 +365,20 @@ __device__ __forceinline__ void count5_edges(const unsigned long long* rows, uin
 // 11 VALU instructions for both operands of 64 columns (int8 operands took 48
 // and bound the count: 92 % VALU busy in the 833-1024 group).  The two sides
 // use codes whose product is 1; the order of the columns is the same for
-// both, so it does not matter which code a column takes.  Products and sums
-// are integers: accumulators start at 2^23 and hold 2^23 + n exactly (n <= d
-// <= 8192), whose low 24 bits are n.  Lane l holds row (or column) l % 32 of
-// the tile and half l / 32 of the word; accumulator r of lane l is tile row
-// (r / 4) * 8 + (l / 32) * 4 + r % 4, column l % 32 (checked on the device
-// over 122,880 sums up to 8192).
+// both, so it does not matter which code a column takes.  Lane l holds row (or
+// column) l % 32 of the tile and half l / 32 of the word; accumulator r of lane
+// l is tile row (r / 4) * 8 + (l / 32) * 4 + r % 4, column l % 32.
+//
+// The sums are whole numbers and exact: every product is 0 or 1 (each code
+// times its partner is a power of two times its inverse), a sum of n <= d <=
+// kMaxBitmapDegree of them is far below 2^24, and f32 holds and adds whole
+// numbers up to 2^24 without rounding, in any order.  Accumulators of the
+// 4-clique count start at 2^23, so that their low 24 bits are the integer n
+// (the asserts below).  Checked against integer sums on the device: 122,880
+// random ones up to 8192, and counts whose sums reach 8,092 of 8,192
+// candidates (no difference, as int32 had none).
+static_assert(kMaxBitmapDegree < (1u << 23), "2^23 + n is a whole f32 with n in its low 24 bits");
+static_assert(16 * kMaxBitmapDegree < (1u << 24), "16 masked sums of a lane add up exactly in f32");
 typedef int kz_v8i __attribute__((ext_vector_type(8)));
 typedef float kz_v16f __attribute__((ext_vector_type(16)));
 
@@ -597,7 +605,7 @@ __device__ __forceinline__ void count5_row(const unsigned long long* rows, uint3
                 if (++kw < wend) load(kw);
                 p = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(A, B, p, 4, 4, 0, 0, 0, 0);
             }
-            // exact: at most 16 r <= 2^17 per tile and lane
+            // exact: whole numbers of at most 16 r <= 2^17 per tile and lane
             float t = 0.f;
 #pragma unroll
             for (int k = 0; k < 16; ++k) t = __builtin_fmaf(p[k], m[k], t);

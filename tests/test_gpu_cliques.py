@@ -354,3 +354,24 @@ def test_five_cliques_on_mfma_tiles(kzdev, d, p):
     print(f"[case] five cliques d={d} p={p}", flush=True)
     assert dg.count_cliques(5, "persistent") == want
     dg.release()
+
+
+@pytest.mark.parametrize("c,b", [(101, 8092), (3, 8190), (1025, 0), (513, 511), (129, 0), (65, 900)])
+def test_largest_sums_of_the_matrix_counts(kzdev, c, b):
+    """c vertices joined to each other and to b more, which are not joined:
+    common neighbour counts up to every candidate of a root, dense tiles, and
+    the largest root the bitmaps take (8,192 candidates)."""
+    import numpy as np
+    from math import comb
+
+    kz = kzdev
+    i, j = np.triu_indices(c, 1)
+    if b:
+        i = np.concatenate([i, np.repeat(np.arange(c), b)])
+        j = np.concatenate([j, np.tile(np.arange(c, c + b), c)])
+    dg = _forward_graph(kz, i, j).to_device()
+    for k in (3, 4, 5):
+        print(f"[case] joined cliques c={c} b={b} k={k}", flush=True)
+        assert dg.count_cliques(k, "persistent") == comb(c, k) + b * comb(c, k - 1)
+        assert dg.last_stats["launches"] == 1
+    dg.release()
