@@ -49,6 +49,24 @@ def test_paged_counts_equal_the_oracle(kzdev, cache):
         dg.release()
 
 
+def test_paged_counts_of_a_graph_cut_in_pieces(kzdev):
+    """More than one piece of roots: the counted batches are the cut's."""
+    import ctypes as C
+
+    from openkhuzdulgraph_amd import _ffi
+    kz = kzdev
+    g = kz.gen_rmat(18, 10, seed=3).oriented()
+    want = oracle.run_app(APPS[3], g.rowptr, g.col)[1][0]
+    print("[case] paged pieces", flush=True)
+    assert g.num_entries > 2 << 20  # two pieces
+    nb = C.c_uint32()
+    assert _ffi.lib().kz_paged_plan(C.byref(g._raw), g.num_entries, 0, None, None, C.byref(nb)) == 0
+    pg = kz.PagedGraph(g, list_bytes=g.num_entries, cache_bytes=0)
+    assert pg.count_cliques(3) == want
+    assert pg.last_stats["batches"] == nb.value
+    pg.release()
+
+
 def test_paged_refuses_a_budget_below_one_root(kzdev):
     kz = kzdev
     g = kz.gen_rmat(12, 16, seed=2).oriented()
