@@ -299,31 +299,62 @@ __global__ void c4_bound_kernel(const uint64_t* __restrict__ rowptr, const uint3
 
 __device__ __forceinline__ uint32_t shfl_u32(uint32_t v, uint32_t l) { return uint32_t(__shfl(int(v), int(l))); }
 
-// The wedges u - v - w (v = N(u)[k], k < pre; w in N(v), w < u) of one root,
-// streamed by one wave: groups of 64 neighbours v (k0, k0 + kstep, ...),
-// whose lists are concatenated as aligned 16-byte groups of 4 entries; each
-// lane walks its own contiguous range of ceil(T / 64) groups of the
-// concatenation (found once per 64 neighbours by a binary search of the list
-// offsets), kC4Unroll loads in flight, moving to the next list when it
-// reaches its offset.  (Single entries took four loads for a group and
-// fetched each line again from L2 while the wave's other lanes' lines pushed
-// it out of L1: 10.4 ms to stream 2.3 G entries, 3.4 ms with groups, 4 in
-// flight.)  The neighbours are in rank order, i.e. by degree, so
-// their lists have similar lengths.  f(w) runs on the lanes holding an
-// endpoint.  `wl` is the wave's LDS (kC4ListWords): 65 offsets (the last one
-// the total), 64 list starts and 64 ends (census lists hold fewer than 2^31
-// entries; the column array is padded to whole groups).
+// A wave's stream of the wedges u - v - w (v = N(u)[k], k < pre; w in N(v), w <
+// u) of one root takes groups of 64 neighbours v, whose lists are concatenated;
+// each lane walks its own contiguous range of a 64th of the concatenation,
+// found by a binary search of the list offsets, and moves to the next list when
+// it reaches its offset.  The neighbours are in rank order, i.e. by degree, so
+// their lists have similar lengths.
+//
+// c4_stage puts the lists (this lane's: entries [vb, ve), `units` steps of the
+// walk) into the wave's LDS wl -- 65 offsets, the last one the total, 64 starts
+// and, ENDS, 64 ends -- and sets this lane's steps [p, e) and the list lo that
+// holds p.  (Census lists hold fewer than 2^31 entries.)
 constexpr uint32_t kC4ListWords = 193;
-constexpr int kHeavyUnroll = 4;  // loads in flight: one 1024-thread workgroup per CU has the registers
 
-template <int kC4Unroll, class F>
+template <bool ENDS>
+__device__ __forceinline__ void c4_stage(uint32_t units, uint32_t vb, uint32_t ve, uint32_t* wl, uint32_t* p,
+                                         uint32_t* e, uint32_t* lo) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t incl = units;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t t = uint32_t(__shfl_up(int(incl), d));
+        if (lane >= uint32_t(d)) incl += t;
+    }
+    const uint32_t T = wave_lane(incl, 63u);
+    wave_lds_sync();
+    wl[lane] = incl - units;
+    wl[65 + lane] = vb;
+    if (ENDS) wl[129 + lane] = ve;
+    if (lane == 63) wl[64] = T;
+    wave_lds_sync();
+    const uint32_t q = (T + 63) / 64;
+    *p = min(lane * q, T);
+    *e = min(*p + q, T);
+    // the last list whose offset is <= p (non-empty)
+    *lo = 0;
+#pragma unroll
+    for (uint32_t step = 32; step; step >>= 1) {
+        const uint32_t t = *lo + step;
+        if (t < 64 && wl[t] <= *p) *lo = t;
+    }
+}
+
+// The wedge stream of neighbours k0 .. k0 + 63, k0 + kstep .., in aligned
+// 16-byte groups of 4 entries, four loads in flight (one 1024-thread workgroup
+// per CU has the registers).  Single entries took four loads for a group and
+// fetched each line again from L2 while the wave's other lanes' lines pushed it
+// out of L1: 10.4 ms to stream 2.3 G entries, 3.4 ms with groups.  f(w) runs on
+// the lanes holding an endpoint; `wl`: kC4ListWords.  The column array is padded
+// to whole groups.
+template <class F>
 __device__ __forceinline__ void c4_wave_wedges(const uint64_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
                                                uint64_t ub, uint32_t pre, uint32_t u, uint32_t k0, uint32_t kstep,
                                                uint32_t* wl, F&& f) {
     const uint32_t lane = threadIdx.x & 63;
-    uint32_t* soff = wl;
-    uint32_t* sstart = wl + 65;
-    uint32_t* send = wl + 129;
+    constexpr int kUnroll = 4;
+    const uint32_t *soff = wl, *sstart = wl + 65, *send = wl + 129;
     for (uint32_t k = k0; k < pre; k += kstep) {
         uint32_t vb = 0, ve = 0;
         if (k + lane < pre) {
@@ -331,39 +362,17 @@ __device__ __forceinline__ void c4_wave_wedges(const uint64_t* __restrict__ rowp
             vb = uint32_t(ldg(rowptr, v));
             ve = uint32_t(ldg(rowptr, v + 1));
         }
-        const uint32_t dv = ve > vb ? ((ve + 3) >> 2) - (vb >> 2) : 0u;  // groups
-        uint32_t incl = dv;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t t = uint32_t(__shfl_up(int(incl), d));
-            if (lane >= uint32_t(d)) incl += t;
-        }
-        const uint32_t T = wave_lane(incl, 63u);
-        wave_lds_sync();
-        soff[lane] = incl - dv;
-        sstart[lane] = vb;
-        send[lane] = ve;
-        if (lane == 63) soff[64] = T;
-        wave_lds_sync();
-        const uint32_t q = (T + 63) / 64;
-        uint32_t p = min(lane * q, T);
-        const uint32_t e = min(p + q, T);
-        // the list holding p: the last whose offset is <= p (non-empty)
-        uint32_t lo = 0;
-#pragma unroll
-        for (uint32_t step = 32; step; step >>= 1) {
-            const uint32_t t = lo + step;
-            if (t < 64 && soff[t] <= p) lo = t;
-        }
+        uint32_t p, e, lo;
+        c4_stage<true>(ve > vb ? ((ve + 3) >> 2) - (vb >> 2) : 0u, vb, ve, wl, &p, &e, &lo);
         uint32_t nxt = soff[lo + 1];
         uint32_t b = sstart[lo], z = send[lo];
         uint32_t adr = (b & ~3u) - 4 * soff[lo];  // col index of group p is adr + 4 p (mod 2^32)
         while (p < e) {
-            u32x4 ws[kC4Unroll];
-            uint32_t first[kC4Unroll], last[kC4Unroll];  // entries [first, last) of the group are the list's
-            const uint32_t cnt = min(uint32_t(kC4Unroll), e - p);
+            u32x4 ws[kUnroll];
+            uint32_t first[kUnroll], last[kUnroll];  // entries [first, last) of the group are the list's
+            const uint32_t cnt = min(uint32_t(kUnroll), e - p);
 #pragma unroll
-            for (int c = 0; c < kC4Unroll; ++c) {
+            for (int c = 0; c < kUnroll; ++c) {
                 first[c] = last[c] = 0;
                 ws[c] = u32x4{0, 0, 0, 0};
                 if (uint32_t(c) < cnt) {
@@ -384,7 +393,7 @@ __device__ __forceinline__ void c4_wave_wedges(const uint64_t* __restrict__ rowp
                 }
             }
 #pragma unroll
-            for (int c = 0; c < kC4Unroll; ++c)
+            for (int c = 0; c < kUnroll; ++c)
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                     if (uint32_t(t) >= first[c] && uint32_t(t) < last[c] && ws[c][t] < u) f(ws[c][t]);
@@ -392,20 +401,18 @@ __device__ __forceinline__ void c4_wave_wedges(const uint64_t* __restrict__ rowp
     }
 }
 
-// The same stream entry by entry, four loads in flight, for the roots counted
-// in a hash of a wave or a workgroup: their inserts, not the loads, bound
-// them, and the groups' entry masks cost more than they save (wave kernel
-// 4.48 against 4.65 ms, workgroup kernel 4.51 against 4.91; Erdos-Renyi, 0.56
-// M vertices of degree 40, all of whose roots are such, 16.2 against 16.9 ms a
-// census).  `wl`: 65 offsets and 64 list starts.
+// The same stream entry by entry, for the roots counted in a hash of a wave or
+// a workgroup: their inserts, not the loads, bound them, and the groups' entry
+// masks cost more than they save (wave kernel 4.48 against 4.65 ms, workgroup
+// kernel 4.51 against 4.91; Erdos-Renyi, 0.56 M vertices of degree 40, all of
+// whose roots are such, 16.2 against 16.9 ms a census).  `wl`: 129 words.
 template <class F>
 __device__ __forceinline__ void c4_wave_entries(const uint64_t* __restrict__ rowptr, const uint32_t* __restrict__ col,
                                                 uint64_t ub, uint32_t pre, uint32_t u, uint32_t k0, uint32_t kstep,
                                                 uint32_t* wl, F&& f) {
     const uint32_t lane = threadIdx.x & 63;
-    constexpr int kC4Unroll = 4;
-    uint32_t* soff = wl;
-    uint32_t* sstart = wl + 65;
+    constexpr int kUnroll = 4;
+    const uint32_t *soff = wl, *sstart = wl + 65;
     for (uint32_t k = k0; k < pre; k += kstep) {
         uint32_t vb = 0, dv = 0;
         if (k + lane < pre) {
@@ -414,35 +421,15 @@ __device__ __forceinline__ void c4_wave_entries(const uint64_t* __restrict__ row
             vb = uint32_t(b);
             dv = uint32_t(ldg(rowptr, v + 1) - b);
         }
-        uint32_t incl = dv;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t t = uint32_t(__shfl_up(int(incl), d));
-            if (lane >= uint32_t(d)) incl += t;
-        }
-        const uint32_t T = wave_lane(incl, 63);
-        wave_lds_sync();
-        soff[lane] = incl - dv;
-        sstart[lane] = vb;
-        if (lane == 63) soff[64] = T;
-        wave_lds_sync();
-        const uint32_t q = (T + 63) / 64;
-        uint32_t p = min(lane * q, T);
-        const uint32_t e = min(p + q, T);
-        // the list holding p: the last whose offset is <= p (non-empty)
-        uint32_t lo = 0;
-#pragma unroll
-        for (uint32_t step = 32; step; step >>= 1) {
-            const uint32_t t = lo + step;
-            if (t < 64 && soff[t] <= p) lo = t;
-        }
+        uint32_t p, e, lo;
+        c4_stage<false>(dv, vb, 0, wl, &p, &e, &lo);
         uint32_t nxt = soff[lo + 1];
         uint32_t adr = sstart[lo] - soff[lo];  // col index of position p is adr + p (mod 2^32)
         while (p < e) {
-            uint32_t ws[kC4Unroll];
-            const uint32_t cnt = min(uint32_t(kC4Unroll), e - p);
+            uint32_t ws[kUnroll];
+            const uint32_t cnt = min(uint32_t(kUnroll), e - p);
 #pragma unroll
-            for (int c = 0; c < kC4Unroll; ++c) {
+            for (int c = 0; c < kUnroll; ++c) {
                 ws[c] = 0xFFFFFFFFu;
                 if (uint32_t(c) < cnt) {
                     if (p == nxt) {
@@ -457,7 +444,7 @@ __device__ __forceinline__ void c4_wave_entries(const uint64_t* __restrict__ row
                 }
             }
 #pragma unroll
-            for (int c = 0; c < kC4Unroll; ++c)
+            for (int c = 0; c < kUnroll; ++c)
                 if (ws[c] < u) f(ws[c]);
         }
     }
@@ -683,9 +670,9 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
             // every id has a counter in at most kC4DenseRanges passes
             for (uint32_t r = 0; r << kC4RangeBits < u; ++r) {
                 if (dense_ranges == 1)
-                    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], count_direct);
+                    c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], count_direct);
                 else
-                    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                    c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                         if (w >> kC4RangeBits == r) count_direct(w);
                     });
                 __syncthreads();
@@ -765,7 +752,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                                 if (kw[c] != kEmpty && part_of(kw[c], parts) == part) add(kw[c]);
                         }
                     } else {
-                        c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                        c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                             if ((b == kAllBuckets || bucket_of(w) == b) && part_of(w, parts) == part) add(w);
                         });
                     }
@@ -806,7 +793,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
             for (uint32_t b = threadIdx.x; b < P; b += blockDim.x) sOff[b] = 0;
             if (threadIdx.x == 0) sB1 = 0;  // a bucket filled up
             __syncthreads();
-            c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+            c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                 const uint32_t b = bucket_of(w);
                 const uint32_t pos = atomicAdd(&sOff[b], 1u);
                 if (pos < cap) scratch[b * cap + pos] = w;
@@ -832,7 +819,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
         } else {
             for (uint32_t b = threadIdx.x; b <= P; b += blockDim.x) sOff[b] = 0;
             __syncthreads();
-            c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
+            c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
                            [&](uint32_t w) { atomicAdd(&sOff[bucket_of(w)], 1u); });
         }
         __syncthreads();
@@ -882,7 +869,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                 // one bucket above the scratch: count it from the wedge stream
                 const uint32_t k = sOff[b0 + 1] - base0;
                 if (ranged) {
-                    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+                    c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                         if (w >> kC4RangeBits == b0) count_direct(w);
                     });
                     __syncthreads();
@@ -898,7 +885,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_heavy_kernel(const uint64_
                 b0 += 1;
                 continue;
             }
-            c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
+            c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave], [&](uint32_t w) {
                 const uint32_t b = place_of(w);
                 if (b >= b0 && b < b1) scratch[atomicAdd(&sOff[b], 1u) - base0] = w;
             });
@@ -936,7 +923,7 @@ __global__ __launch_bounds__(kC4Block) void census_c4_hist_kernel(const uint64_t
     const uint32_t pre = lower_bound_global(col + ub, du, u);
     for (uint32_t i = threadIdx.x; i < nranges; i += blockDim.x) sHist[i] = 0;
     __syncthreads();
-    c4_wave_wedges<kHeavyUnroll>(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
+    c4_wave_wedges(rowptr, col, ub, pre, u, wave * 64, nw * 64, sList[wave],
                    [&](uint32_t w) { atomicAdd(&sHist[w >> kC4RangeBits], 1u); });
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < nranges; i += blockDim.x) hist[size_t(blockIdx.x) * nranges + i] = sHist[i];

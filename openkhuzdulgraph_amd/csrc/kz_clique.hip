@@ -741,12 +741,12 @@ __device__ __forceinline__ void core_rows_block(const uint32_t* core, uint32_t n
 
 // ----------------------------------------------------------- block tasks --
 // One task per workgroup, rows in LDS.  Dynamic LDS: [rows Dmax*W u64 (k >= 4;
-// TRI, 4-cliques only: packed, tri_words(Dmax) u64)]
+// TRI: packed, tri_words(Dmax) u64)]
 // [row descriptors Dmax u64][probe queues 64 uint2 per wave (QU)][hash keys
 // H u32][L Dmax u32][group prefix Dmax+1 u32][filter FW u32][hash vals H u16].
 // QU (queued probes, where the LDS leaves room for them without costing a
-// workgroup per CU): the stream's filter passes are probed 64 at a time.  Register budget: WPE
-// waves per SIMD.  The default, 6 (at most 80 VGPRs), is the occupancy the
+// workgroup per CU): the stream's filter passes are probed 64 at a time.
+// Register budget: WPE waves per SIMD.  The default, 6 (at most 80 VGPRs), is the occupancy the
 // LDS of the middle buckets allows; there the latency-bound count phase
 // loses more to fewer waves than the stream gains from more registers.
 // Buckets whose LDS leaves at most 4 waves per SIMD (4-cliques on the
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(WPE))) voi
                 else rows[word_base<TRI>(kk, d) + i] = w;
             });
         __syncthreads();
-                if (K == 4) count_rows_mfma4<TRI, (WPE <= 4 ? 2 : 1)>(rows, d, d, &sTile, acc);
+        if (K == 4) count_rows_mfma4<TRI, (WPE <= 4 ? 2 : 1)>(rows, d, d, &sTile, acc);
         else if (K == 5) {
             // (RMAT-22: up to 128 candidates the edge loop is the faster, 9.4
             // against 10.0 ms for the two buckets; above, MFMA tiles)
