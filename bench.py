@@ -10,9 +10,9 @@ form (one hipGraph launch of the degree-bucketed kernels) is the headline;
 the plain level-by-level form is timed beside it.  `value` is the persistent
 form's seconds per count; the count is checked against the committed
 oracle count of the same graph (tests/golden/config_counts.json, matched by
-CSR digest).  The roofline uses the bytes the kernels must stream,
-4 (m + sum over edges (u, v) of d+(v)), over the HIP-event time of the
-launch.  The CPU baseline is the oracle's restatement of the kautomine
+CSR digest).  The roofline divides the counted traffic of one launch
+(profiles/, used only where it is of this graph and of the present kernel
+sources) by the HIP-event time of the launch.  The CPU baseline is the oracle's restatement of the kautomine
 four_clique schedule on a bounded sample of roots, on this host's cores,
 with its time projected to the whole count by merge-model bytes.
 
@@ -40,8 +40,10 @@ Other workloads (each prints its own JSON line; the default is the one above):
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import tempfile
 import time
@@ -574,6 +576,28 @@ def host_cpu() -> dict:
     return {"nproc": usable, "cpu_model": model}
 
 
+def kernel_sources_sha() -> str:
+    """Digest of the persistent clique kernels' sources without comments and
+    white space."""
+    h = hashlib.sha256()
+    for name in ("kz_clique.hip", "kz_core.h", "kz_stream.h", "kz_kernels.h"):
+        text = re.sub(r"//.*", "", (ROOT / "openkhuzdulgraph_amd" / "csrc" / name).read_text())
+        h.update(re.sub(r"\s+", "", text).encode())
+    return h.hexdigest()[:16]
+
+
+def committed_traffic(args, digest: str) -> dict:
+    """Counter profile of one persistent launch (profiles/), or {} where none
+    is of this graph and of these kernel sources."""
+    f = ROOT / "profiles" / f"rmat{args.scale}_k{args.k}_persistent_traffic.json"
+    tr = json.loads(f.read_text()) if f.exists() else {}
+    if tr.get("csr_digest") == digest and tr.get("kernel_sources") == kernel_sources_sha():
+        return tr
+    if tr:
+        log(f"{f.name}: not of this graph or of these kernel sources, no traffic reported")
+    return {}
+
+
 def bench_clique(kz, args) -> int:
     from openkhuzdulgraph_amd import workloads as wl
 
@@ -646,19 +670,18 @@ def bench_clique(kz, args) -> int:
     # (column ids, 4 B each): a size of the problem, not what the kernels
     # read, which take most rows as bits of the core bitmap
     b_vc = 4 * (work["m"] + work["sum_dv"])
-    # the roofline uses the measured traffic of one launch where its profile
-    # is committed, else the graph read once
-    traffic_file = ROOT / "profiles" / f"rmat{args.scale}_k{args.k}_persistent_traffic.json"
-    tr = json.loads(traffic_file.read_text()) if traffic_file.exists() else {}
-    b_run = tr.get("bytes_per_launch") or 4 * work["m"] + 8 * (dg.num_vertices + 1)
-    achieved = b_run / (dev_avg_ms / 1e3) / 1e9
+    # the roofline divides the measured traffic of one launch by this run's
+    # time: only where the committed profile is of this graph and of the
+    # kernels' present sources
+    tr = committed_traffic(args, digest)
+    b_run = tr.get("bytes_per_launch")
+    achieved = b_run / (dev_avg_ms / 1e3) / 1e9 if b_run else None
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": achieved / HBM_PEAK_GBS, "traffic": tr.get("bytes_per_launch"),
+                "frac": achieved / HBM_PEAK_GBS if b_run else None, "traffic": b_run,
                 "kernel": "clique_block_kernel/clique_wave_kernel (persistent bucket graph, one hipGraph launch)",
-                "bytes_per_launch": b_run, "avg_launch_ms": dev_avg_ms}
-    if tr:
-        roofline["l2_hit_rate"] = tr.get("l2_hit_rate")
-        roofline["measured_copy_GBps"] = tr.get("copy_GBps")
+                "bytes_per_launch": b_run, "avg_launch_ms": dev_avg_ms,
+                "graph_read_once_GBps": (4 * work["m"] + 8 * (dg.num_vertices + 1)) / (dev_avg_ms / 1e3) / 1e9,
+                "l2_hit_rate": tr.get("l2_hit_rate"), "measured_copy_GBps": tr.get("copy_GBps")}
 
     cpu = None
     if not args.no_cpu:
