@@ -267,14 +267,17 @@ constexpr uint32_t kAllBuckets = 0xFFFFFFFFu;
 // a hash insert.
 constexpr uint32_t kC4RangeBits = 15, kC4Range = 1u << kC4RangeBits;
 // Graphs of at most kC4DenseRanges ranges: one wedge stream per range, no
-// scratch (a census of 99 K vertices, 4 ranges, takes 4.15 ms bucketed and 4.25
-// ms in four streams, 60 K in two streams 2.37 against 2.75 bucketed).
+// scratch.  A census in streams against bucketed: 60 K vertices, 2 ranges, 2.38
+// / 2.75 ms; 75 K, 3 ranges, 3.21 / 3.23; 90 K 4.52 / 4.41; 100 K, 4 ranges, 4.25
+// / 4.04.
 constexpr uint32_t kC4DenseRanges = 2;
-// Larger graphs: roots above this bound are bucketed by range, the others by
-// hash (a range costs its barriers and load latency however few endpoints it
-// gets; 4.84 M vertices, 148 ranges, a census by bound 16 / 32 / 64 / 128 / 256
-// K: 55.1 / 53.2 / 52.2 / 52.3 / 53.1 ms).
-constexpr uint64_t kC4RangeBound = 64u << 10;
+// Larger graphs: roots of more than this many endpoints per range of the graph
+// are bucketed by range, the others by hash (a range costs its barriers and
+// load latency however few endpoints it gets).  A census by the bound, which is
+// 4 K at least, at 4 K / 16 K / 64 K / 96 K: 250 K vertices, 8 ranges, 8.84 / 9.11
+// / 9.38 / 9.49 ms; 1.2 M, 37 ranges, 16.78 / 16.60 / 16.78 / 16.93; 4.84 M, 148
+// ranges, 65.2 / 55.2 / 52.0 / 51.8.
+constexpr uint64_t kC4RangeBoundPerRange = 512;
 constexpr uint64_t kC4HistBytes = 256u << 20;   // most memory of their range histograms
 
 // b(u) for every vertex (one wave per vertex).
@@ -604,7 +607,7 @@ __device__ void block_exclusive_scan(uint32_t* a, uint32_t P, uint32_t* wave_tot
 // Roots with b(u) > kC4BlockBound: one workgroup each.  In graphs of at most
 // kC4DenseRanges ranges of ids every endpoint has its own counter in LDS: one
 // stream of the wedges per range, no buckets.  In larger graphs the roots
-// above kC4RangeBound are bucketed by range (their sizes per range are part
+// above a bound are bucketed by range (their sizes per range are part
 // of the prepared state) and each bucket is counted by adding its endpoints
 // and then taking each counter once.  Few buckets (148 for 4.84 M vertices,
 // not 4096) keep the buckets' tail lines in L2, so the scratch is written
@@ -1099,7 +1102,7 @@ static int prepare_c4(Ranked& R, uint32_t* ranged) {
     R.c4_ranges = (n + kC4Range - 1) >> kC4RangeBits;
     // (any KZ_C4_* knob leaves direct counters to KZ_C4_RANGE_BOUND, which
     // buckets the roots above it by range in a graph of any size)
-    uint64_t range_bound = kC4RangeBound;
+    uint64_t range_bound = kC4RangeBoundPerRange * R.c4_ranges;
     const char* rb = std::getenv("KZ_C4_RANGE_BOUND");
     if (rb) range_bound = std::strtoull(rb, nullptr, 10);
     const bool knobs = rb || std::getenv("KZ_C4_DIRECT_BOUND") || std::getenv("KZ_C4_SCRATCH_KEYS") ||
