@@ -159,7 +159,9 @@ int kz_count_cliques(kz_graph g, int k, int method, uint64_t* count, kz_run_stat
     double dev_ms = 0;
     kz_run_stats st;
     std::memset(&st, 0, sizeof(st));
+    std::unique_lock<std::mutex> lk(d.exec_mu, std::defer_lock);
     if (method == KZ_METHOD_PERSISTENT) {
+        lk.lock();
         if (int e = ensure_forward(d)) return e;
         // a root whose forward list cannot be staged in LDS even after the
         // orientation (a clique core of more than kMaxBitmapDegree vertices)
@@ -173,6 +175,7 @@ int kz_count_cliques(kz_graph g, int k, int method, uint64_t* count, kz_run_stat
         st.launches = 1;
         st.tasks = j->ntasks;
     } else if (method == KZ_METHOD_PLAIN) {
+        if (lk.owns_lock()) lk.unlock();
         PlanDesc pd;
         plan_clique(k, &pd);
         uint64_t counts[KZ_MAX_AGGREGATORS] = {0};
@@ -191,6 +194,7 @@ int kz_count_cliques(kz_graph g, int k, int method, uint64_t* count, kz_run_stat
 
 int kz_clique_kept_bytes(kz_graph g, int k, uint64_t* out3) {
     if (!g || !out3 || k < 3 || k > 5) KZ_FAIL(KZ_ERR_INVALID, "bad argument");
+    std::lock_guard<std::mutex> lk(g->g.exec_mu);
     const CliqueJob* j = static_cast<const CliqueJob*>(g->g.clique_exec[k].get());
     out3[0] = g->g.fwd_bytes;
     out3[1] = j ? j->bytes : 0;
@@ -208,6 +212,7 @@ int kz_clique_set_buckets(kz_graph g, int k, const kz_bucket_cfg* cfg) {
     if (!g || !cfg || k < 3 || k > 5) KZ_FAIL(KZ_ERR_INVALID, "bad argument");
     BucketCfg c = from_abi(*cfg);
     if (int e = check_buckets(c)) return e;
+    std::lock_guard<std::mutex> lk(g->g.exec_mu);
     store_buckets(g->g, k, c);
     return KZ_OK;
 }
@@ -216,6 +221,7 @@ int kz_clique_tune(kz_graph g, int k, uint32_t reps, kz_bucket_cfg* chosen, doub
     if (!g || k < 3 || k > 5) KZ_FAIL(KZ_ERR_INVALID, "bad argument");
     if (int e = ensure_ready()) return e;
     DeviceGraph& d = g->g;
+    std::lock_guard<std::mutex> lk(d.exec_mu);
     if (reps == 0) reps = 1;
     double best = 1e300;
     BucketCfg best_cfg = default_buckets();
@@ -255,6 +261,7 @@ int kz_batch_create(const kz_graph* graphs, uint32_t num_graphs, const int* ks, 
             delete b;
             KZ_FAIL(KZ_ERR_INVALID, "null graph in batch");
         }
+        std::lock_guard<std::mutex> lk(g->g.exec_mu);
         if (int e = ensure_forward(g->g)) {
             delete b;
             return e;
@@ -332,7 +339,9 @@ int kz_clique_workload(kz_graph g, uint64_t* out6) {
     if (!g || !out6) KZ_FAIL(KZ_ERR_INVALID, "null argument");
     if (int e = ensure_ready()) return e;
     DeviceGraph& d = g->g;
+    std::unique_lock<std::mutex> lk(d.exec_mu);
     if (int e = ensure_forward(d)) return e;
+    lk.unlock();
     CliqueView v;
     v.rowptr = d.fwd_rowptr;
     v.col = d.fwd_col;

@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "kz_internal.h"
@@ -69,7 +70,11 @@ struct DeviceGraph {
     uint64_t fwd_bytes = 0;
     uint32_t fwd_max = 0;  // largest forward out-degree
     // prepared persistent clique executions, indexed by k (3..5), and the
-    // degree-bucket configuration each uses (set or autotuned)
+    // degree-bucket configuration each uses (set or autotuned).  exec_mu: they
+    // and the forward part are built, run (one cursor and result array each)
+    // and dropped by one call at a time; counting plans of size 3 run one too.
+    // (The server's threads need not take it: its graphs are its own.)
+    std::mutex exec_mu;
     std::shared_ptr<void> clique_exec[6];
     // motif-census state: the graph relabelled by (degree, id) rank, its
     // forward part, counter slabs and the 4-clique job (kz_census.hip)

@@ -34,6 +34,7 @@
 
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 
 #include "kz_device.h"
 #include "kz_kernels.h"
@@ -123,8 +124,7 @@ void add_members(Weights& w, uint32_t pred, int code, bool oriented, uint64_t ti
 int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats* st, bool* taken) {
     *taken = false;
     const char* env = std::getenv("KZ_PLAN_FLAT");  // =0: the general path (for comparisons)
-    if (p.pattern_size != 3 || (env && env[0] == '0') || g.n == 0 || g.plan3 == 2 || plan_validate(p) != KZ_OK)
-        return KZ_OK;
+    if (p.pattern_size != 3 || (env && env[0] == '0') || g.n == 0 || plan_validate(p) != KZ_OK) return KZ_OK;
     auto nbr = [](const kz_set_ref& r) { return r.kind == KZ_SET_NBR; };
     Weights w[KZ_MAX_AGGREGATORS];
     // size 1: order code 0
@@ -180,6 +180,11 @@ int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats
             }
         }
     }
+    // several threads may run plans on one graph: one at a time takes the
+    // closed form, which shares the graph's prepared execution (the executor,
+    // which shares nothing, runs without the lock)
+    std::lock_guard<std::mutex> lk(g.exec_mu);
+    if (g.plan3 == 2) return KZ_OK;
     // (the largest forward degree of an oriented graph is its own; a symmetric
     // graph's is known once its forward copy is built)
     const uint32_t fwd_max = g.oriented ? g.max_degree : g.fwd_ready ? g.fwd_max : 0u;

@@ -143,3 +143,38 @@ def test_size3_plans_equal_the_interpreter_and_the_executor(kzdev, monkeypatch, 
         monkeypatch.delenv("KZ_PLAN_FLAT")
     assert taken >= 5 if name in QUALIFY else taken == 0
     dg.release()
+
+
+def test_threads_run_plans_and_counts_on_one_graph(kzdev):
+    """Threads share a graph: the closed form's first calls (forward copy,
+    3-clique execution) and later ones, beside clique counts of the same k and
+    plans that take the executor, all at once."""
+    import threading
+
+    kz = kzdev
+    g = kz.gen_rmat(12, 12, seed=5)
+    rng = np.random.default_rng(3)
+    plans = [_plan(rng, outside=i % 4 == 3) for i in range(8)]
+    want = [oracle.run_plan(p, g.rowptr, g.col) for p in plans]
+    tri = oracle.run_app("kautomine_triangle", g.rowptr, g.col)[1][0]
+    assert sum(_closed(p, False) for p in plans) >= 4
+    for _ in range(3):
+        dg = g.to_device()
+        print("[case] threads on one graph", flush=True)
+        gate, bad = threading.Barrier(6), []
+
+        def work(t):
+            gate.wait()
+            for i in range(8):
+                j = (i + t) % 8
+                got = dg.count_cliques(3) if t == 5 else dg.count_plan(plans[j])
+                if got != (tri if t == 5 else want[j]):
+                    bad.append((t, j, got))
+
+        threads = [threading.Thread(target=work, args=(t,)) for t in range(6)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad, bad[:3]
+        dg.release()
