@@ -51,7 +51,8 @@ struct DeviceGraph {
     uint32_t max_degree = 0;
     int oriented = 0;
     // no self-loops, and every edge upwards (oriented) or both ways: 1 yes,
-    // 2 no, 0 not checked yet (kz_plan3.hip; a resident graph does not change)
+    // 2 no, 0 not checked yet (kz_plan3.hip; a resident graph does not change);
+    // 3: yes, but the triangle count's execution could not be built
     int plan3 = 0;
     uint64_t* rowptr = nullptr;
     uint32_t* col = nullptr;

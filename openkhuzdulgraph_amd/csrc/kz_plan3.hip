@@ -185,10 +185,7 @@ int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats
     // which shares nothing, runs without the lock)
     std::lock_guard<std::mutex> lk(g.exec_mu);
     if (g.plan3 == 2) return KZ_OK;
-    // (the largest forward degree of an oriented graph is its own; a symmetric
-    // graph's is known once its forward copy is built)
-    const uint32_t fwd_max = g.oriented ? g.max_degree : g.fwd_ready ? g.fwd_max : 0u;
-    if (members && fwd_max > kMaxBitmapDegree) return KZ_OK;
+    if (members && (g.plan3 == 3 || (g.oriented && g.max_degree > kMaxBitmapDegree))) return KZ_OK;
     hipStream_t s = rt().stream;
     DeviceWords dev;
     if (hipMalloc(&dev.p, 8 * (kSums + 1)) != hipSuccess) {
@@ -225,7 +222,13 @@ int plan3_execute(DeviceGraph& g, const PlanDesc& p, uint64_t* raw, kz_run_stats
     double t_ms = 0;
     if (members) {
         CliqueJob* job = nullptr;
-        if (ensure_forward(g) != KZ_OK || g.fwd_max > kMaxBitmapDegree || graph_job(g, 3, &job) != KZ_OK) return KZ_OK;
+        const bool kept = g.fwd_ready;
+        if (ensure_forward(g) != KZ_OK || g.fwd_max > kMaxBitmapDegree || graph_job(g, 3, &job) != KZ_OK) {
+            // not tried again on every call; a copy built for nothing is freed
+            g.plan3 = 3;
+            if (!kept) release_forward(g);
+            return KZ_OK;
+        }
         if (int err = clique_job_run(*job, &T, &t_ms)) return err;
     }
     for (uint32_t a = 0; a < p.num_aggregators; ++a) {

@@ -178,3 +178,41 @@ def test_threads_run_plans_and_counts_on_one_graph(kzdev):
             t.join()
         assert not bad, bad[:3]
         dg.release()
+
+
+def test_roots_too_wide_for_the_triangle_count(kzdev):
+    """An oriented graph with a root of 9,000 neighbours, more than the clique
+    kernels take: plans that count common neighbours run on the executor, the
+    others in closed form."""
+    import tempfile
+
+    kz = kzdev
+    rng = np.random.default_rng(1)
+    pairs = np.concatenate([np.stack([np.zeros(9000, np.int64), np.arange(1, 9001)], 1),
+                            np.sort(rng.choice(9001, (3000, 2)), 1)])
+    pairs = np.unique(pairs[pairs[:, 0] < pairs[:, 1]], axis=0).astype(np.uint32)
+    with tempfile.NamedTemporaryFile(suffix=".dgraph") as f:
+        f.write(np.uint32(9001).tobytes() + np.uint64(len(pairs)).tobytes() + np.zeros(2, np.int32).tobytes())
+        f.write(pairs.tobytes())
+        f.flush()
+        g = kz.load_dgraph(f.name)
+    assert g.oriented_flag and g.max_degree == 9000
+    dg = g.to_device()
+    seen = set()
+    for i in range(24):
+        p = _plan(rng)
+        closed = _closed(p, True)
+        # counts of a third corner above v0 < v1 (a plan whose operation is
+        # the same on both lists counts none)
+        reached = any((p.lists[0].outs[o].pred >> 2) & 1 for o in range(p.lists[0].num_outs)
+                      if p.lists[0].outs[o].kind == _ffi.KZ_OUT_SCATTER)
+        lst = p.lists[p.type_table[2][2]]
+        common = [lst.ops[j].lhs.a != lst.ops[j].rhs.a for j in range(lst.num_ops)]
+        members = reached and any(lst.outs[o].src.kind == _ffi.KZ_SET_SLOT and common[lst.outs[o].src.b]
+                                  and (lst.outs[o].pred >> 4) & 1 for o in range(lst.num_outs))
+        for _ in range(2):
+            assert dg.count_plan(p) == oracle.run_plan(p, g.rowptr, g.col), i
+            assert _took_closed_form(dg.last_stats) == (closed and not members), (i, dg.last_stats)
+        seen.add((closed, members))
+    assert {(True, True), (True, False)} <= seen
+    dg.release()
